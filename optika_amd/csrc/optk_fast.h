@@ -18,11 +18,10 @@
 //    cancellation-free quadratic formula).  Surfaces flagged steep take two
 //    more Newton steps of the residual in float64.
 //  * Apertures, material, ruling and multilayer efficiencies are float32;
-//    normals are float64 (fast square roots) at the float64 hit point.  The multilayer transfer matrices run both polarizations in
-//    one pass and evaluate each layer's index, cosine and phase once (Snell
-//    invariant n sin(theta)); below a grazing threshold, or where the
-//    reference's |U11| < 1e10 guard trips, the float64 routine of
-//    optk_physics.h is used instead.
+//    normals are float64 (fast square roots) at the float64 hit point.
+//    Multilayers are multilayer_column<float>; what it does not cover
+//    (grazing incidence, the reference's |U11| < 1e10 guard) takes the
+//    float64 routine of optk_physics.h.
 //  * Snell's law and the grating equation update the float64 direction with
 //    fast float64 reciprocals and square roots (hardware seed + Newton).
 //
@@ -99,31 +98,6 @@ OPTK_HD double sqrt64(double x) {
 
 using Cf = C<float>;
 
-OPTK_HD Cf fcdiv(Cf a, Cf b) {
-  float inv = 1.0f / (b.re * b.re + b.im * b.im);
-  return {(a.re * b.re + a.im * b.im) * inv, (a.im * b.re - a.re * b.im) * inv};
-}
-
-OPTK_HD Cf fcrcp(Cf b) {
-  float inv = 1.0f / (b.re * b.re + b.im * b.im);
-  return {b.re * inv, -b.im * inv};
-}
-
-OPTK_HD Cf fcsqrt(Cf z) {  // principal branch
-  float x = z.re, y = z.im;
-  float d = sqrtf(x * x + y * y);
-  if (x >= 0.0f) {
-    float r = sqrtf(0.5f * (d + x));
-    float s = (r > 0.0f) ? 0.5f * y / r : 0.0f;
-    return {r, s};
-  }
-  float s = sqrtf(0.5f * (d - x));
-  float r = 0.5f * fabsf(y) / s;
-  return {r, copysignf(s, y)};
-}
-
-OPTK_HD float fabs2(Cf a) { return a.re * a.re + a.im * a.im; }
-
 // ---------------------------------------------------------------------------
 // records of the float32 form, derived once per system from the optk_surface
 // records (host side, float64 composition of the transformations)
@@ -164,7 +138,6 @@ struct FastSpec {
   int32_t pad;
 };
 
-#define OPTK_GRAZING_COS 0.25f   // multilayers: below this cosine, float64
 #define OPTK_STEEP_SLOPE 0.5     // sag slope above which the intercept is polished
 
 // host-side affine algebra (float64) --------------------------------------
@@ -396,6 +369,7 @@ struct FRay {
   double dx, dy, dz;  // direction
   float wavelength, intensity, attenuation, index;
   bool unvignetted;
+  bool rare = false;  // a multilayer was left to the float64 routine (FEAT_DEFER)
 };
 
 OPTK_HD void affine32_apply(const Affine32 &a, float &x, float &y, float &z) {
@@ -731,275 +705,54 @@ OPTK_HD Cf chemical_nf(const optk_chemical &ch, const float *tables, float wavel
   return {(n[lo + 1] - n[lo]) * inv_dx * dx + n[lo], (k[lo + 1] - k[lo]) * inv_dx * dx + k[lo]};
 }
 
-// ---------------------------------------------------------------------------
-// float32 multilayer: both polarizations in one pass
-// ---------------------------------------------------------------------------
-
-struct MLMedium {
-  Cf n, cos;     // index and cosine (Snell invariant n sin)
-  Cf qs, qp;     // s: n cos ; p: conj(cos) / n
-  Cf u00, u11;   // propagation phases exp(-i beta), exp(+i beta)
-  bool ok;       // |u00| < 1e10 (the reference's validity guard)
+// index of a layer record at the wavelength, from the float32 tables
+struct LayerIndex32 {
+  const StackView &sv;
+  const float *tables32;
+  float wavelength;
+  OPTK_HD Cf operator()(const optk_layer &L) const {
+    if (L.chemical < 0) return {1.0f, 0.0f};
+    return chemical_nf(sv.chemicals[L.chemical], tables32, wavelength,
+                       sv.grids ? sv.grids + L.chemical : nullptr, sv.grid_lo);
+  }
 };
-
-struct MLPair {
-  M2<float> s, p;
-};
-
-OPTK_HD MLMedium ml_medium(Cf n, Cf kappa2, float thickness, float wavelength) {
-  MLMedium m;
-  m.n = n;
-  Cf ratio = fcdiv(kappa2, cmul(n, n));
-  m.cos = fcsqrt(Cf{1.0f - ratio.re, -ratio.im});
-  m.qs = cmul(m.cos, n);
-  m.qp = fcdiv(cconj(m.cos), n);
-  if (thickness == 0.0f) {
-    m.u00 = {1.0f, 0.0f};
-    m.u11 = {1.0f, 0.0f};
-    m.ok = true;
-    return m;
-  }
-  // beta = 2 pi h n cos / wavelength (matrices.py:241-246)
-  Cf nc = m.qs;
-  float scale = 6.283185307179586f * thickness / wavelength;
-  float bre = scale * nc.re, bim = scale * nc.im;
-  float sb, cb;
-  sincosf(bre, &sb, &cb);
-  float e = expf(bim);
-  float ei = expf(-bim);
-  m.u00 = {e * cb, -e * sb};
-  m.u11 = {ei * cb, ei * sb};
-  m.ok = e < 1e10f;
-  return m;
-}
-
-OPTK_HD float ml_profile(int kind, float width, float wavelength, Cf di, Cf n) {
-  if (kind == OPTK_PROFILE_NONE) return 1.0f;
-  // s = Re(4 pi n di / wavelength) (profiles.py:103-126)
-  float s = 12.566370614359172f * (n.re * di.re - n.im * di.im) / wavelength;
-  switch (kind) {
-  case OPTK_PROFILE_ERF: {
-    float sw = s * width;
-    return expf(-(sw * sw) * 0.5f);
-  }
-  case OPTK_PROFILE_EXPONENTIAL: {
-    float sw = s * width;
-    return 1.0f / (1.0f + (sw * sw) * 0.5f);
-  }
-  case OPTK_PROFILE_LINEAR: {
-    float x = 1.7320508075688772f * width * s;
-    return sinf(x) / x;
-  }
-  case OPTK_PROFILE_SINUSOIDAL: {
-    const float pi = 3.14159265358979f;
-    float a = pi / (pi * pi - 8.0f);
-    float x = a * width * s;
-    float x1 = x - pi / 2.0f, x2 = x + pi / 2.0f;
-    return pi * (sinf(x1) / x1 + sinf(x2) / x2) / 4.0f;
-  }
-  }
-  return 1.0f;
-}
-
-// interface i -> j followed by propagation through j:
-// (1/t) [[1, r], [r, 1]] diag(u00, u11) with 1/t = (qi + qj) / (2 qi) and
-// r/t = f (qi - qj) / (2 qi)
-OPTK_HD M2<float> ml_step(Cf qi, Cf qj, float f, Cf u00, Cf u11) {
-  Cf w = fcrcp(cscale(2.0f, qi));
-  Cf A = cmul(cadd(qi, qj), w);
-  Cf B = cscale(f, cmul(csub(qi, qj), w));
-  return {cmul(A, u00), cmul(B, u11), cmul(B, u00), cmul(A, u11)};
-}
-
-OPTK_HD MLPair ml_transfer(const MLMedium &i, const MLMedium &j, const optk_layer &layer_j,
-                           float wavelength) {
-  float fs = 1.0f, fp = 1.0f;
-  if (layer_j.profile_kind != OPTK_PROFILE_NONE) {
-    fs = ml_profile(layer_j.profile_kind, (float)layer_j.profile_width, wavelength, i.cos, i.n);
-    fp = ml_profile(layer_j.profile_kind, (float)layer_j.profile_width, wavelength, cconj(i.cos),
-                    i.n);
-  }
-  return {ml_step(i.qs, j.qs, fs, j.u00, j.u11), ml_step(i.qp, j.qp, fp, j.u00, j.u11)};
-}
-
-OPTK_HD MLPair ml_mul(const MLPair &x, const MLPair &y) { return {mmul(x.s, y.s), mmul(x.p, y.p)}; }
-
-OPTK_HD MLPair ml_identity() { return {midentity<float>(), midentity<float>()}; }
-
-OPTK_HD MLPair ml_power(MLPair m, int exponent) {
-  MLPair result = ml_identity();
-  bool have = false;
-  while (exponent > 0) {
-    if (exponent & 1) {
-      result = have ? ml_mul(result, m) : m;
-      have = true;
-    }
-    exponent >>= 1;
-    if (exponent) m = ml_mul(m, m);
-  }
-  return result;
-}
-
-OPTK_HD Cf ml_layer_n(const optk_layer &L, const StackView &sv, const float *tables32,
-                      float wavelength) {
-  if (L.chemical < 0) return {1.0f, 0.0f};
-  return chemical_nf(sv.chemicals[L.chemical], tables32, wavelength,
-                     sv.grids ? sv.grids + L.chemical : nullptr, sv.grid_lo);
-}
-
-// Reflectance (mirror) or transmittance (film) averaged over s and p, or a
-// negative value when the float32 evaluation does not apply (grazing
-// incidence, the validity guard, more than 4 layers in a periodic block).
-// im_q_sub (optional, film only): Im(n_sub cos_sub) of the wave refracted
-// into the substrate
-OPTK_HD float fast_multilayer(const StackView &sv, const float *tables32, int stack_index,
-                              float wavelength, Cf cos_amb, Cf n_amb, bool film,
-                              float *im_q_sub = nullptr) {
-  if (fabsf(cos_amb.re) < OPTK_GRAZING_COS) return -1.0f;
-  const optk_stack &stk = sv.stacks[stack_index];
-  // Snell invariant: kappa^2 = n_amb^2 (1 - cos_amb^2)
-  Cf one_minus = {1.0f - (cos_amb.re * cos_amb.re - cos_amb.im * cos_amb.im),
-                  -2.0f * cos_amb.re * cos_amb.im};
-  Cf kappa2 = cmul(cmul(n_amb, n_amb), one_minus);
-  MLMedium amb;
-  amb.n = n_amb;
-  amb.cos = cos_amb;
-  amb.qs = cmul(cos_amb, n_amb);
-  amb.qp = fcdiv(cconj(cos_amb), n_amb);
-  amb.ok = true;
-  MLMedium prev = amb;
-  MLPair m = ml_identity();
-  bool ok = true;
-  for (int b = 0; b < stk.num_blocks; ++b) {
-    const optk_block &blk = stk.blocks[b];
-    MLPair x;
-    if (blk.kind == OPTK_BLOCK_PERIODIC) {
-      if (blk.num_layers < 1 || blk.num_layers > 4) return -1.0f;
-      const optk_layer &L1 = sv.layers[blk.first_layer];
-      MLMedium first = ml_medium(ml_layer_n(L1, sv, tables32, wavelength), kappa2,
-                                 (float)L1.thickness, wavelength);
-      ok = ok && first.ok;
-      // layers 2..m, shared by the first period and the repeated period
-      MLPair inner = ml_identity();
-      MLMedium last = first;
-      for (int j = 1; j < blk.num_layers; ++j) {
-        const optk_layer &L = sv.layers[blk.first_layer + j];
-        MLMedium med = ml_medium(ml_layer_n(L, sv, tables32, wavelength), kappa2,
-                                 (float)L.thickness, wavelength);
-        ok = ok && med.ok;
-        MLPair st = ml_transfer(last, med, L, wavelength);
-        inner = (j == 1) ? st : ml_mul(inner, st);
-        last = med;
-      }
-      MLPair start = ml_transfer(prev, first, L1, wavelength);
-      MLPair period = ml_transfer(last, first, L1, wavelength);
-      if (blk.num_layers > 1) {
-        start = ml_mul(start, inner);
-        period = ml_mul(period, inner);
-      }
-      x = (blk.num_periods > 1) ? ml_mul(start, ml_power(period, blk.num_periods - 1)) : start;
-      prev = last;
-    } else {
-      x = ml_identity();
-      for (int j = 0; j < blk.num_layers; ++j) {
-        const optk_layer &L = sv.layers[blk.first_layer + j];
-        MLMedium med = ml_medium(ml_layer_n(L, sv, tables32, wavelength), kappa2,
-                                 (float)L.thickness, wavelength);
-        ok = ok && med.ok;
-        x = ml_mul(x, ml_transfer(prev, med, L, wavelength));
-        prev = med;
-      }
-    }
-    m = (b == 0) ? x : ml_mul(m, x);
-  }
-  if (!ok) return -1.0f;
-  // substrate: interface only (thickness zero)
-  optk_layer sub = {-1, OPTK_PROFILE_NONE, 0.0, 0.0};
-  if (stk.substrate_layer >= 0) sub = sv.layers[stk.substrate_layer];
-  MLMedium msub = ml_medium(ml_layer_n(sub, sv, tables32, wavelength), kappa2, 0.0f, wavelength);
-  m = ml_mul(m, ml_transfer(prev, msub, sub, wavelength));
-  if (!film) {
-    float rs = fabs2(m.s.c) / fabs2(m.s.a);
-    float rp = fabs2(m.p.c) / fabs2(m.p.a);
-    return 0.5f * (rs + rp);
-  }
-  float ts = 1.0f / fabs2(m.s.a);
-  float tp = 1.0f / fabs2(m.p.a);
-  float gs = fcdiv(msub.qs, amb.qs).re;
-  float gp = fcdiv(msub.qp, amb.qp).re;
-  if (im_q_sub) *im_q_sub = msub.qs.im;
-  return 0.5f * (ts * gs + tp * gp);
-}
-
-// The float64 multilayer (optk_physics.h) for the rays the float32 pass
-// hands back.  Kept out of line on the device: its registers are then
-// allocated for this rare path alone instead of raising the pressure (and
-// the spills) of every ray's main path.
-#if defined(__HIP_DEVICE_COMPILE__)
-__device__ __attribute__((noinline))
-#else
-inline
-#endif
-float multilayer_fallback64(const StackView &sv, int stack, float wavelength, double cos_theta,
-                            float index, float attenuation, bool film) {
-  double k64 = (double)attenuation * (double)wavelength / (4.0 * M_PI) * 1e-6;
-  MultilayerRT<double> rt = multilayer_efficiency<double>(
-      sv, stack, (double)wavelength, C<double>{cos_theta, 0.0}, C<double>{(double)index, k64}, film);
-  return (float)(film ? (rt.T[0] + rt.T[1]) / 2.0 : (rt.R[0] + rt.R[1]) / 2.0);
-}
-
-// the silicon sensor's absorbance in float64, for the same rays
-#if defined(__HIP_DEVICE_COMPILE__)
-__device__ __attribute__((noinline))
-#else
-inline
-#endif
-float silicon_fallback64(const StackView &sv, int stack, double thickness, float wavelength,
-                         double cos_theta, float index, float attenuation) {
-  double k64 = (double)attenuation * (double)wavelength / (4.0 * M_PI) * 1e-6;
-  return (float)silicon_absorbance_average(sv, stack, thickness, (double)wavelength,
-                                           C<double>{cos_theta, 0.0},
-                                           C<double>{(double)index, k64});
-}
 
 template <int F, uint32_t K = 0>
 OPTK_HD float fast_material_efficiency(const optk_surface &s, const StackView &sv,
                                       const float *tables32, float wavelength, V3<double> a,
-                                      float index, float attenuation, V3<double> normal) {
+                                      float index, float attenuation, V3<double> normal,
+                                      bool &rare) {
   switch (k_material<K>(s)) {
   case OPTK_MATERIAL_MEASURED_MIRROR: {
     const float *w = tables32 + s.material_table;
     return interp1f(w, w + s.material_table_len, s.material_table_len, wavelength);
   }
   case OPTK_MATERIAL_MULTILAYER_MIRROR:
-  case OPTK_MATERIAL_MULTILAYER_FILM: {  // _multilayers.py:839-935
+  case OPTK_MATERIAL_MULTILAYER_FILM:   // _multilayers.py:839-935
+  case OPTK_MATERIAL_SILICON_SENSOR: {  // sensors/materials/_materials.py:2231-2243
     if (!(F & FEAT_MULTILAYER)) return 1.0f;
-    float k = attenuation * wavelength / (4.0f * 3.14159265358979f) * 1e-6f;
-    float cosv = (float)(-(a.x * normal.x + a.y * normal.y + a.z * normal.z));
-    bool film = k_material<K>(s) == OPTK_MATERIAL_MULTILAYER_FILM;
-    float eff = fast_multilayer(sv, tables32, s.stack, wavelength, Cf{cosv, 0.0f},
-                                Cf{index, k}, film);
-    if (eff < 0.0f) {
-      // grazing incidence or the validity guard: the float64 routine
-      double c64 = -(a.x * normal.x + a.y * normal.y + a.z * normal.z);
-      eff = multilayer_fallback64(sv, s.stack, wavelength, c64, index, attenuation, film);
+    const bool silicon = k_material<K>(s) == OPTK_MATERIAL_SILICON_SENSOR;
+    const bool film = k_material<K>(s) != OPTK_MATERIAL_MULTILAYER_MIRROR;
+    const double c64 = -(a.x * normal.x + a.y * normal.y + a.z * normal.z);
+    if (!(F & FEAT_REFERENCE)) {
+      const float k = attenuation * wavelength / (4.0f * 3.14159265358979f) * 1e-6f;
+      MLResult<float> m = multilayer_column<float>(sv, s.stack, wavelength, Cf{(float)c64, 0.0f}, Cf{index, k},
+                                                   film, LayerIndex32{sv, tables32, wavelength});
+      if (m.ok || (F & FEAT_DEFER)) {
+        rare = rare || !m.ok;
+        if (!silicon) return m.efficiency;
+        // the decay 1 - exp(-alpha d) is the same for both polarizations
+        const float absorption = 4.0f * 3.14159265358979f * m.im_q_sub / wavelength;
+        return m.efficiency - m.efficiency * expf(-absorption * (float)s.material_p[0]);
+      }
     }
-    return eff;
-  }
-  case OPTK_MATERIAL_SILICON_SENSOR: {  // _materials.py:2231-2243
-    if (!(F & FEAT_MULTILAYER)) return 1.0f;
-    float k = attenuation * wavelength / (4.0f * 3.14159265358979f) * 1e-6f;
-    float cosv = (float)(-(a.x * normal.x + a.y * normal.y + a.z * normal.z));
-    float im_q = 0.0f;
-    float t = fast_multilayer(sv, tables32, s.stack, wavelength, Cf{cosv, 0.0f}, Cf{index, k},
-                              true, &im_q);
-    if (t < 0.0f) {
-      double c64 = -(a.x * normal.x + a.y * normal.y + a.z * normal.z);
-      return silicon_fallback64(sv, s.stack, s.material_p[0], wavelength, c64, index, attenuation);
-    }
-    // the decay 1 - exp(-alpha d) is the same for both polarizations
-    float absorption = 4.0f * 3.14159265358979f * im_q / wavelength;
-    return t - t * expf(-absorption * (float)s.material_p[0]);
+    // grazing incidence or the validity guard: the float64 routine
+    const double w64 = wavelength;
+    const C<double> n64 = {(double)index, (double)attenuation * w64 / (4.0 * M_PI) * 1e-6};
+    if (silicon)
+      return (float)silicon_absorbance_average(sv, s.stack, s.material_p[0], w64, C<double>{c64, 0.0}, n64);
+    MultilayerRT<double> rt = multilayer_efficiency<double>(sv, s.stack, w64, C<double>{c64, 0.0}, n64, film);
+    return (float)(film ? (rt.T[0] + rt.T[1]) / 2.0 : (rt.R[0] + rt.R[1]) / 2.0);
   }
   default:
     return 1.0f;
@@ -1104,7 +857,7 @@ OPTK_HD void fast_propagate(const FastSurface &f, const optk_surface &s, const F
   const double n2 = fast_index<K>(s, (double)r.wavelength, n1);
   V3<double> b = fast_snell(a, n1, n2, normal, k_mirror<K>(s), !ruled);
   float eff = fast_material_efficiency<F, K>(s, v.sv, v.tables32, r.wavelength, a, r.index,
-                                             r.attenuation, normal);
+                                             r.attenuation, normal, r.rare);
   if (ruled) {
     V3<float> p1 = {(float)hx, (float)hy, (float)hz};
     V3<float> af = {(float)a.x, (float)a.y, (float)a.z};
@@ -1188,6 +941,7 @@ OPTK_HD FRay fast_grid_ray(float fx, float fy, float ux, float uy, float wavelen
   r.attenuation = 0.0f;
   r.index = 1.0f;
   r.unvignetted = true;
+  r.rare = false;
   return r;
 }
 

@@ -209,6 +209,49 @@ typedef __attribute__((address_space(4))) const FastSpec ConstFastSpec;
 typedef __attribute__((address_space(4))) const FastSurface ConstFastSurface;
 typedef __attribute__((address_space(4))) const optk_surface ConstSurface;
 
+// an input ray in the sag frame of the first surface traced: surface 0, or
+// (skip) surface 1 past a pass-through surface 0
+__device__ __forceinline__ void fast_first_hop(const FastArgs &A, bool skip, FRay &r) {
+  ConstFastSpec *c_spec = (ConstFastSpec *)A.spec;
+  if (skip) {
+    // surface 0 is a pass-through on whose plane the grid rays start; a ray
+    // parallel to it meets it at t = -0/0 = NaN
+    const bool parallel = r.dz == 0.0;
+    fast_xf(*(const optk_affine *)&c_spec->first_skip, r);
+    if (parallel) {
+      r.px = r.py = r.pz = NAN;
+      r.intensity = NAN;
+    }
+  } else {
+    fast_xf(*(const optk_affine *)&c_spec->first_hop[A.entry], r);
+  }
+}
+
+template <int IO, typename In>
+__device__ __forceinline__ FRay fast_start(const FastArgs &A, const In &in, bool skip, int64_t i) {
+  FRay r = load_ray<IO>(in, i);
+  fast_first_hop(A, skip, r);
+  return r;
+}
+
+// surfaces k0 .. of path `path`
+template <int F, bool ACCUM>
+__device__ __forceinline__ void fast_path(ConstFastSurface *c_fast, ConstSurface *c_surf, const FastView &v, int k0,
+                                          int num_surfaces, int path, int num_paths, int64_t n, int64_t i,
+                                          const FRaysOut &accum, FRay &r) {
+  for (int k = k0; k < num_surfaces; ++k) {
+    const FastSurface &fk = *(const FastSurface *)&c_fast[k];
+    const optk_surface &sk = *(const optk_surface *)&c_surf[k];
+    if (k > k0) fast_xf(fk.hop, r);
+    fast_propagate<F>(fk, sk, v, path, r);
+    if (ACCUM) {
+      FRay g = r;
+      fast_xf(fk.to_global, g);
+      store_f(accum, ((int64_t)k * num_paths + path) * n + i, g);
+    }
+  }
+}
+
 template <int F, bool ACCUM, int IO, typename In>
 __device__ __forceinline__ void fast_body(const FastArgs &A, const In &in, const FRaysOut &accum) {
   ConstFastSpec *c_spec = (ConstFastSpec *)A.spec;
@@ -230,33 +273,14 @@ __device__ __forceinline__ void fast_body(const FastArgs &A, const In &in, const
   // it in scalar registers (blockDim.x would be a per-lane load)
   const int64_t stride = (int64_t)gridDim.x * TRACE_BLOCK;
   for (int64_t i = (int64_t)blockIdx.x * TRACE_BLOCK + threadIdx.x; i < n; i += stride) {
-    FRay r0 = load_ray<IO>(in, i);
-    if (skip) {
-      // surface 0 is a pass-through on whose plane the grid rays start; a ray
-      // parallel to it meets it at t = -0/0 = NaN
-      const bool parallel = r0.dz == 0.0;
-      fast_xf(*(const optk_affine *)&c_spec->first_skip, r0);
-      if (parallel) {
-        r0.px = r0.py = r0.pz = NAN;
-        r0.intensity = NAN;
-      }
-    } else {
-      fast_xf(*(const optk_affine *)&c_spec->first_hop[A.entry], r0);
-    }
+    const FRay r0 = fast_start<IO>(A, in, skip, i);
     for (int path = 0; path < num_paths; ++path) {
       FRay r = r0;
-      for (int k = k0; k < num_surfaces; ++k) {
-        const FastSurface &fk = *(const FastSurface *)&c_fast[k];
-        const optk_surface &sk = *(const optk_surface *)&c_surf[k];
-        if (k > k0) {
-          fast_xf(fk.hop, r);
-        }
-        fast_propagate<F>(fk, sk, v, path, r);
-        if (ACCUM) {
-          FRay g = r;
-          fast_xf(fk.to_global, g);
-          store_f(accum, ((int64_t)k * num_paths + path) * n + i, g);
-        }
+      fast_path<F | FEAT_DEFER, ACCUM>(c_fast, c_surf, v, k0, num_surfaces, path, num_paths, n, i, accum, r);
+      if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
+        // the whole path again, so that nothing is kept live for it above
+        r = fast_start<IO>(A, in, skip, i);
+        fast_path<F | FEAT_REFERENCE, ACCUM>(c_fast, c_surf, v, k0, num_surfaces, path, num_paths, n, i, accum, r);
       }
       const optk_affine &last = *(const optk_affine *)&c_spec->last[A.apply_post];
       fast_xf(last, r);
@@ -333,20 +357,18 @@ __device__ __forceinline__ void fast_spec_body(const FastArgs &A, const In &in) 
   const bool skip = A.entry == 1 && c_spec->skip_first != 0;
   const int k0 = skip ? 1 : 0;
   FRay r0 = load_ray32<IO>(in, i32);
-  if (skip) {
-    const bool parallel = r0.dz == 0.0;
-    fast_xf(*(const optk_affine *)&c_spec->first_skip, r0);
-    if (parallel) {
-      r0.px = r0.py = r0.pz = NAN;
-      r0.intensity = NAN;
-    }
-  } else {
-    fast_xf(*(const optk_affine *)&c_spec->first_hop[A.entry], r0);
-  }
+  fast_first_hop(A, skip, r0);
   for (int path = 0; path < num_paths; ++path) {
     FRay r = r0;
     int k = 0;
-    (fast_spec_step<F, K>(k++, k0, c_fast, c_surf, v, path, r), ...);
+    (fast_spec_step<F | FEAT_DEFER, K>(k++, k0, c_fast, c_surf, v, path, r), ...);
+    if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
+      // the whole path again, so that nothing is kept live for it above
+      r = load_ray32<IO>(in, i32);
+      fast_first_hop(A, skip, r);
+      fast_path<F | FEAT_REFERENCE, false>(c_fast, c_surf, v, k0, A.num_surfaces, path, num_paths, A.n, i32,
+                                           FRaysOut{}, r);
+    }
     const optk_affine &last = *(const optk_affine *)&c_spec->last[A.apply_post];
     fast_xf(last, r);
     store_ray32<IO>(A.out, (uint32_t)path * n32 + i32, r);
@@ -438,18 +460,9 @@ template <int F> struct Tracer32 {
                 sizeof(optk_surface) * (size_t)A.num_surfaces);
   }
 
-  __device__ __forceinline__ void trace(int64_t i, int path, double &x, double &y, double &inten,
-                                        bool &unv) {
-    FastView v;
-    v.surfaces = s_surf;
-    v.fast = s_fast;
-    v.sv = A.sv;
-    v.tables32 = A.tables32;
+  __device__ __forceinline__ FRay start(int64_t i) {
     FRay r = load_fray(in, i);
-    // a pass-through surface 0 is elided as in the grid kernels
-    const bool skip = s_spec->skip_first != 0;
-    const int k0 = skip ? 1 : 0;
-    if (skip) {
+    if (s_spec->skip_first != 0) {
       const bool parallel = r.dz == 0.0;
       fast_xf(s_spec->first_skip, r);
       if (parallel) {
@@ -459,12 +472,34 @@ template <int F> struct Tracer32 {
     } else {
       fast_xf(s_spec->first_hop[1], r);
     }
+    return r;
+  }
+
+  // the whole path with the float64 multilayer (FRay::rare)
+  __device__ __forceinline__ void reference(const FastView &v, int64_t i, int path, FRay &r) {
+    const int k0 = s_spec->skip_first != 0 ? 1 : 0;
+    r = start(i);
     for (int k = k0; k < A.num_surfaces; ++k) {
-      if (k > k0) {
-        fast_xf(s_fast[k].hop, r);
-      }
-      fast_propagate<F>(s_fast[k], s_surf[k], v, path, r);
+      if (k > k0) fast_xf(s_fast[k].hop, r);
+      fast_propagate<F | FEAT_REFERENCE>(s_fast[k], s_surf[k], v, path, r);
     }
+  }
+
+  __device__ __forceinline__ void trace(int64_t i, int path, double &x, double &y, double &inten,
+                                        bool &unv) {
+    FastView v;
+    v.surfaces = s_surf;
+    v.fast = s_fast;
+    v.sv = A.sv;
+    v.tables32 = A.tables32;
+    // a pass-through surface 0 is elided as in the grid kernels
+    const int k0 = s_spec->skip_first != 0 ? 1 : 0;
+    FRay r = start(i);
+    for (int k = k0; k < A.num_surfaces; ++k) {
+      if (k > k0) fast_xf(s_fast[k].hop, r);
+      fast_propagate<F | FEAT_DEFER>(s_fast[k], s_surf[k], v, path, r);
+    }
+    if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) reference(v, i, path, r);
     const optk_affine &last = s_spec->last[A.apply_post];
     fast_xf(last, r);
     store_f(out, (int64_t)path * A.n + i, r);
@@ -495,21 +530,11 @@ template <int F, uint32_t... K> struct Tracer32Spec : Tracer32<F> {
     v.fast = this->s_fast;
     v.sv = this->A.sv;
     v.tables32 = this->A.tables32;
-    FRay r = load_fray(this->in, i);
-    const bool skip = this->s_spec->skip_first != 0;
-    const int k0 = skip ? 1 : 0;
-    if (skip) {
-      const bool parallel = r.dz == 0.0;
-      fast_xf(this->s_spec->first_skip, r);
-      if (parallel) {
-        r.px = r.py = r.pz = NAN;
-        r.intensity = NAN;
-      }
-    } else {
-      fast_xf(this->s_spec->first_hop[1], r);
-    }
+    const int k0 = this->s_spec->skip_first != 0 ? 1 : 0;
+    FRay r = this->start(i);
     int k = 0;
-    (batch_fast_step<F, K>(k++, k0, this->s_fast, this->s_surf, v, path, r), ...);
+    (batch_fast_step<F | FEAT_DEFER, K>(k++, k0, this->s_fast, this->s_surf, v, path, r), ...);
+    if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) this->reference(v, i, path, r);
     const optk_affine &last = this->s_spec->last[this->A.apply_post];
     fast_xf(last, r);
     store_f(this->out, (int64_t)path * this->A.n + i, r);

@@ -301,8 +301,17 @@ __device__ __forceinline__ void trace_body(const TraceArgs &A, const In &in, con
     for (int path = 0; path < num_paths; ++path) {
       Ray<double> r = r0;
       for (int k = 0; k < num_surfaces; ++k) {
-        propagate_surface<F>(*(const optk_surface *)&c_surf[k], sys, path, r);
+        propagate_surface<F | FEAT_DEFER>(*(const optk_surface *)&c_surf[k], sys, path, r);
         if (ACCUM) store(accum, ((int64_t)k * num_paths + path) * n + i, r);
+      }
+      if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
+        // the whole path again, so that nothing is kept live for it above
+        r = load_io<IO>(in, i);
+        apply_pre(spec, r);
+        for (int k = 0; k < num_surfaces; ++k) {
+          propagate_surface<F | FEAT_REFERENCE>(*(const optk_surface *)&c_surf[k], sys, path, r);
+          if (ACCUM) store(accum, ((int64_t)k * num_paths + path) * n + i, r);
+        }
       }
       if (A.apply_post) {
         xf_inverse_ray(spec.post, r.px, r.py, r.pz, r.dx, r.dy, r.dz);
@@ -361,7 +370,14 @@ __device__ __forceinline__ void spec_body(const TraceArgs &A, const In &in) {
   for (int path = 0; path < num_paths; ++path) {
     Ray<double> r = r0;
     int k = 0;
-    (propagate_surface<F, K>(*(const optk_surface *)&c_surf[k++], sys, path, r), ...);
+    (propagate_surface<F | FEAT_DEFER, K>(*(const optk_surface *)&c_surf[k++], sys, path, r), ...);
+    if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
+      // the whole path again, so that nothing is kept live for it above
+      r = load_io32<IO>(in, i32);
+      apply_pre(spec, r);
+      for (k = 0; k < A.num_surfaces; ++k)
+        propagate_surface<F | FEAT_REFERENCE>(*(const optk_surface *)&c_surf[k], sys, path, r);
+    }
     if (A.apply_post) xf_inverse_ray(spec.post, r.px, r.py, r.pz, r.dx, r.dy, r.dz);
     store_io32<IO>(A.out, (uint32_t)path * n32 + i32, r);
   }
@@ -579,7 +595,12 @@ template <int F> struct Tracer64 {
     apply_pre(*s_spec, r);
     SystemView sys = s_spec->sys;
     sys.surfaces = s_surf;
-    for (int k = 0; k < A.num_surfaces; ++k) propagate_surface<F>(s_surf[k], sys, path, r);
+    for (int k = 0; k < A.num_surfaces; ++k) propagate_surface<F | FEAT_DEFER>(s_surf[k], sys, path, r);
+    if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
+      r = load_ray(in, i);
+      apply_pre(*s_spec, r);
+      for (int k = 0; k < A.num_surfaces; ++k) propagate_surface<F | FEAT_REFERENCE>(s_surf[k], sys, path, r);
+    }
     if (A.apply_post) {
       xf_inverse_ray(s_spec->post, r.px, r.py, r.pz, r.dx, r.dy, r.dz);
     }
@@ -602,7 +623,13 @@ template <int F, uint32_t... K> struct Tracer64Spec : Tracer64<F> {
     SystemView sys = this->s_spec->sys;
     sys.surfaces = this->s_surf;
     int k = 0;
-    (propagate_surface<F, K>(this->s_surf[k++], sys, path, r), ...);
+    (propagate_surface<F | FEAT_DEFER, K>(this->s_surf[k++], sys, path, r), ...);
+    if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
+      r = load_ray(this->in, i);
+      apply_pre(*this->s_spec, r);
+      for (k = 0; k < this->A.num_surfaces; ++k)
+        propagate_surface<F | FEAT_REFERENCE>(this->s_surf[k], sys, path, r);
+    }
     if (this->A.apply_post) {
       xf_inverse_ray(this->s_spec->post, r.px, r.py, r.pz, r.dx, r.dy, r.dz);
     }
@@ -781,10 +808,13 @@ __global__ __launch_bounds__(256) void eval_f64(const EvalParams E) {
                                    {in[4][i], in[5][i], in[6][i]}, {in[7][i], in[8][i], in[9][i]},
                                    E.sys.sv.tables);
     break;
-  case OPTK_OP_MATERIAL_EFF:
-    out[0][i] = material_efficiency(s, E.sys.sv, in[0][i], {in[1][i], in[2][i], in[3][i]}, in[4][i],
-                                    in[5][i], {in[6][i], in[7][i], in[8][i]});
+  case OPTK_OP_MATERIAL_EFF: {
+    bool rare = false;
+    out[0][i] = material_efficiency<FEAT_ALL | FEAT_REFERENCE>(
+        s, E.sys.sv, in[0][i], {in[1][i], in[2][i], in[3][i]}, in[4][i], in[5][i],
+        {in[6][i], in[7][i], in[8][i]}, rare);
     break;
+  }
   case OPTK_OP_INDEX:
     out[0][i] = material_index(s, in[0][i], in[1][i]);
     break;

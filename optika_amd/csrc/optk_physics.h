@@ -259,6 +259,7 @@ template <typename T> struct Ray {
   T dx, dy, dz;
   T wavelength, intensity, attenuation, index;
   bool unvignetted;
+  bool rare = false;  // a multilayer was left to the reference's operations (FEAT_DEFER)
 };
 
 // ---------------------------------------------------------------------------
@@ -684,6 +685,394 @@ OPTK_HD MultilayerRT<T> multilayer_efficiency(const StackView &sv, int stack_ind
     out.T[0] = (ts * ts) * cdiv(q_sub_s, q_amb_s).re;
     out.T[1] = (tp * tp) * cdiv(q_sub_p, q_amb_p).re;
   }
+  return out;
+}
+
+// ---------------------------------------------------------------------------
+// The multilayer efficiency of the trace kernels (both forms).
+//
+// Everything a mirror or film needs of the stack's transfer matrix is its
+// first column (r = c / a, t = 1 / a), so a 2-vector per polarization is
+// carried from the substrate to the ambient medium instead of a product of
+// matrices from the ambient medium down; only a repeated period needs its
+// matrix, for the squarings of the binary powering (5 products each, and a
+// matrix-vector product of 4 per set bit).  Each medium's index, cosine and
+// phases are evaluated once: the cosine from the Snell invariant
+// n^2 sin^2, the two phases exp(-+ i beta) from one exponential, one
+// reciprocal and one sine and cosine, and the interface i -> j as
+// (q_i +- q_j) / (2 q_i) from one reciprocal per medium.  Products use fused
+// multiply-adds.  multilayer_rt above follows the reference's operations
+// instead (a matrix per layer and polarization, the period evaluated twice,
+// four complex divisions per interface, two complex exponentials and two
+// complex square roots per layer): about 10,000 VALU instructions for the
+// 40-period Mo/Si mirror, against about 1,500 here.  The two agree to a few
+// 1e-15 relative where this one applies; it hands back (ok = false) what it
+// does not cover: grazing incidence, where the refracted cosine cancels and
+// the reference's own rounding decides the result, the reference's
+// |exp(-i beta)| < 1e10 validity guard, lossless total reflection (the sign
+// of a zero picks the branch), and magnitudes near the range's ends.
+// ---------------------------------------------------------------------------
+
+#define OPTK_GRAZING_COS 0.25  // multilayers: below this cosine, multilayer_rt
+
+OPTK_HD double ml_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+OPTK_HD float ml_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
+// reciprocal of a finite nonzero value: hardware seed (2^-24.4) and two
+// Newton steps, within an ulp
+OPTK_HD double ml_rcp(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double r = __builtin_amdgcn_rcp(x);
+  r = ml_fma(r, ml_fma(-x, r, 1.0), r);
+  return ml_fma(r, ml_fma(-x, r, 1.0), r);
+#else
+  return 1.0 / x;
+#endif
+}
+OPTK_HD float ml_rcp(float x) { return 1.0f / x; }
+
+// square root of a finite value >= 0: hardware reciprocal square root
+// (2^-24.2), one coupled Newton step for the root and its half reciprocal
+// and one on the residual x - g^2
+OPTK_HD double ml_sqrt(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double e = ml_fma(-h, g, 0.5);
+  g = ml_fma(g, e, g);
+  h = ml_fma(h, e, h);
+  g = ml_fma(ml_fma(-g, g, x), h, g);
+  return x == 0.0 ? x : g;
+#else
+  return sqrt(x);
+#endif
+}
+OPTK_HD float ml_sqrt(float x) { return sqrtf(x); }
+
+// sin and cos for |x| <= ml_angle_limit: x - k pi/2 with pi/2 in three (two)
+// parts, then the Maclaurin series on [-pi/4, pi/4] (through x^17 and x^16,
+// truncation below 1e-17; float32 through x^9 and x^8, below 3e-9)
+OPTK_HD double ml_angle_limit(double) { return 1e5; }
+OPTK_HD float ml_angle_limit(float) { return 1e3f; }
+
+OPTK_HD void ml_sincos(double x, double &s, double &c) {
+  const double k = rint(x * 0.63661977236758134308);
+  double r = ml_fma(-k, 1.5707963267948966, x);
+  r = ml_fma(-k, 6.123233995736766e-17, r);
+  r = ml_fma(-k, -1.4973849048591833e-33, r);
+  const double z = r * r;
+  double p = 1.0 / 355687428096000.0;
+  p = ml_fma(p, z, -1.0 / 1307674368000.0);
+  p = ml_fma(p, z, 1.0 / 6227020800.0);
+  p = ml_fma(p, z, -1.0 / 39916800.0);
+  p = ml_fma(p, z, 1.0 / 362880.0);
+  p = ml_fma(p, z, -1.0 / 5040.0);
+  p = ml_fma(p, z, 1.0 / 120.0);
+  p = ml_fma(p, z, -1.0 / 6.0);
+  const double sr = ml_fma(r * z, p, r);
+  double q = 1.0 / 20922789888000.0;
+  q = ml_fma(q, z, -1.0 / 87178291200.0);
+  q = ml_fma(q, z, 1.0 / 479001600.0);
+  q = ml_fma(q, z, -1.0 / 3628800.0);
+  q = ml_fma(q, z, 1.0 / 40320.0);
+  q = ml_fma(q, z, -1.0 / 720.0);
+  q = ml_fma(q, z, 1.0 / 24.0);
+  q = ml_fma(q, z, -0.5);
+  const double cr = ml_fma(q, z, 1.0);
+  const int n = (int)k;
+  const double a = (n & 1) ? cr : sr, b = (n & 1) ? sr : cr;
+  s = (n & 2) ? -a : a;
+  c = ((n + 1) & 2) ? -b : b;
+}
+
+OPTK_HD void ml_sincos(float x, float &s, float &c) {
+  const float k = rintf(x * 0.636619772f);
+  float r = ml_fma(-k, 1.57079637f, x);
+  r = ml_fma(-k, -4.37113883e-8f, r);
+  const float z = r * r;
+  float p = 1.0f / 362880.0f;
+  p = ml_fma(p, z, -1.0f / 5040.0f);
+  p = ml_fma(p, z, 1.0f / 120.0f);
+  p = ml_fma(p, z, -1.0f / 6.0f);
+  const float sr = ml_fma(r * z, p, r);
+  float q = 1.0f / 40320.0f;
+  q = ml_fma(q, z, -1.0f / 720.0f);
+  q = ml_fma(q, z, 1.0f / 24.0f);
+  q = ml_fma(q, z, -0.5f);
+  const float cr = ml_fma(q, z, 1.0f);
+  const int n = (int)k;
+  const float a = (n & 1) ? cr : sr, b = (n & 1) ? sr : cr;
+  s = (n & 2) ? -a : a;
+  c = ((n + 1) & 2) ? -b : b;
+}
+
+// exp for |x| <= 24 (the validity guard ends at 23.03): x - k ln 2 with ln 2
+// in two parts, then the Maclaurin series on [-ln 2 / 2, ln 2 / 2] through
+// x^13 (truncation below 1e-17 relative)
+OPTK_HD double ml_exp(double x) {
+  const double k = rint(x * 1.4426950408889634);
+  double r = ml_fma(-k, 0.6931471805599453, x);
+  r = ml_fma(-k, 2.3190468138462996e-17, r);
+  double p = 1.0 / 6227020800.0;
+  p = ml_fma(p, r, 1.0 / 479001600.0);
+  p = ml_fma(p, r, 1.0 / 39916800.0);
+  p = ml_fma(p, r, 1.0 / 3628800.0);
+  p = ml_fma(p, r, 1.0 / 362880.0);
+  p = ml_fma(p, r, 1.0 / 40320.0);
+  p = ml_fma(p, r, 1.0 / 5040.0);
+  p = ml_fma(p, r, 1.0 / 720.0);
+  p = ml_fma(p, r, 1.0 / 120.0);
+  p = ml_fma(p, r, 1.0 / 24.0);
+  p = ml_fma(p, r, 1.0 / 6.0);
+  p = ml_fma(p, r, 0.5);
+  p = ml_fma(p, r, 1.0);
+  p = ml_fma(p, r, 1.0);
+  return ldexp(p, (int)k);
+}
+OPTK_HD float ml_exp(float x) { return expf(x); }
+
+// complex helpers with fused products
+template <typename T> OPTK_HD C<T> ml_mul(C<T> a, C<T> b) {
+  return {ml_fma(a.re, b.re, -(a.im * b.im)), ml_fma(a.re, b.im, a.im * b.re)};
+}
+template <typename T> OPTK_HD C<T> ml_mad(C<T> a, C<T> b, C<T> c) {  // a b + c
+  return {ml_fma(a.re, b.re, ml_fma(-a.im, b.im, c.re)), ml_fma(a.re, b.im, ml_fma(a.im, b.re, c.im))};
+}
+template <typename T> OPTK_HD C<T> ml_sqr(C<T> a) {
+  return {ml_fma(a.re, a.re, -(a.im * a.im)), T(2) * a.re * a.im};
+}
+template <typename T> OPTK_HD C<T> ml_inv(C<T> a) {
+  const T i = ml_rcp(ml_fma(a.re, a.re, a.im * a.im));
+  return {a.re * i, -a.im * i};
+}
+template <typename T> OPTK_HD T ml_abs2(C<T> a) { return ml_fma(a.re, a.re, a.im * a.im); }
+
+template <typename T> struct MLColumn {
+  C<T> a, c;  // first column of the matrices so far
+};
+template <typename T> struct MLPhase {
+  C<T> u00, u11;  // exp(-i beta), exp(+i beta)
+};
+// one medium: index, cosine, and for each polarization q (s: n cos, p:
+// conj(cos) / n) and 1 / (2 q)
+template <typename T> struct MLMedium {
+  C<T> n, cos, qs, qp, hs, hp;
+};
+
+template <typename T>
+OPTK_HD MLMedium<T> ml_medium_of(C<T> n, C<T> ninv, C<T> cosine) {
+  MLMedium<T> m;
+  m.n = n;
+  m.cos = cosine;
+  m.qs = ml_mul(cosine, n);
+  m.qp = ml_mul(cconj(cosine), ninv);
+  // of the rounded q, so that an interface and its reverse multiply to the
+  // identity to within the reciprocal's rounding (a repeated period raises
+  // what is left to the number of periods)
+  m.hs = cscale(T(0.5), ml_inv(m.qs));
+  m.hp = cscale(T(0.5), ml_inv(m.qp));
+  return m;
+}
+
+// the medium of index n, its cosine from the Snell invariant
+// kappa2 = (n_amb sin_amb)^2
+template <typename T> OPTK_HD MLMedium<T> ml_medium(C<T> n, C<T> kappa2, bool &ok) {
+  const C<T> n2inv = ml_inv(ml_sqr(n));
+  const C<T> s2 = ml_mul(kappa2, n2inv);
+  const T x = T(1) - s2.re, y = -s2.im;
+  // principal square root of x + i y
+  const T d = ml_sqrt(ml_fma(x, x, y * y));
+  const T w = ml_sqrt(T(0.5) * (d + fabs(x)));
+  const T v = T(0.5) * fabs(y) * ml_rcp(w);
+  ok = ok && !(x <= T(0) && y == T(0));
+  const C<T> cosine = x >= T(0) ? C<T>{w, copysign(v, y)} : C<T>{v, copysign(w, y)};
+  return ml_medium_of<T>(n, ml_mul(n, n2inv), cosine);
+}
+
+// beta = 2 pi h n cos / wavelength (matrices.py:241-246)
+template <typename T>
+OPTK_HD MLPhase<T> ml_phase(const MLMedium<T> &m, T thickness, T wavelength, T inv_wavelength, bool &ok) {
+  // the quotient corrected by its residual: its relative error is the
+  // phase's, and a repeated period multiplies it
+  const T turn = T(2.0 * M_PI) * thickness;
+  const T quot = turn * inv_wavelength;
+  const T scale = ml_fma(ml_fma(-quot, wavelength, turn), inv_wavelength, quot);
+  const T b_re = scale * m.qs.re, b_im = scale * m.qs.im;
+  ok = ok && !(fabs(b_re) > ml_angle_limit(T(0))) && !(fabs(b_im) > T(24));
+  T s, c;
+  ml_sincos(b_re, s, c);
+  const T e = ml_exp(b_im);
+  const T ei = ml_rcp(e);
+  ok = ok && !(e >= T(1e10));
+  return {{e * c, -e * s}, {ei * c, ei * s}};
+}
+
+// the interface i -> j of one polarization: 1/t = (q_i + q_j) / (2 q_i) and
+// r/t = f (q_i - q_j) / (2 q_i), f the roughness factor
+template <typename T> struct MLInterface {
+  C<T> A, B;
+};
+template <typename T> OPTK_HD MLInterface<T> ml_interface(C<T> qi, C<T> hi, C<T> qj, T f) {
+  return {ml_mul(cadd(qi, qj), hi), cscale(f, ml_mul(csub(qi, qj), hi))};
+}
+template <typename T> struct MLCross {
+  MLInterface<T> s, p;
+};
+template <typename T>
+OPTK_HD MLCross<T> ml_cross(const MLMedium<T> &i, const MLMedium<T> &j, const optk_layer &layer_j,
+                            T wavelength) {
+  T fs = T(1), fp = T(1);
+  if (layer_j.profile_kind != OPTK_PROFILE_NONE) {
+    fs = profile_factor<T>(layer_j.profile_kind, T(layer_j.profile_width), wavelength, i.cos, i.n);
+    fp = profile_factor<T>(layer_j.profile_kind, T(layer_j.profile_width), wavelength, cconj(i.cos), i.n);
+  }
+  return {ml_interface<T>(i.qs, i.hs, j.qs, fs), ml_interface<T>(i.qp, i.hp, j.qp, fp)};
+}
+
+template <typename T> OPTK_HD void ml_apply(const MLInterface<T> &x, MLColumn<T> &v) {
+  const C<T> a = ml_mad(x.A, v.a, ml_mul(x.B, v.c));
+  v.c = ml_mad(x.A, v.c, ml_mul(x.B, v.a));
+  v.a = a;
+}
+template <typename T> OPTK_HD void ml_apply(const MLPhase<T> &u, MLColumn<T> &v) {
+  v.a = ml_mul(u.u00, v.a);
+  v.c = ml_mul(u.u11, v.c);
+}
+template <typename T> OPTK_HD void ml_apply(const M2<T> &m, MLColumn<T> &v) {
+  const C<T> a = ml_mad(m.a, v.a, ml_mul(m.b, v.c));
+  v.c = ml_mad(m.d, v.c, ml_mul(m.c, v.a));
+  v.a = a;
+}
+// interface times phases: a layer's matrix
+template <typename T> OPTK_HD M2<T> ml_layer(const MLInterface<T> &x, const MLPhase<T> &u) {
+  return {ml_mul(x.A, u.u00), ml_mul(x.B, u.u11), ml_mul(x.B, u.u00), ml_mul(x.A, u.u11)};
+}
+// interface times phases times m
+template <typename T> OPTK_HD M2<T> ml_layer_times(const MLInterface<T> &x, const MLPhase<T> &u, const M2<T> &m) {
+  const M2<T> y = {ml_mul(u.u00, m.a), ml_mul(u.u00, m.b), ml_mul(u.u11, m.c), ml_mul(u.u11, m.d)};
+  return {ml_mad(x.A, y.a, ml_mul(x.B, y.c)), ml_mad(x.A, y.b, ml_mul(x.B, y.d)),
+          ml_mad(x.B, y.a, ml_mul(x.A, y.c)), ml_mad(x.B, y.b, ml_mul(x.A, y.d))};
+}
+template <typename T> OPTK_HD M2<T> ml_square(const M2<T> &m) {
+  const C<T> bc = ml_mul(m.b, m.c), tr = cadd(m.a, m.d);
+  return {ml_mad(m.a, m.a, bc), ml_mul(m.b, tr), ml_mul(m.c, tr), ml_mad(m.d, m.d, bc)};
+}
+
+template <typename T> struct MLResult {
+  T efficiency;  // s/p average of the reflectance (mirror) or transmittance (film)
+  T im_q_sub;    // Im(n cos) of the wave in the substrate
+  bool ok;       // false: evaluate multilayer_efficiency instead
+};
+
+// index(layer): the refractive index of a layer record at the wavelength
+template <typename T, typename Index>
+OPTK_HD MLResult<T> multilayer_column(const StackView &sv, int stack_index, T wavelength,
+                                      C<T> cos_amb, C<T> n_amb, bool film, Index index) {
+  const optk_stack &stk = sv.stacks[stack_index];
+  MLResult<T> out;
+  bool ok = !(fabs(cos_amb.re) < T(OPTK_GRAZING_COS));
+  const C<T> one_minus = {T(1) - (cos_amb.re * cos_amb.re - cos_amb.im * cos_amb.im),
+                          T(-2) * cos_amb.re * cos_amb.im};
+  const C<T> kappa2 = ml_mul(ml_sqr(n_amb), one_minus);
+  const T inv_wavelength = ml_rcp(wavelength);
+  optk_layer right = {-1, OPTK_PROFILE_NONE, 0.0, 0.0};  // the layer whose left interface is pending
+  if (stk.substrate_layer >= 0) right = sv.layers[stk.substrate_layer];
+  MLMedium<T> cur = ml_medium<T>(index(right), kappa2, ok);
+  const C<T> qs_sub = cur.qs, qp_sub = cur.qp;
+  MLColumn<T> s = {{T(1), T(0)}, {T(0), T(0)}}, p = s;
+  for (int b = stk.num_blocks - 1; b >= 0; --b) {
+    const optk_block &blk = stk.blocks[b];
+    const bool periodic = blk.kind == OPTK_BLOCK_PERIODIC;
+    int k = blk.num_layers - 1;
+    if (k < 0) continue;
+    // the block's last medium, and the interface from it to the right
+    optk_layer L = sv.layers[blk.first_layer + k];
+    MLMedium<T> med = ml_medium<T>(index(L), kappa2, ok);
+    MLPhase<T> u = ml_phase<T>(med, T(L.thickness), wavelength, inv_wavelength, ok);
+    MLCross<T> x = ml_cross<T>(med, cur, right, wavelength);
+    ml_apply(x.s, s);
+    ml_apply(x.p, p);
+    if (!periodic) {
+      for (; k > 0; --k) {
+        ml_apply(u, s);
+        ml_apply(u, p);
+        right = L;
+        cur = med;
+        L = sv.layers[blk.first_layer + k - 1];
+        med = ml_medium<T>(index(L), kappa2, ok);
+        u = ml_phase<T>(med, T(L.thickness), wavelength, inv_wavelength, ok);
+        x = ml_cross<T>(med, cur, right, wavelength);
+        ml_apply(x.s, s);
+        ml_apply(x.p, p);
+      }
+      ml_apply(u, s);
+      ml_apply(u, p);
+    } else if (k == 0) {
+      // a period of one layer: crossing into itself is the identity
+      for (int j = 0; j < blk.num_periods || j < 1; ++j) {
+        ml_apply(u, s);
+        ml_apply(u, p);
+      }
+    } else {
+      // inner: layers 2 .. m, shared by the first period (which starts at
+      // the medium to the left) and the repeated one (which starts at the
+      // period's own last medium)
+      const MLMedium<T> last = med;
+      M2<T> inner_s, inner_p;
+      bool first = true;
+      for (; k > 0; --k) {
+        const MLPhase<T> uk = u;
+        right = L;
+        cur = med;
+        L = sv.layers[blk.first_layer + k - 1];
+        med = ml_medium<T>(index(L), kappa2, ok);
+        u = ml_phase<T>(med, T(L.thickness), wavelength, inv_wavelength, ok);
+        x = ml_cross<T>(med, cur, right, wavelength);
+        inner_s = first ? ml_layer(x.s, uk) : ml_layer_times(x.s, uk, inner_s);
+        inner_p = first ? ml_layer(x.p, uk) : ml_layer_times(x.p, uk, inner_p);
+        first = false;
+      }
+      int e = blk.num_periods - 1;
+      if (e > 0) {
+        x = ml_cross<T>(last, med, L, wavelength);
+        M2<T> zs = ml_layer_times(x.s, u, inner_s), zp = ml_layer_times(x.p, u, inner_p);
+        for (;;) {
+          if (e & 1) {
+            ml_apply(zs, s);
+            ml_apply(zp, p);
+          }
+          e >>= 1;
+          if (e == 0) break;
+          zs = ml_square(zs);
+          zp = ml_square(zp);
+        }
+      }
+      ml_apply(inner_s, s);
+      ml_apply(inner_p, p);
+      ml_apply(u, s);
+      ml_apply(u, p);
+    }
+    right = L;
+    cur = med;
+  }
+  const MLMedium<T> amb = ml_medium_of<T>(n_amb, ml_inv(n_amb), cos_amb);
+  const MLCross<T> x = ml_cross<T>(amb, cur, right, wavelength);
+  ml_apply(x.s, s);
+  ml_apply(x.p, p);
+  const T as = ml_abs2(s.a), ap = ml_abs2(p.a);
+  const T big = sizeof(T) == 8 ? T(1e300) : T(1e37);
+  ok = ok && !(as > big) && !(ap > big) && !(as < T(1) / big) && !(ap < T(1) / big);
+  out.im_q_sub = qs_sub.im;
+  const T is = ml_rcp(as), ip = ml_rcp(ap);
+  if (film) {
+    // |t|^2 Re(q_sub / q_amb), 1 / q_amb = 2 h
+    const T gs = T(2) * ml_mul(qs_sub, amb.hs).re, gp = T(2) * ml_mul(qp_sub, amb.hp).re;
+    out.efficiency = T(0.5) * ml_fma(is, gs, ip * gp);
+  } else {
+    out.efficiency = T(0.5) * ml_fma(ml_abs2(s.c), is, ml_abs2(p.c) * ip);
+  }
+  // a NaN stands only where the ray brought one (it missed a surface)
+  out.ok = ok && (out.efficiency == out.efficiency || cos_amb.re != cos_amb.re || wavelength != wavelength);
   return out;
 }
 

@@ -16,6 +16,14 @@ enum : int {
   FEAT_RULINGS = 2,
   FEAT_MULTILAYER = 4,
   FEAT_ALL = 7,
+  // how multilayers are evaluated: by multilayer_column, and what it hands
+  // back at once by the reference's operations (neither bit); handed back to
+  // the caller in the ray's `rare` flag (DEFER), which then traces the path
+  // again by the reference's operations alone (REFERENCE).  The kernels
+  // defer: inlined at every surface, the rare path's registers would be
+  // every ray's.
+  FEAT_DEFER = 8,
+  FEAT_REFERENCE = 16,
 };
 
 // Compile-time kinds of one surface record.  A specialised kernel fixes the
@@ -535,33 +543,44 @@ OPTK_HD double silicon_absorbance_average(const StackView &sv, int stack, double
   return (s_abs + p_abs) / 2.0;
 }
 
+struct LayerIndex64 {
+  const StackView &sv;
+  double wavelength;
+  OPTK_HD C<double> operator()(const optk_layer &L) const { return layer_index<double>(L, sv, wavelength); }
+};
+
 template <int F = FEAT_ALL, uint32_t K = 0>
 OPTK_HD double material_efficiency(const optk_surface &s, const StackView &sv, double wavelength,
                                    V3<double> a, double index, double attenuation,
-                                   V3<double> normal) {
+                                   V3<double> normal, bool &rare) {
   switch (k_material<K>(s)) {
   case OPTK_MATERIAL_MEASURED_MIRROR: {  // _materials.py:279-305
     const double *w = sv.tables + s.material_table;
     return interp1(w, w + s.material_table_len, s.material_table_len, wavelength);
   }
   case OPTK_MATERIAL_MULTILAYER_MIRROR:
-  case OPTK_MATERIAL_MULTILAYER_FILM: {  // _multilayers.py:839-935
+  case OPTK_MATERIAL_MULTILAYER_FILM:    // _multilayers.py:839-935
+  case OPTK_MATERIAL_SILICON_SENSOR: {   // sensors/materials/_materials.py:2231-2243
     if (!(F & FEAT_MULTILAYER)) return 1.0;
+    const bool silicon = k_material<K>(s) == OPTK_MATERIAL_SILICON_SENSOR;
+    const bool film = k_material<K>(s) != OPTK_MATERIAL_MULTILAYER_MIRROR;
     double k = attenuation * wavelength / (4.0 * M_PI) * 1e-6;
     C<double> n = {index, k};
-    double cosv = -dot3(a, normal);
-    bool film = k_material<K>(s) == OPTK_MATERIAL_MULTILAYER_FILM;
-    MultilayerRT<double> rt =
-        multilayer_efficiency<double>(sv, s.stack, wavelength, C<double>{cosv, 0.0}, n, film);
+    C<double> cosv = {-dot3(a, normal), 0.0};
+    if (!(F & FEAT_REFERENCE)) {
+      MLResult<double> m = multilayer_column<double>(sv, s.stack, wavelength, cosv, n, film,
+                                                     LayerIndex64{sv, wavelength});
+      if (m.ok || (F & FEAT_DEFER)) {
+        rare = rare || !m.ok;
+        if (!silicon) return m.efficiency;
+        // Beer-Lambert absorption of the refracted wave, the same for both
+        // polarizations
+        return m.efficiency - m.efficiency * exp(-(4.0 * M_PI * m.im_q_sub / wavelength) * s.material_p[0]);
+      }
+    }
+    if (silicon) return silicon_absorbance_average(sv, s.stack, s.material_p[0], wavelength, cosv, n);
+    MultilayerRT<double> rt = multilayer_efficiency<double>(sv, s.stack, wavelength, cosv, n, film);
     return film ? (rt.T[0] + rt.T[1]) / 2.0 : (rt.R[0] + rt.R[1]) / 2.0;
-  }
-  case OPTK_MATERIAL_SILICON_SENSOR: {  // _materials.py:2231-2243
-    if (!(F & FEAT_MULTILAYER)) return 1.0;
-    double k = attenuation * wavelength / (4.0 * M_PI) * 1e-6;
-    C<double> n = {index, k};
-    double cosv = -dot3(a, normal);
-    return silicon_absorbance_average(sv, s.stack, s.material_p[0], wavelength,
-                                      C<double>{cosv, 0.0}, n);
   }
   default:
     return 1.0;
@@ -651,15 +670,20 @@ OPTK_HD bool aperture_contains(const optk_surface &s, const double *tables, doub
 // the surface step
 // ---------------------------------------------------------------------------
 
+// Up to the intercept, which no diffraction order enters: the ray leaves in
+// the surface frame, at the sag, with the normal there.
 template <int F = FEAT_ALL, uint32_t K = 0>
-OPTK_HD void propagate_surface(const optk_surface &s, const SystemView &sys, int path,
-                               Ray<double> &r) {
+OPTK_HD V3<double> surface_arrive(const optk_surface &s, Ray<double> &r) {
   xf_inverse_ray<Kinds<K>::xf>(s.transform, r.px, r.py, r.pz, r.dx, r.dy, r.dz);
-
   sag_propagate<F, K>(s, r);
-  V3<double> p1 = {r.px, r.py, r.pz};
-  V3<double> normal = sag_normal<K>(s, p1.x, p1.y, p1.z);
+  return sag_normal<K>(s, r.px, r.py, r.pz);
+}
 
+// From the intercept on, along diffraction-order path `path`.
+template <int F = FEAT_ALL, uint32_t K = 0>
+OPTK_HD void surface_leave(const optk_surface &s, const SystemView &sys, int path, V3<double> normal,
+                           Ray<double> &r) {
+  V3<double> p1 = {r.px, r.py, r.pz};
   V3<double> a = {r.dx, r.dy, r.dz};
   int order = 0;
   const bool ruled = (F & FEAT_RULINGS) && k_rulings<K>(s) != OPTK_RULINGS_NONE;
@@ -675,7 +699,8 @@ OPTK_HD void propagate_surface(const optk_surface &s, const SystemView &sys, int
   double wavelength_2 = ratio == 1.0 ? r.wavelength : r.wavelength / ratio;
   V3<double> b = snells_law(a, n1, n2, normal, k_mirror<K>(s));
   double eff =
-      material_efficiency<F, K>(s, sys.sv, r.wavelength, a, r.index, r.attenuation, normal);
+      material_efficiency<F, K>(s, sys.sv, r.wavelength, a, r.index, r.attenuation, normal,
+                                r.rare);
   if (ruled)
     eff = eff * rulings_efficiency<double, K>(s, order, r.wavelength, a, p1, normal, sys.sv.tables);
   r.intensity = r.intensity * eff;
@@ -694,6 +719,13 @@ OPTK_HD void propagate_surface(const optk_surface &s, const SystemView &sys, int
   }
 
   xf_apply_ray<Kinds<K>::xf>(s.transform, r.px, r.py, r.pz, r.dx, r.dy, r.dz);
+}
+
+template <int F = FEAT_ALL, uint32_t K = 0>
+OPTK_HD void propagate_surface(const optk_surface &s, const SystemView &sys, int path,
+                               Ray<double> &r) {
+  const V3<double> normal = surface_arrive<F, K>(s, r);
+  surface_leave<F, K>(s, sys, path, normal, r);
 }
 
 // ---------------------------------------------------------------------------
@@ -787,6 +819,7 @@ OPTK_HD Ray<double> grid_ray(double fx, double fy, double ux, double uy, double 
   r.attenuation = 0.0;
   r.index = 1.0;
   r.unvignetted = true;
+  r.rare = false;
   return r;
 }
 

@@ -215,6 +215,25 @@ def multilayer(layers, substrate, wavelength, cos, n):
     return outs
 
 
+def multilayer_column(layers, substrate, wavelength, cos, n, film):
+    """Host s/p-averaged efficiency through the trace kernels' multilayer
+    code: (float64, float32, where the float64 one applies, where the
+    float32 one does)."""
+    from optika_amd import _compile, materials, surfaces
+
+    s = surfaces.Surface(material=materials.MultilayerMirror(layers=layers, substrate=substrate))
+    d, tab = _desc(_compile.build_records([s]))
+    wl, c = (np.ascontiguousarray(np.broadcast_to(a, np.shape(wavelength)), dtype=np.float64)
+             for a in (wavelength, cos))
+    nn = np.broadcast_to(np.asarray(n, complex), wl.shape)
+    nre, nim = np.ascontiguousarray(nn.real), np.ascontiguousarray(nn.imag)
+    e64, e32 = np.empty(wl.size), np.empty(wl.size)
+    ok = np.empty(wl.size, np.uint8)
+    lib().host_multilayer_column(ctypes.byref(d), _dp(wl), _dp(c), _dp(nre), _dp(nim), ctypes.c_int64(wl.size),
+                                 ctypes.c_int(int(film)), _dp(e64), _dp(e32), ok.ctypes.data_as(ctypes.c_void_p))
+    return e64, e32, (ok & 1).astype(bool), (ok & 2).astype(bool)
+
+
 def grid_bracket(w, x):
     """Brackets of ``x`` in the ascending table ``w`` through the index grid
     of optk_physics.h: (j, steps walked, cell count)."""
