@@ -545,7 +545,7 @@ OPTK_HD float toroid_residual_solve(const FastSurface &f, float X, float Y, floa
     float zs = f.surf_row[0] * x + f.surf_row[1] * y + f.surf_row[2] * z + f.surf_tz;
     float step = (zs - e.z) / (dzs - (e.dzdx * ux + e.dzdy * uy));
     s -= step;
-    if (fabsf(step) <= 1e-6f) break;
+    if (newton_done(step, f.c, f.r, 1e-6f, 1e-9f)) break;
   }
   return s;
 }

@@ -198,6 +198,24 @@ OPTK_HD V3<double> sag_normal(const optk_surface &s, double x, double y, double 
 #define OPTK_NEWTON_MAX_ITER 64
 #define OPTK_NEWTON_TOL 1e-13
 
+// The toroid's Newton iteration is done after a step whose square, times the
+// curvature, leaves less than the root's own rounding: the next error is at
+// most about step^2 (|c| + 1/|r|) / 2.  A fixed tolerance of 1e-13 mm lies
+// below one ulp of a path of a metre (2.3e-13), so on the spectrograph's
+// grating the step kept dithering about the root: 34 iterations a ray on
+// average and 64 in every wave, against 3 or 4 with this rule, and no
+// closer to it (CPU check over 2e4 rays: 1.34e-13 against 1.1e-13 mm rms of
+// the root in extended precision).  The host build keeps the fixed
+// tolerance and with it the oracle's very iterates.  A NaN (a ray that
+// misses) ends the iteration too.
+template <typename T> OPTK_HD bool newton_done(T step, T c, T r, T tol, T rounding) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return !(fabs(step) > tol && step * step * (fabs(c * r) + T(1)) > rounding * fabs(r));
+#else
+  return fabs(step) <= tol;
+#endif
+}
+
 // Intercept in the sag frame: returns the path length t along u.
 template <uint32_t K = 0>
 OPTK_HD double sag_intercept_t(const optk_surface &s, double ox, double oy, double oz, double ux,
@@ -293,7 +311,7 @@ OPTK_HD double toroid_intercept_t(const optk_surface &s, double ox, double oy, d
     double fder = uz - (dzdx * vx + dzdy * vy);
     double step = fval / fder;
     t = t - step;
-    if (fabs(step) <= OPTK_NEWTON_TOL) break;
+    if (newton_done(step, c, r, OPTK_NEWTON_TOL, 1e-15)) break;
   }
   return t;
 }
