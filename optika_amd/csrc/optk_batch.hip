@@ -341,9 +341,10 @@ int32_t optk_batch_create(const optk_batch_desc *desc, optk_batch **out) {
   for (auto &s : surfaces) derive_constants(s);
   // the specialised kernels serve a batch whose instances all match one
   // signature (perturbations keep the kinds of every record)
-  int32_t signature = find_signature(surfaces.data(), S, features);
+  const bool bilayers = all_bilayers(base);
+  int32_t signature = find_signature(surfaces.data(), S, features, bilayers);
   for (int i = 1; i < N && signature >= 0; ++i)
-    if (find_signature(surfaces.data() + (size_t)i * S, S, features) != signature) signature = -1;
+    if (find_signature(surfaces.data() + (size_t)i * S, S, features, bilayers) != signature) signature = -1;
 
   optk_batch *b = new optk_batch();
   b->num_instances = N;

@@ -736,8 +736,11 @@ OPTK_HD float fast_material_efficiency(const optk_surface &s, const StackView &s
     const double c64 = -(a.x * normal.x + a.y * normal.y + a.z * normal.z);
     if (!(F & FEAT_REFERENCE)) {
       const float k = attenuation * wavelength / (4.0f * 3.14159265358979f) * 1e-6f;
-      MLResult<float> m = multilayer_column<float>(sv, s.stack, wavelength, Cf{(float)c64, 0.0f}, Cf{index, k},
-                                                   film, LayerIndex32{sv, tables32, wavelength});
+      const Cf cosv = {(float)c64, 0.0f}, n = {index, k};
+      const LayerIndex32 at{sv, tables32, wavelength};
+      MLResult<float> m = (F & FEAT_BILAYER) || is_bilayer(sv.layers, sv.stacks[s.stack])
+                              ? multilayer_bilayer<float>(sv, s.stack, wavelength, cosv, n, film, at)
+                              : multilayer_column<float>(sv, s.stack, wavelength, cosv, n, film, at);
       if (m.ok || (F & FEAT_DEFER)) {
         rare = rare || !m.ok;
         if (!silicon) return m.efficiency;
@@ -751,7 +754,7 @@ OPTK_HD float fast_material_efficiency(const optk_surface &s, const StackView &s
     const C<double> n64 = {(double)index, (double)attenuation * w64 / (4.0 * M_PI) * 1e-6};
     if (silicon)
       return (float)silicon_absorbance_average(sv, s.stack, s.material_p[0], w64, C<double>{c64, 0.0}, n64);
-    MultilayerRT<double> rt = multilayer_efficiency<double>(sv, s.stack, w64, C<double>{c64, 0.0}, n64, film);
+    MultilayerRT<double> rt = multilayer_efficiency<double, (F & FEAT_BILAYER) != 0>(sv, s.stack, w64, C<double>{c64, 0.0}, n64, film);
     return (float)(film ? (rt.T[0] + rt.T[1]) / 2.0 : (rt.R[0] + rt.R[1]) / 2.0);
   }
   default:

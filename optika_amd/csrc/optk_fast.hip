@@ -189,9 +189,8 @@ size_t fast_staged_bytes(int num_surfaces) {
 template <int F> struct FastWaves {
   static constexpr int value = F == 0 ? 6 : ((F & FEAT_MULTILAYER) ? 2 : 4);
 };
-// the specialised kernels: 3 waves for the multilayer layout (168 VGPRs)
-// measured 2 % faster on the spectrograph than 2 (256 VGPRs), 4 (128
-// VGPRs) 16 % slower
+// the specialised kernels: 3 waves for the multilayer layouts (168 VGPRs;
+// spectrograph, 8.4M rays: 2.29 ms, at 2 waves 2.52 ms)
 template <int F> struct FastSpecWaves {
   static constexpr int value = F == 0 ? 6 : ((F & FEAT_MULTILAYER) ? 3 : 4);
 };
@@ -361,13 +360,13 @@ __device__ __forceinline__ void fast_spec_body(const FastArgs &A, const In &in) 
   for (int path = 0; path < num_paths; ++path) {
     FRay r = r0;
     int k = 0;
-    (fast_spec_step<F | FEAT_DEFER, K>(k++, k0, c_fast, c_surf, v, path, r), ...);
+    (fast_spec_step<F | FEAT_DEFER | FEAT_BILAYER, K>(k++, k0, c_fast, c_surf, v, path, r), ...);
     if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
       // the whole path again, so that nothing is kept live for it above
       r = load_ray32<IO>(in, i32);
       fast_first_hop(A, skip, r);
-      fast_path<F | FEAT_REFERENCE, false>(c_fast, c_surf, v, k0, A.num_surfaces, path, num_paths, A.n, i32,
-                                           FRaysOut{}, r);
+      k = 0;
+      (fast_spec_step<F | FEAT_REFERENCE | FEAT_BILAYER, K>(k++, k0, c_fast, c_surf, v, path, r), ...);
     }
     const optk_affine &last = *(const optk_affine *)&c_spec->last[A.apply_post];
     fast_xf(last, r);
@@ -533,8 +532,12 @@ template <int F, uint32_t... K> struct Tracer32Spec : Tracer32<F> {
     const int k0 = this->s_spec->skip_first != 0 ? 1 : 0;
     FRay r = this->start(i);
     int k = 0;
-    (batch_fast_step<F | FEAT_DEFER, K>(k++, k0, this->s_fast, this->s_surf, v, path, r), ...);
-    if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) this->reference(v, i, path, r);
+    (batch_fast_step<F | FEAT_DEFER | FEAT_BILAYER, K>(k++, k0, this->s_fast, this->s_surf, v, path, r), ...);
+    if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
+      r = this->start(i);
+      k = 0;
+      (batch_fast_step<F | FEAT_REFERENCE | FEAT_BILAYER, K>(k++, k0, this->s_fast, this->s_surf, v, path, r), ...);
+    }
     const optk_affine &last = this->s_spec->last[this->A.apply_post];
     fast_xf(last, r);
     store_f(this->out, (int64_t)path * this->A.n + i, r);

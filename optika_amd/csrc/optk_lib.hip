@@ -163,11 +163,11 @@ static size_t staged_bytes(int num_surfaces) {
 template <int F> struct Waves {
   static constexpr int value = (F & FEAT_MULTILAYER) ? 2 : 4;
 };
-// the specialised kernels: 4 waves also for the multilayer layout (128
-// VGPRs, more of the multilayer's temporaries spilled), measured 2.5 %
-// faster on the spectrograph than 2 waves with 256 VGPRs
+// the specialised kernels: the multilayer layouts at 2 waves (256 VGPRs, the
+// main path without spills).  Spectrograph, 2.0M rays: 864 us at 2 waves,
+// 892 us at 3 (168 VGPRs, 100 spills)
 template <int F> struct SpecWaves {
-  static constexpr int value = 4;
+  static constexpr int value = (F & FEAT_MULTILAYER) ? 2 : 4;
 };
 
 // I/O layouts of the kernels.  IO_ANY honours every null pointer of the
@@ -370,13 +370,13 @@ __device__ __forceinline__ void spec_body(const TraceArgs &A, const In &in) {
   for (int path = 0; path < num_paths; ++path) {
     Ray<double> r = r0;
     int k = 0;
-    (propagate_surface<F | FEAT_DEFER, K>(*(const optk_surface *)&c_surf[k++], sys, path, r), ...);
+    (propagate_surface<F | FEAT_DEFER | FEAT_BILAYER, K>(*(const optk_surface *)&c_surf[k++], sys, path, r), ...);
     if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
       // the whole path again, so that nothing is kept live for it above
       r = load_io32<IO>(in, i32);
       apply_pre(spec, r);
-      for (k = 0; k < A.num_surfaces; ++k)
-        propagate_surface<F | FEAT_REFERENCE>(*(const optk_surface *)&c_surf[k], sys, path, r);
+      k = 0;
+      (propagate_surface<F | FEAT_REFERENCE | FEAT_BILAYER, K>(*(const optk_surface *)&c_surf[k++], sys, path, r), ...);
     }
     if (A.apply_post) xf_inverse_ray(spec.post, r.px, r.py, r.pz, r.dx, r.dy, r.dz);
     store_io32<IO>(A.out, (uint32_t)path * n32 + i32, r);
@@ -623,12 +623,12 @@ template <int F, uint32_t... K> struct Tracer64Spec : Tracer64<F> {
     SystemView sys = this->s_spec->sys;
     sys.surfaces = this->s_surf;
     int k = 0;
-    (propagate_surface<F | FEAT_DEFER, K>(this->s_surf[k++], sys, path, r), ...);
+    (propagate_surface<F | FEAT_DEFER | FEAT_BILAYER, K>(this->s_surf[k++], sys, path, r), ...);
     if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
       r = load_ray(this->in, i);
       apply_pre(*this->s_spec, r);
-      for (k = 0; k < this->A.num_surfaces; ++k)
-        propagate_surface<F | FEAT_REFERENCE>(this->s_surf[k], sys, path, r);
+      k = 0;
+      (propagate_surface<F | FEAT_REFERENCE | FEAT_BILAYER, K>(this->s_surf[k++], sys, path, r), ...);
     }
     if (this->A.apply_post) {
       xf_inverse_ray(this->s_spec->post, r.px, r.py, r.pz, r.dx, r.dy, r.dz);
@@ -1547,7 +1547,8 @@ int32_t optk_system_create(const optk_system_desc *desc, optk_system **out) {
   s->host_surfaces.assign(desc->surfaces, desc->surfaces + desc->num_surfaces);
   for (auto &surf : s->host_surfaces) derive_constants(surf);
   s->features = variant_of(features_of(desc));
-  s->signature = find_signature(s->host_surfaces.data(), desc->num_surfaces, s->features);
+  s->signature = find_signature(s->host_surfaces.data(), desc->num_surfaces, s->features,
+                                all_bilayers(*desc));
   if ((rc = upload(&s->surfaces, s->host_surfaces.data(), desc->num_surfaces)) ||
       (rc = upload(&s->layers, desc->layers, desc->num_layers)) ||
       (rc = upload(&s->stacks, desc->stacks, desc->num_stacks)) ||

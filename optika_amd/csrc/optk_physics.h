@@ -481,7 +481,8 @@ template <typename T> struct M2Pair {
 
 // matrices.refraction (matrices.py:127-161) for one polarization, from the
 // incident medium (n_i, cos_i) into (n_j, cos_j)
-template <typename T>
+// (SMOOTH: no layer of the stack has a roughness profile)
+template <typename T, bool SMOOTH = false>
 OPTK_HD M2<T> refraction_matrix(const optk_layer &layer, T wavelength, bool pol_s, C<T> n_i,
                                 C<T> cos_i, C<T> n_j, C<T> cos_j) {
   C<T> one = {T(1), T(0)};
@@ -494,7 +495,7 @@ OPTK_HD M2<T> refraction_matrix(const optk_layer &layer, T wavelength, bool pol_
   C<T> a = cadd(qi, qj);
   C<T> r = cdiv(csub(qi, qj), a);
   C<T> t = cdiv(cscale(T(2), qi), a);
-  if (layer.profile_kind != OPTK_PROFILE_NONE) {
+  if (!SMOOTH && layer.profile_kind != OPTK_PROFILE_NONE) {
     T f = profile_factor<T>(layer.profile_kind, T(layer.profile_width), wavelength, di, n_i);
     r = cscale(f, r);  // r * factor (real factor promoted to complex)
   }
@@ -510,14 +511,14 @@ OPTK_HD M2<T> refraction_matrix(const optk_layer &layer, T wavelength, bool pol_
 // matrix keeps the reference's operation order, so the result is the same
 // as two separate per-polarization passes.  `n_int` is the layer's index
 // at this wavelength (chemical_n).
-template <typename T>
+template <typename T, bool SMOOTH = false>
 OPTK_HD M2Pair<T> layer_transfer2(const optk_layer &layer, C<T> n_int, T wavelength,
                                   LayerState<T> &st, T thickness) {
   C<T> d_int = snell_scalar(st.direction, st.n, n_int);
   M2Pair<T> refr;
   if (st.where) {
-    refr.s = refraction_matrix<T>(layer, wavelength, true, st.n, st.direction, n_int, d_int);
-    refr.p = refraction_matrix<T>(layer, wavelength, false, st.n, st.direction, n_int, d_int);
+    refr.s = refraction_matrix<T, SMOOTH>(layer, wavelength, true, st.n, st.direction, n_int, d_int);
+    refr.p = refraction_matrix<T, SMOOTH>(layer, wavelength, false, st.n, st.direction, n_int, d_int);
   } else {
     refr.s = midentity<T>();
     refr.p = midentity<T>();
@@ -569,7 +570,7 @@ OPTK_HD C<T> layer_index(const optk_layer &L, const StackView &sv, T wavelength)
 // LayerSequence.transfer over layers first .. first + count - 1, both
 // polarizations; `n_cache` holds the indices of the first 4 layers when
 // `cached` (a periodic block's second pass reuses its first pass's lookups)
-template <typename T>
+template <typename T, bool SMOOTH = false>
 OPTK_HD M2Pair<T> sequence_transfer2(const StackView &sv, int first, int count, T wavelength,
                                      LayerState<T> &st, C<T> n_cache[4], bool cached) {
   M2Pair<T> result = {midentity<T>(), midentity<T>()};
@@ -588,7 +589,7 @@ OPTK_HD M2Pair<T> sequence_transfer2(const StackView &sv, int first, int count, 
       if (i == 2) n_cache[2] = n_int;
       if (i == 3) n_cache[3] = n_int;
     }
-    M2Pair<T> x = layer_transfer2<T>(L, n_int, wavelength, st, T(L.thickness));
+    M2Pair<T> x = layer_transfer2<T, SMOOTH>(L, n_int, wavelength, st, T(L.thickness));
     result.s = mmul(result.s, x.s);
     result.p = mmul(result.p, x.p);
   }
@@ -602,7 +603,7 @@ template <typename T> struct MultilayerOut {
 };
 
 // multilayer_coefficients (optika/materials/_multilayers.py:186-237)
-template <typename T>
+template <typename T, bool SMOOTH = false>
 OPTK_HD MultilayerOut<T> multilayer_rt(const StackView &sv, int stack_index, T wavelength,
                                        C<T> direction, C<T> n_ambient) {
   const optk_stack &stk = sv.stacks[stack_index];
@@ -616,13 +617,13 @@ OPTK_HD MultilayerOut<T> multilayer_rt(const StackView &sv, int stack_index, T w
     M2Pair<T> x;
     if (blk.kind == OPTK_BLOCK_PERIODIC) {
       M2Pair<T> start =
-          sequence_transfer2<T>(sv, blk.first_layer, blk.num_layers, wavelength, st, n_cache, false);
+          sequence_transfer2<T, SMOOTH>(sv, blk.first_layer, blk.num_layers, wavelength, st, n_cache, false);
       M2Pair<T> periodic =
-          sequence_transfer2<T>(sv, blk.first_layer, blk.num_layers, wavelength, st, n_cache, true);
+          sequence_transfer2<T, SMOOTH>(sv, blk.first_layer, blk.num_layers, wavelength, st, n_cache, true);
       x.s = mmul(start.s, matrix_power(periodic.s, blk.num_periods - 1));
       x.p = mmul(start.p, matrix_power(periodic.p, blk.num_periods - 1));
     } else {
-      x = sequence_transfer2<T>(sv, blk.first_layer, blk.num_layers, wavelength, st, n_cache, false);
+      x = sequence_transfer2<T, SMOOTH>(sv, blk.first_layer, blk.num_layers, wavelength, st, n_cache, false);
     }
     // a single top-level block is returned by its own transfer(); several
     // blocks are folded left from the identity (LayerSequence.transfer)
@@ -637,7 +638,7 @@ OPTK_HD MultilayerOut<T> multilayer_rt(const StackView &sv, int stack_index, T w
   // substrate (thickness forced to zero)
   optk_layer sub = {-1, OPTK_PROFILE_NONE, 0.0, 0.0};
   if (stk.substrate_layer >= 0) sub = sv.layers[stk.substrate_layer];
-  M2Pair<T> ms = layer_transfer2<T>(sub, layer_index<T>(sub, sv, wavelength), wavelength, st, T(0));
+  M2Pair<T> ms = layer_transfer2<T, SMOOTH>(sub, layer_index<T>(sub, sv, wavelength), wavelength, st, T(0));
   M2<T> mt[2] = {mmul(m.s, ms.s), mmul(m.p, ms.p)};
   for (int p = 0; p < 2; ++p) {
     out.r[p] = cdiv(mt[p].c, mt[p].a);
@@ -654,12 +655,12 @@ template <typename Real> struct MultilayerRT {
 };
 
 // multilayer_efficiency (optika/materials/_multilayers.py:485-532)
-template <typename T>
+template <typename T, bool SMOOTH = false>
 OPTK_HD MultilayerRT<T> multilayer_efficiency(const StackView &sv, int stack_index, T wavelength,
                                               C<T> direction, C<T> n_ambient,
                                               bool want_transmission,
                                               MultilayerOut<T> *coeffs = nullptr) {
-  MultilayerOut<T> co = multilayer_rt<T>(sv, stack_index, wavelength, direction, n_ambient);
+  MultilayerOut<T> co = multilayer_rt<T, SMOOTH>(sv, stack_index, wavelength, direction, n_ambient);
   if (coeffs) *coeffs = co;
   MultilayerRT<T> out;
   for (int p = 0; p < 2; ++p) {
@@ -853,6 +854,29 @@ template <typename T> struct MLColumn {
 template <typename T> struct MLPhase {
   C<T> u00, u11;  // exp(-i beta), exp(+i beta)
 };
+// the Snell invariant (n_amb sin_amb)^2
+template <typename T> OPTK_HD C<T> ml_kappa2(C<T> cos_amb, C<T> n_amb) {
+  const C<T> one_minus = {T(1) - (cos_amb.re * cos_amb.re - cos_amb.im * cos_amb.im),
+                          T(-2) * cos_amb.re * cos_amb.im};
+  return ml_mul(ml_sqr(n_amb), one_minus);
+}
+
+// the refracted cosine: the principal square root of 1 - s2, s2 the squared
+// sine
+template <typename T> OPTK_HD C<T> ml_cosine(C<T> s2, bool &ok) {
+  const T x = T(1) - s2.re, y = -s2.im;
+  const T d = ml_sqrt(ml_fma(x, x, y * y));
+  const T w = ml_sqrt(T(0.5) * (d + fabs(x)));
+  const T v = T(0.5) * fabs(y) * ml_rcp(w);
+  ok = ok && !(x <= T(0) && y == T(0));
+  return x >= T(0) ? C<T>{w, copysign(v, y)} : C<T>{v, copysign(w, y)};
+}
+
+// a NaN stands only where the ray brought one (it missed a surface)
+template <typename T> OPTK_HD bool ml_accept(T value, T cosine, T wavelength) {
+  return value == value || cosine != cosine || wavelength != wavelength;
+}
+
 // one medium: index, cosine, and for each polarization q (s: n cos, p:
 // conj(cos) / n) and 1 / (2 q)
 template <typename T> struct MLMedium {
@@ -874,30 +898,21 @@ OPTK_HD MLMedium<T> ml_medium_of(C<T> n, C<T> ninv, C<T> cosine) {
   return m;
 }
 
-// the medium of index n, its cosine from the Snell invariant
-// kappa2 = (n_amb sin_amb)^2
+// the medium of index n
 template <typename T> OPTK_HD MLMedium<T> ml_medium(C<T> n, C<T> kappa2, bool &ok) {
   const C<T> n2inv = ml_inv(ml_sqr(n));
-  const C<T> s2 = ml_mul(kappa2, n2inv);
-  const T x = T(1) - s2.re, y = -s2.im;
-  // principal square root of x + i y
-  const T d = ml_sqrt(ml_fma(x, x, y * y));
-  const T w = ml_sqrt(T(0.5) * (d + fabs(x)));
-  const T v = T(0.5) * fabs(y) * ml_rcp(w);
-  ok = ok && !(x <= T(0) && y == T(0));
-  const C<T> cosine = x >= T(0) ? C<T>{w, copysign(v, y)} : C<T>{v, copysign(w, y)};
-  return ml_medium_of<T>(n, ml_mul(n, n2inv), cosine);
+  return ml_medium_of<T>(n, ml_mul(n, n2inv), ml_cosine<T>(ml_mul(kappa2, n2inv), ok));
 }
 
 // beta = 2 pi h n cos / wavelength (matrices.py:241-246)
 template <typename T>
-OPTK_HD MLPhase<T> ml_phase(const MLMedium<T> &m, T thickness, T wavelength, T inv_wavelength, bool &ok) {
+OPTK_HD MLPhase<T> ml_phase(C<T> n_cos, T thickness, T wavelength, T inv_wavelength, bool &ok) {
   // the quotient corrected by its residual: its relative error is the
   // phase's, and a repeated period multiplies it
   const T turn = T(2.0 * M_PI) * thickness;
   const T quot = turn * inv_wavelength;
   const T scale = ml_fma(ml_fma(-quot, wavelength, turn), inv_wavelength, quot);
-  const T b_re = scale * m.qs.re, b_im = scale * m.qs.im;
+  const T b_re = scale * n_cos.re, b_im = scale * n_cos.im;
   ok = ok && !(fabs(b_re) > ml_angle_limit(T(0))) && !(fabs(b_im) > T(24));
   T s, c;
   ml_sincos(b_re, s, c);
@@ -971,9 +986,7 @@ OPTK_HD MLResult<T> multilayer_column(const StackView &sv, int stack_index, T wa
   const optk_stack &stk = sv.stacks[stack_index];
   MLResult<T> out;
   bool ok = !(fabs(cos_amb.re) < T(OPTK_GRAZING_COS));
-  const C<T> one_minus = {T(1) - (cos_amb.re * cos_amb.re - cos_amb.im * cos_amb.im),
-                          T(-2) * cos_amb.re * cos_amb.im};
-  const C<T> kappa2 = ml_mul(ml_sqr(n_amb), one_minus);
+  const C<T> kappa2 = ml_kappa2<T>(cos_amb, n_amb);
   const T inv_wavelength = ml_rcp(wavelength);
   optk_layer right = {-1, OPTK_PROFILE_NONE, 0.0, 0.0};  // the layer whose left interface is pending
   if (stk.substrate_layer >= 0) right = sv.layers[stk.substrate_layer];
@@ -988,7 +1001,7 @@ OPTK_HD MLResult<T> multilayer_column(const StackView &sv, int stack_index, T wa
     // the block's last medium, and the interface from it to the right
     optk_layer L = sv.layers[blk.first_layer + k];
     MLMedium<T> med = ml_medium<T>(index(L), kappa2, ok);
-    MLPhase<T> u = ml_phase<T>(med, T(L.thickness), wavelength, inv_wavelength, ok);
+    MLPhase<T> u = ml_phase<T>(med.qs, T(L.thickness), wavelength, inv_wavelength, ok);
     MLCross<T> x = ml_cross<T>(med, cur, right, wavelength);
     ml_apply(x.s, s);
     ml_apply(x.p, p);
@@ -1000,7 +1013,7 @@ OPTK_HD MLResult<T> multilayer_column(const StackView &sv, int stack_index, T wa
         cur = med;
         L = sv.layers[blk.first_layer + k - 1];
         med = ml_medium<T>(index(L), kappa2, ok);
-        u = ml_phase<T>(med, T(L.thickness), wavelength, inv_wavelength, ok);
+        u = ml_phase<T>(med.qs, T(L.thickness), wavelength, inv_wavelength, ok);
         x = ml_cross<T>(med, cur, right, wavelength);
         ml_apply(x.s, s);
         ml_apply(x.p, p);
@@ -1026,7 +1039,7 @@ OPTK_HD MLResult<T> multilayer_column(const StackView &sv, int stack_index, T wa
         cur = med;
         L = sv.layers[blk.first_layer + k - 1];
         med = ml_medium<T>(index(L), kappa2, ok);
-        u = ml_phase<T>(med, T(L.thickness), wavelength, inv_wavelength, ok);
+        u = ml_phase<T>(med.qs, T(L.thickness), wavelength, inv_wavelength, ok);
         x = ml_cross<T>(med, cur, right, wavelength);
         inner_s = first ? ml_layer(x.s, uk) : ml_layer_times(x.s, uk, inner_s);
         inner_p = first ? ml_layer(x.p, uk) : ml_layer_times(x.p, uk, inner_p);
@@ -1071,8 +1084,88 @@ OPTK_HD MLResult<T> multilayer_column(const StackView &sv, int stack_index, T wa
   } else {
     out.efficiency = T(0.5) * ml_fma(ml_abs2(s.c), is, ml_abs2(p.c) * ip);
   }
-  // a NaN stands only where the ray brought one (it missed a surface)
-  out.ok = ok && (out.efficiency == out.efficiency || cos_amb.re != cos_amb.re || wavelength != wavelength);
+  out.ok = ok && ml_accept<T>(out.efficiency, cos_amb.re, wavelength);
+  return out;
+}
+
+// The coating of a normal-incidence EUV or soft x-ray mirror is one periodic
+// block of two smooth layers on a substrate.  For that form the column's
+// polarizations run one after the other, so that one period matrix, one
+// inner matrix and one column are live at a time instead of two: with both
+// at once the spectrograph's float64 kernel spilled 1,400 registers, and
+// waited on that scratch traffic for three quarters of its time.
+OPTK_HD bool is_bilayer(const optk_layer *layers, const optk_stack &s) {
+  if (s.num_blocks != 1 || s.blocks[0].kind != OPTK_BLOCK_PERIODIC || s.blocks[0].num_layers != 2) return false;
+  const optk_layer *l = layers + s.blocks[0].first_layer;
+  return l[0].profile_kind == OPTK_PROFILE_NONE && l[1].profile_kind == OPTK_PROFILE_NONE &&
+         (s.substrate_layer < 0 || layers[s.substrate_layer].profile_kind == OPTK_PROFILE_NONE);
+}
+
+template <typename T> struct MLSlim {
+  C<T> n, ninv, cos;
+};
+
+template <typename T> OPTK_HD MLSlim<T> ml_slim(C<T> n, C<T> kappa2, bool &ok) {
+  const C<T> n2inv = ml_inv(ml_sqr(n));
+  const C<T> s2 = ml_mul(kappa2, n2inv);
+  return {n, ml_mul(n, n2inv), ml_cosine<T>(s2, ok)};
+}
+
+// q of one polarization (0: s, n cos; 1: p, conj(cos) / n)
+template <typename T> OPTK_HD C<T> ml_q(const MLSlim<T> &m, int pol) {
+  return pol ? ml_mul(cconj(m.cos), m.ninv) : ml_mul(m.cos, m.n);
+}
+
+template <typename T, typename Index>
+OPTK_HD MLResult<T> multilayer_bilayer(const StackView &sv, int stack_index, T wavelength, C<T> cos_amb,
+                                       C<T> n_amb, bool film, Index index) {
+  const optk_stack &stk = sv.stacks[stack_index];
+  const optk_layer *layer = sv.layers + stk.blocks[0].first_layer;
+  MLResult<T> out;
+  bool ok = !(fabs(cos_amb.re) < T(OPTK_GRAZING_COS));
+  const C<T> kappa2 = ml_kappa2<T>(cos_amb, n_amb);
+  const T inv_wavelength = ml_rcp(wavelength);
+  optk_layer sub = {-1, OPTK_PROFILE_NONE, 0.0, 0.0};
+  if (stk.substrate_layer >= 0) sub = sv.layers[stk.substrate_layer];
+  const MLSlim<T> m0 = {n_amb, ml_inv(n_amb), cos_amb};
+  const MLSlim<T> m1 = ml_slim<T>(index(layer[0]), kappa2, ok);
+  const MLSlim<T> m2 = ml_slim<T>(index(layer[1]), kappa2, ok);
+  const MLSlim<T> m3 = ml_slim<T>(index(sub), kappa2, ok);
+  const MLPhase<T> u1 = ml_phase<T>(ml_mul(m1.cos, m1.n), T(layer[0].thickness), wavelength, inv_wavelength, ok);
+  const MLPhase<T> u2 = ml_phase<T>(ml_mul(m2.cos, m2.n), T(layer[1].thickness), wavelength, inv_wavelength, ok);
+  const int periods = stk.blocks[0].num_periods;
+  const T big = sizeof(T) == 8 ? T(1e300) : T(1e37);
+  out.efficiency = T(0);
+#pragma unroll 1
+  for (int pol = 0; pol < 2; ++pol) {
+    const C<T> q1 = ml_q<T>(m1, pol), q2 = ml_q<T>(m2, pol), q3 = ml_q<T>(m3, pol);
+    const C<T> h2 = cscale(T(0.5), ml_inv(q2));
+    MLColumn<T> v = {ml_mul(cadd(q2, q3), h2), ml_mul(csub(q2, q3), h2)};
+    const MLInterface<T> x12 = ml_interface<T>(q1, cscale(T(0.5), ml_inv(q1)), q2, T(1));
+    const M2<T> inner = ml_layer(x12, u2);
+    int e = periods - 1;
+    if (e > 0) {
+      M2<T> z = ml_layer_times(ml_interface<T>(q2, h2, q1, T(1)), u1, inner);
+      for (;;) {
+        if (e & 1) ml_apply(z, v);
+        e >>= 1;
+        if (e == 0) break;
+        z = ml_square(z);
+      }
+    }
+    ml_apply(inner, v);
+    ml_apply(u1, v);
+    const C<T> q0 = ml_q<T>(m0, pol);
+    const C<T> h0 = cscale(T(0.5), ml_inv(q0));
+    ml_apply(ml_interface<T>(q0, h0, q1, T(1)), v);
+    const T a2 = ml_abs2(v.a);
+    ok = ok && !(a2 > big) && !(a2 < T(1) / big);
+    // |r|^2, or |t|^2 Re(q_sub / q_amb) with 1 / q_amb = 2 h
+    const T value = film ? T(2) * ml_mul(q3, h0).re : ml_abs2(v.c);
+    out.efficiency = ml_fma(T(0.5) * value, ml_rcp(a2), out.efficiency);
+  }
+  out.im_q_sub = ml_mul(m3.cos, m3.n).im;
+  out.ok = ok && ml_accept<T>(out.efficiency, cos_amb.re, wavelength);
   return out;
 }
 

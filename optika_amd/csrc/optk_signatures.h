@@ -89,12 +89,20 @@ constexpr Signature SIGNATURES[NUM_SIGNATURES] = {
     {FEAT_ALL, 5, {OPTK_SIGNATURE_SPECTROGRAPH_TILTED}},
 };
 
-// the signature a system's records match (features: its kernel variant),
-// or -1
-inline int find_signature(const optk_surface *surfaces, int num_surfaces, int features) {
+// every coating of the system in the form the specialised kernels evaluate
+inline bool all_bilayers(const optk_system_desc &d) {
+  for (int i = 0; i < d.num_stacks; ++i)
+    if (!is_bilayer(d.layers, d.stacks[i])) return false;
+  return true;
+}
+
+// the signature a system's records match (features: its kernel variant;
+// bilayers: all_bilayers, which the multilayer layouts need), or -1
+inline int find_signature(const optk_surface *surfaces, int num_surfaces, int features, bool bilayers) {
   for (int k = 0; k < NUM_SIGNATURES; ++k) {
     const Signature &sig = SIGNATURES[k];
     if (sig.num_surfaces != num_surfaces || sig.features != features) continue;
+    if ((sig.features & FEAT_MULTILAYER) && !bilayers) continue;
     bool same = true;
     for (int i = 0; i < num_surfaces && same; ++i) same = kinds_of(surfaces[i]) == sig.kinds[i];
     if (same) return k;

@@ -24,6 +24,8 @@ enum : int {
   // every ray's.
   FEAT_DEFER = 8,
   FEAT_REFERENCE = 16,
+  // every stack of the system is a bilayer (is_bilayer), by the host's rule
+  FEAT_BILAYER = 32,
 };
 
 // Compile-time kinds of one surface record.  A specialised kernel fixes the
@@ -586,8 +588,10 @@ OPTK_HD double material_efficiency(const optk_surface &s, const StackView &sv, d
     C<double> n = {index, k};
     C<double> cosv = {-dot3(a, normal), 0.0};
     if (!(F & FEAT_REFERENCE)) {
-      MLResult<double> m = multilayer_column<double>(sv, s.stack, wavelength, cosv, n, film,
-                                                     LayerIndex64{sv, wavelength});
+      const LayerIndex64 at{sv, wavelength};
+      MLResult<double> m = (F & FEAT_BILAYER) || is_bilayer(sv.layers, sv.stacks[s.stack])
+                               ? multilayer_bilayer<double>(sv, s.stack, wavelength, cosv, n, film, at)
+                               : multilayer_column<double>(sv, s.stack, wavelength, cosv, n, film, at);
       if (m.ok || (F & FEAT_DEFER)) {
         rare = rare || !m.ok;
         if (!silicon) return m.efficiency;
@@ -597,7 +601,7 @@ OPTK_HD double material_efficiency(const optk_surface &s, const StackView &sv, d
       }
     }
     if (silicon) return silicon_absorbance_average(sv, s.stack, s.material_p[0], wavelength, cosv, n);
-    MultilayerRT<double> rt = multilayer_efficiency<double>(sv, s.stack, wavelength, cosv, n, film);
+    MultilayerRT<double> rt = multilayer_efficiency<double, (F & FEAT_BILAYER) != 0>(sv, s.stack, wavelength, cosv, n, film);
     return film ? (rt.T[0] + rt.T[1]) / 2.0 : (rt.R[0] + rt.R[1]) / 2.0;
   }
   default:

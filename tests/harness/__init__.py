@@ -215,9 +215,10 @@ def multilayer(layers, substrate, wavelength, cos, n):
     return outs
 
 
-def multilayer_column(layers, substrate, wavelength, cos, n, film):
+def multilayer_column(layers, substrate, wavelength, cos, n, film, general=True):
     """Host s/p-averaged efficiency through the trace kernels' multilayer
-    code: (float64, float32, where the float64 one applies, where the
+    code (``general``: the form for every stack also where the bilayer's
+    serves): (float64, float32, where the float64 one applies, where the
     float32 one does)."""
     from optika_amd import _compile, materials, surfaces
 
@@ -230,7 +231,7 @@ def multilayer_column(layers, substrate, wavelength, cos, n, film):
     e64, e32 = np.empty(wl.size), np.empty(wl.size)
     ok = np.empty(wl.size, np.uint8)
     lib().host_multilayer_column(ctypes.byref(d), _dp(wl), _dp(c), _dp(nre), _dp(nim), ctypes.c_int64(wl.size),
-                                 ctypes.c_int(int(film)), _dp(e64), _dp(e32), ok.ctypes.data_as(ctypes.c_void_p))
+                                 ctypes.c_int(int(film)), ctypes.c_int(int(general)), _dp(e64), _dp(e32), ok.ctypes.data_as(ctypes.c_void_p))
     return e64, e32, (ok & 1).astype(bool), (ok & 2).astype(bool)
 
 

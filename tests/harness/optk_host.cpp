@@ -259,19 +259,23 @@ int host_multilayer(const optk_system_desc *d, int stack, const double *wl, cons
   return 0;
 }
 
-// s/p-averaged efficiency of stack 0 through multilayer_column in both
-// precisions; ok[i] bit 0: the float64 one applies, bit 1: the float32 one
+// s/p-averaged efficiency of stack 0 through the trace kernels' multilayer
+// (multilayer_bilayer where the stack has its form, unless `general`) in
+// both precisions; ok[i] bit 0: the float64 one applies, bit 1: the float32 one
 void host_multilayer_column(const optk_system_desc *d, const double *wl, const double *cosine, const double *n_re,
-                            const double *n_im, int64_t n, int film, double *eff64, double *eff32, uint8_t *ok) {
+                            const double *n_im, int64_t n, int film, int general, double *eff64, double *eff32, uint8_t *ok) {
   SystemView v = view_of(d);
+  const bool two = !general && is_bilayer(v.sv.layers, v.sv.stacks[0]);
   std::vector<float> t32(d->tables, d->tables + d->num_tables);
   for (int64_t i = 0; i < n; ++i) {
-    const MLResult<double> a =
-        multilayer_column<double>(v.sv, 0, wl[i], C<double>{cosine[i], 0.0}, C<double>{n_re[i], n_im[i]},
-                                  film != 0, LayerIndex64{v.sv, wl[i]});
-    const MLResult<float> b = multilayer_column<float>(
-        v.sv, 0, (float)wl[i], Cf{(float)cosine[i], 0.0f}, Cf{(float)n_re[i], (float)n_im[i]}, film != 0,
-        LayerIndex32{v.sv, t32.data(), (float)wl[i]});
+    const C<double> c64 = {cosine[i], 0.0}, n64 = {n_re[i], n_im[i]};
+    const Cf c32 = {(float)cosine[i], 0.0f}, n32 = {(float)n_re[i], (float)n_im[i]};
+    const LayerIndex64 at64{v.sv, wl[i]};
+    const LayerIndex32 at32{v.sv, t32.data(), (float)wl[i]};
+    const MLResult<double> a = two ? multilayer_bilayer<double>(v.sv, 0, wl[i], c64, n64, film != 0, at64)
+                                   : multilayer_column<double>(v.sv, 0, wl[i], c64, n64, film != 0, at64);
+    const MLResult<float> b = two ? multilayer_bilayer<float>(v.sv, 0, (float)wl[i], c32, n32, film != 0, at32)
+                                  : multilayer_column<float>(v.sv, 0, (float)wl[i], c32, n32, film != 0, at32);
     eff64[i] = a.efficiency;
     eff32[i] = b.efficiency;
     ok[i] = (a.ok ? 1 : 0) | (b.ok ? 2 : 0);

@@ -1,5 +1,5 @@
-"""The trace kernels' multilayer (multilayer_column) on the CPU against the
-oracle's, over every form of stack it accepts, and what it hands back.
+"""The trace kernels' multilayer (multilayer_column, and multilayer_bilayer for
+the stacks of its form) on the CPU against the oracle's, over every form of stack it accepts, and what it hands back.
 
 Float64: both evaluate the same transfer matrices by different orders of a
 few thousand operations (M periods of L layers); each is within a few times
@@ -44,10 +44,13 @@ STACKS = {
 }
 
 
+BILAYERS = ("one period", "two periods", "forty periods")
+
+
 @pytest.mark.parametrize("film", [False, True])
 @pytest.mark.parametrize("cos", [1.0, 0.8, 0.2501])
-@pytest.mark.parametrize("name", sorted(STACKS))
-def test_column_against_the_oracle(name, cos, film):
+@pytest.mark.parametrize("name, general", [(n, True) for n in sorted(STACKS)] + [(n, False) for n in BILAYERS])
+def test_column_against_the_oracle(name, general, cos, film):
     layers = STACKS[name]
     wl = np.linspace(12.0, 70.0, 61).astype(np.float32).astype(np.float64)
     cos = float(np.float32(cos))
@@ -55,31 +58,36 @@ def test_column_against_the_oracle(name, cos, film):
         (Rs, Rp), (Ts, Tp) = oracle.multilayer_efficiency(wl, np.full(wl.shape, cos), np.full(wl.shape, n),
                                                           layers, Layer(OX))
         want = (Ts + Tp) / 2 if film else (Rs + Rp) / 2
-        e64, e32, ok64, ok32 = multilayer_column(layers, Layer(OX), wl, cos, n, film)
+        e64, e32, ok64, ok32 = multilayer_column(layers, Layer(OX), wl, cos, n, film, general)
         assert ok64.all() and ok32.mean() > 0.8
         scale = np.abs(want).max()
         assert np.abs(e64 - want).max() <= 2e-13 * scale
         assert np.abs(e32 - want)[ok32].max() <= 2e-5 * scale
 
 
-def test_column_hands_back_what_it_does_not_cover():
+@pytest.mark.parametrize("general", [True, False])
+def test_column_hands_back_what_it_does_not_cover(general):
+    from functools import partial
+
+    multilayer = partial(multilayer_column, general=general)
     two = STACKS["two periods"]
     wl = np.full(4, 60.0)
     # grazing incidence, either side of the line
-    _, _, ok64, ok32 = multilayer_column(two, Layer(OX), wl, np.array([0.2499, 0.1, -0.1, 0.0]), 1.0, False)
+    _, _, ok64, ok32 = multilayer(two, Layer(OX), wl, np.array([0.2499, 0.1, -0.1, 0.0]), 1.0, False)
     assert not ok64.any() and not ok32.any()
-    _, _, ok64, ok32 = multilayer_column(two, Layer(OX), wl, np.array([0.2501, 0.9, -0.9, 1.0]), 1.0, False)
+    _, _, ok64, ok32 = multilayer(two, Layer(OX), wl, np.array([0.2501, 0.9, -0.9, 1.0]), 1.0, False)
     assert ok64.all() and ok32.all()
     # the reference's |exp(-i beta)| < 1e10 guard: 20 um of silicon
-    thick = LayerSequence([Layer(SI, thickness=20000.0)])
-    _, _, ok64, ok32 = multilayer_column(thick, Layer(OX), wl, 1.0, 1.0, False)
+    thick = _period(1, Layer(SI, thickness=20000.0), Layer(MO, thickness=2.7))
+    _, _, ok64, ok32 = multilayer(thick, Layer(OX), wl, 1.0, 1.0, False)
     assert not ok64.any() and not ok32.any()
     # a ray that missed brings a NaN cosine and keeps it, without being handed back
-    e64, e32, ok64, ok32 = multilayer_column(two, Layer(OX), wl, np.nan, 1.0, False)
+    e64, e32, ok64, ok32 = multilayer(two, Layer(OX), wl, np.nan, 1.0, False)
     assert np.isnan(e64).all() and np.isnan(e32).all() and ok64.all() and ok32.all()
 
 
-def test_lossless_total_reflection_is_handed_back(monkeypatch):
+@pytest.mark.parametrize("general", [True, False])
+def test_lossless_total_reflection_is_handed_back(monkeypatch, general):
     """From inside a denser lossless ambient at an angle beyond the critical
     one the cosine is a purely imaginary root whose sign a signed zero picks
     in the reference's chain of operations."""
@@ -88,6 +96,6 @@ def test_lossless_total_reflection_is_handed_back(monkeypatch):
     w = np.array([1.0, 1e6])
     monkeypatch.setattr(chemicals, "nk_table", lambda f: (w, np.full(2, 1.2), np.zeros(2)))
     cos = np.array([0.4, 0.7])  # sin 0.917 and 0.714 against 1.2 / 1.5 = 0.8
-    _, _, ok64, _ = multilayer_column(LayerSequence([Layer(SI, thickness=3.0)]), Layer(OX),
-                                      np.full(2, 60.0), cos, 1.5, False)
+    _, _, ok64, _ = multilayer_column(_period(2, Layer(SI, thickness=3.0), Layer(MO, thickness=2.0)), Layer(OX),
+                                      np.full(2, 60.0), cos, 1.5, False, general)
     assert ok64.tolist() == [False, True]
