@@ -5,10 +5,15 @@
 // A launch holds as many blocks as the device keeps resident.  Each block
 // takes work tiles (block * rays_per_thread rays of one instance) from a
 // global counter until the queue is empty, so instances with 1k rays and
-// instances with 64k rays load-balance.  Per tile, the block stages that
-// instance's records into LDS (only when the instance changes), traces its
-// rays and reduces per-path statistics of the final positions with wave
-// shuffles and one LDS pass: one float64 atomic per statistic per tile.
+// instances with 64k rays load-balance.  Per tile, the block traces the
+// instance's rays -- the records read through the constant address space at
+// a uniform index, scalar loads as in the single-system kernels -- and
+// reduces per-path statistics of the final positions with wave shuffles and
+// one LDS pass: one float64 atomic per statistic per tile.  (Records staged
+// in LDS came back in vector registers, and with them every index and branch
+// condition they hold: the coatings' records then cost chains of vector
+// loads.  Tolerance batch of 256 spectrographs, float32: 1468 us staged,
+// 1111 us.)
 #pragma once
 
 #include "optk_internal.h"
@@ -43,48 +48,48 @@ __device__ __forceinline__ void block_accumulate(double acc[6], double *stats,
   __syncthreads();
 }
 
-// Tracer: stage(instance) copies that instance's records into LDS (all
-// threads), trace(i, path, x, y, intensity, unvignetted) traces ray i.
+// Tracer: select(instance) points it at that instance's records; trace(i, path0, path1, emit) traces ray i along paths path0 ..
+// path1 - 1 and calls emit(path, x, y, intensity, unvignetted) for each.
+// Two paths at a time share the part of the trace before the orders split.
 template <class Tracer>
 __device__ __forceinline__ void batch_loop(const BatchArgs &A, Tracer &tr) {
   __shared__ int s_tile;
   __shared__ double s_red[OPTK_BATCH_MAX_WAVES][6];
-  int current = -1;
   const int tid = threadIdx.x;
   const int block = blockDim.x;
   for (;;) {
     if (tid == 0) s_tile = atomicAdd(A.counter, 1);
     __syncthreads();
-    const int64_t t = s_tile;
+    const int64_t t = __builtin_amdgcn_readfirstlane(s_tile);
     if (t >= A.num_tiles) break;  // uniform: every thread read the same s_tile
     const BatchTile tile = A.tiles[t];
-    if (tile.instance != current) {
-      tr.stage(tile.instance);
-      __syncthreads();
-      current = tile.instance;
-    }
-    for (int path = 0; path < tr.num_paths(); ++path) {
-      double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    tr.select(__builtin_amdgcn_readfirstlane(tile.instance));
+    const int paths = tr.num_paths();
+    for (int path0 = 0; path0 < paths; path0 += 2) {
+      const int path1 = path0 + 2 < paths ? path0 + 2 : paths;
+      double acc[2][6] = {{0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}};
       for (int j = 0; j < A.rays_per_thread; ++j) {
         const int local = tid + j * block;
         if (local < tile.count) {
-          double x, y, inten;
-          bool unv;
-          tr.trace(tile.start + local, path, x, y, inten, unv);
-          if (unv) {
-            acc[0] += 1.0;
-            acc[1] += inten;
-            acc[2] += x;
-            acc[3] += y;
-            acc[4] += x * x;
-            acc[5] += y * y;
-          }
+          tr.trace(tile.start + local, path0, path1,
+                   [&](int path, double x, double y, double inten, bool unv) {
+                     // a ray that does not count adds zeros (its values may
+                     // be infinite: a select, not a product)
+                     const double v[6] = {unv ? 1.0 : 0.0, unv ? inten : 0.0, unv ? x : 0.0,
+                                          unv ? y : 0.0,   unv ? x * x : 0.0, unv ? y * y : 0.0};
+#pragma unroll
+                     for (int k = 0; k < 6; ++k) {
+                       acc[0][k] += path == path0 ? v[k] : 0.0;
+                       acc[1][k] += path == path0 ? 0.0 : v[k];
+                     }
+                   });
         }
       }
-      block_accumulate(acc, A.stats + ((int64_t)tile.instance * A.num_paths + path) * OPTK_BATCH_STATS,
-                       s_red);
+      double *stats = A.stats + ((int64_t)tile.instance * A.num_paths + path0) * OPTK_BATCH_STATS;
+      block_accumulate(acc[0], stats, s_red);
+      if (path1 - path0 > 1) block_accumulate(acc[1], stats + OPTK_BATCH_STATS, s_red);
     }
-    // every thread is past its reads of s_tile and of the staged records
+    // every thread is past its read of s_tile
     __syncthreads();
   }
 }

@@ -224,8 +224,8 @@ int call_signature(const optk_batch *b, int32_t flags) {
 int resident_blocks(const optk_batch *b, int32_t precision, int block, int32_t flags) {
   const int sig = call_signature(b, flags);
   if (precision == OPTK_F64)
-    return batch_occupancy_f64(b->features, sig, block, batch_lds_f64(b->num_surfaces));
-  return batch_occupancy_f32(b->features, sig, block, batch_lds_f32(b->num_surfaces));
+    return batch_occupancy_f64(b->features, sig, block);
+  return batch_occupancy_f32(b->features, sig, block);
 }
 
 // zero the statistics and the queue head, run the persistent kernel, reduce

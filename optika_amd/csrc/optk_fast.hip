@@ -179,24 +179,23 @@ template <int IO> __device__ __forceinline__ void store_ray32(const FRaysOut &o,
   store_ray<IO>(o, (int64_t)j, r);
 }
 
-size_t fast_staged_bytes(int num_surfaces) {
-  return sizeof(FastSpec) + (sizeof(FastSurface) + sizeof(optk_surface)) * (size_t)num_surfaces;
-}
-
 // occupancy targets (waves per SIMD): the geometric kernel at 6 (80 VGPRs;
 // measured faster than 5 or 8 on the Newtonian workload), the rulings /
 // toroid kernel at 4, the multilayer kernels at 2 (VALU-bound, register-heavy)
 template <int F> struct FastWaves {
   static constexpr int value = F == 0 ? 6 : ((F & FEAT_MULTILAYER) ? 2 : 4);
 };
-// the specialised kernels: 3 waves for the multilayer layouts (168 VGPRs;
-// spectrograph, 8.4M rays: 2.29 ms, at 2 waves 2.52 ms)
+// the specialised kernels: 4 waves for the multilayer layouts (128 VGPRs;
+// spectrograph, 8.4M rays: 1.29 ms, at 3 waves 1.33 ms)
 template <int F> struct FastSpecWaves {
-  static constexpr int value = F == 0 ? 6 : ((F & FEAT_MULTILAYER) ? 3 : 4);
+  static constexpr int value = F == 0 ? 6 : 4;
 };
 // the batched kernels keep 4 / 2 (at 6 the geometric one spills)
 template <int F> struct BatchWaves {
   static constexpr int value = (F & FEAT_MULTILAYER) ? 2 : 4;
+};
+template <int F> struct BatchSpecWaves {
+  static constexpr int value = 3;
 };
 
 // The system's records are read through the constant address space: every
@@ -233,22 +232,33 @@ __device__ __forceinline__ FRay fast_start(const FastArgs &A, const In &in, bool
   return r;
 }
 
-// surfaces k0 .. of path `path`
-template <int F, bool ACCUM>
-__device__ __forceinline__ void fast_path(ConstFastSurface *c_fast, ConstSurface *c_surf, const FastView &v, int k0,
-                                          int num_surfaces, int path, int num_paths, int64_t n, int64_t i,
-                                          const FRaysOut &accum, FRay &r) {
-  for (int k = k0; k < num_surfaces; ++k) {
+// a path whose multilayers are left to the float64 routine (FRay::rare),
+// from its input (kernels with the arguments (FastArgs, In, FRaysOut))
+template <int F, bool ACCUM, int IO, typename In>
+OPTK_RARE_PATH void fast_rare_path(const void *args, int64_t i, int path) {
+  const char *base = uniform_address(args);
+  const FastArgs &A = kernel_arg<FastArgs>(base, 0);
+  const In &in = kernel_arg<In>(base, sizeof(FastArgs));
+  ConstFastSpec *c_spec = (ConstFastSpec *)A.spec;
+  ConstFastSurface *c_fast = (ConstFastSurface *)A.fast;
+  ConstSurface *c_surf = (ConstSurface *)A.surfaces;
+  const FastView v = {A.surfaces, A.fast, A.sv, A.tables32};
+  const bool skip = A.entry == 1 && !ACCUM && c_spec->skip_first != 0;
+  const int k0 = skip ? 1 : 0;
+  FRay r = fast_start<IO>(A, in, skip, i);
+  for (int k = k0; k < A.num_surfaces; ++k) {
     const FastSurface &fk = *(const FastSurface *)&c_fast[k];
-    const optk_surface &sk = *(const optk_surface *)&c_surf[k];
     if (k > k0) fast_xf(fk.hop, r);
-    fast_propagate<F>(fk, sk, v, path, r);
+    fast_propagate<F | FEAT_REFERENCE>(fk, *(const optk_surface *)&c_surf[k], v, path, r);
     if (ACCUM) {
       FRay g = r;
       fast_xf(fk.to_global, g);
-      store_f(accum, ((int64_t)k * num_paths + path) * n + i, g);
+      store_f(kernel_arg<FRaysOut>(base, sizeof(FastArgs) + sizeof(In)),
+              ((int64_t)k * A.num_paths + path) * A.n + i, g);
     }
   }
+  fast_xf(*(const optk_affine *)&c_spec->last[A.apply_post], r);
+  store_ray<IO>(A.out, (int64_t)path * A.n + i, r);
 }
 
 template <int F, bool ACCUM, int IO, typename In>
@@ -263,6 +273,7 @@ __device__ __forceinline__ void fast_body(const FastArgs &A, const In &in, const
   v.tables32 = A.tables32;
   const int num_paths = (F & FEAT_RULINGS) ? A.num_paths : 1;
   const int num_surfaces = A.num_surfaces;
+  const int split = num_paths > 1 ? first_split((const optk_surface *)c_surf, num_surfaces) : num_surfaces;
   const int64_t n = A.n;
   // grid entry without per-surface accumulation: a pass-through surface 0
   // is elided (FastSpec::skip_first)
@@ -272,14 +283,33 @@ __device__ __forceinline__ void fast_body(const FastArgs &A, const In &in, const
   // it in scalar registers (blockDim.x would be a per-lane load)
   const int64_t stride = (int64_t)gridDim.x * TRACE_BLOCK;
   for (int64_t i = (int64_t)blockIdx.x * TRACE_BLOCK + threadIdx.x; i < n; i += stride) {
-    const FRay r0 = fast_start<IO>(A, in, skip, i);
+    FRay r = fast_start<IO>(A, in, skip, i), at_split;
+    FastHit hit_split = {};
     for (int path = 0; path < num_paths; ++path) {
-      FRay r = r0;
-      fast_path<F | FEAT_DEFER, ACCUM>(c_fast, c_surf, v, k0, num_surfaces, path, num_paths, n, i, accum, r);
+      if (path > 0) r = at_split;
+      for (int k = path > 0 ? split : k0; k < num_surfaces; ++k) {
+        const FastSurface &fk = *(const FastSurface *)&c_fast[k];
+        const optk_surface &sk = *(const optk_surface *)&c_surf[k];
+        FastHit hit = hit_split;
+        if (path == 0 || k != split) {
+          if (k > k0) fast_xf(fk.hop, r);
+          hit = fast_arrive<F>(fk, r);
+        }
+        if (k == split && path == 0) {
+          at_split = r;
+          hit_split = hit;
+        }
+        fast_leave<F | FEAT_DEFER>(fk, sk, v, path, hit, r);
+        if (ACCUM) {
+          FRay g = r;
+          fast_xf(fk.to_global, g);
+          for (int q = path; q < (k < split ? num_paths : path + 1); ++q)
+            store_f(accum, ((int64_t)k * num_paths + q) * n + i, g);
+        }
+      }
       if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
-        // the whole path again, so that nothing is kept live for it above
-        r = fast_start<IO>(A, in, skip, i);
-        fast_path<F | FEAT_REFERENCE, ACCUM>(c_fast, c_surf, v, k0, num_surfaces, path, num_paths, n, i, accum, r);
+        fast_rare_path<F, ACCUM, IO, In>(kernel_args(), i, path);
+        continue;
       }
       const optk_affine &last = *(const optk_affine *)&c_spec->last[A.apply_post];
       fast_xf(last, r);
@@ -328,18 +358,34 @@ FastArgs make_args(const optk_system *sys, const FRaysOut &out, int64_t n, int32
 // ray per thread, the surfaces unrolled in order with their kinds fixed at
 // compile time; the arithmetic is that of fast_body.
 template <int F, uint32_t K>
-__device__ __forceinline__ void fast_spec_step(int k, int k0, ConstFastSurface *c_fast,
-                                               ConstSurface *c_surf, const FastView &v, int path,
-                                               FRay &r) {
+__device__ __forceinline__ void fast_spec_step(int k, int k0, const FastSurface &fk, const optk_surface &sk,
+                                               const FastView &v, int path, FRay &r) {
   if (k < k0) return;
-  const FastSurface &fk = *(const FastSurface *)&c_fast[k];
-  const optk_surface &sk = *(const optk_surface *)&c_surf[k];
   if (k > k0) fast_xf(fk.hop, r);
   fast_propagate<F, K>(fk, sk, v, path, r);
 }
 
-template <typename In, int F, int IO, uint32_t... K>
-__device__ __forceinline__ void fast_spec_body(const FastArgs &A, const In &in) {
+// surface I up to the split (before it whole, the split surface up to its
+// intercept), and from the split on (split > k0: an elided surface 0 has no
+// rulings)
+template <int F, uint32_t K, int I, int SPLIT>
+__device__ __forceinline__ void fast_spec_before(int k0, const FastSurface &fk, const optk_surface &sk,
+                                                 const FastView &v, FastHit &hit, FRay &r) {
+  if (I < SPLIT) fast_spec_step<F, K>(I, k0, fk, sk, v, 0, r);
+  if (I == SPLIT) {
+    if (I > k0) fast_xf(fk.hop, r);
+    hit = fast_arrive<F, K>(fk, r);
+  }
+}
+template <int F, uint32_t K, int I, int SPLIT>
+__device__ __forceinline__ void fast_spec_after(int k0, const FastSurface &fk, const optk_surface &sk,
+                                                const FastView &v, int path, const FastHit &hit, FRay &r) {
+  if (I == SPLIT) fast_leave<F, K>(fk, sk, v, path, hit, r);
+  if (I > SPLIT) fast_spec_step<F, K>(I, k0, fk, sk, v, path, r);
+}
+
+template <typename In, int F, int IO, uint32_t... K, int... I>
+__device__ __forceinline__ void fast_spec_body(const FastArgs &A, const In &in, std::integer_sequence<int, I...>) {
   // the host launches these kernels with n * paths < 2^29: indices and
   // every element offset fit 32 bits
   const uint32_t i32 = blockIdx.x * (uint32_t)TRACE_BLOCK + threadIdx.x, n32 = (uint32_t)A.n;
@@ -355,18 +401,20 @@ __device__ __forceinline__ void fast_spec_body(const FastArgs &A, const In &in) 
   const int num_paths = (F & FEAT_RULINGS) ? A.num_paths : 1;
   const bool skip = A.entry == 1 && c_spec->skip_first != 0;
   const int k0 = skip ? 1 : 0;
+  constexpr int FAST = F | FEAT_DEFER | FEAT_BILAYER;
+  constexpr int SPLIT = (F & FEAT_RULINGS) ? first_ruled<K...>() : (int)sizeof...(K);
   FRay r0 = load_ray32<IO>(in, i32);
+  FastHit hit = {};
   fast_first_hop(A, skip, r0);
+  (fast_spec_before<FAST, K, I, SPLIT>(k0, *(const FastSurface *)&c_fast[I], *(const optk_surface *)&c_surf[I], v,
+                                       hit, r0), ...);
   for (int path = 0; path < num_paths; ++path) {
     FRay r = r0;
-    int k = 0;
-    (fast_spec_step<F | FEAT_DEFER | FEAT_BILAYER, K>(k++, k0, c_fast, c_surf, v, path, r), ...);
+    (fast_spec_after<FAST, K, I, SPLIT>(k0, *(const FastSurface *)&c_fast[I], *(const optk_surface *)&c_surf[I], v,
+                                        path, hit, r), ...);
     if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
-      // the whole path again, so that nothing is kept live for it above
-      r = load_ray32<IO>(in, i32);
-      fast_first_hop(A, skip, r);
-      k = 0;
-      (fast_spec_step<F | FEAT_REFERENCE | FEAT_BILAYER, K>(k++, k0, c_fast, c_surf, v, path, r), ...);
+      fast_rare_path<F | FEAT_BILAYER, false, IO, In>(kernel_args(), i32, path);
+      continue;
     }
     const optk_affine &last = *(const optk_affine *)&c_spec->last[A.apply_post];
     fast_xf(last, r);
@@ -377,13 +425,13 @@ __device__ __forceinline__ void fast_spec_body(const FastArgs &A, const In &in) 
 template <int F, int IO, uint32_t... K>
 __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(FastSpecWaves<F>::value)))
 void trace_grid_f32_spec(const FastArgs A, const FGridIn g) {
-  fast_spec_body<FGridIn, F, IO, K...>(A, g);
+  fast_spec_body<FGridIn, F, IO, K...>(A, g, std::make_integer_sequence<int, sizeof...(K)>());
 }
 
 template <int F, int IO, uint32_t... K>
 __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(FastSpecWaves<F>::value)))
 void trace_rays_f32_spec(const FastArgs A, const FRaysIn in) {
-  fast_spec_body<FRaysIn, F, IO, K...>(A, in);
+  fast_spec_body<FRaysIn, F, IO, K...>(A, in, std::make_integer_sequence<int, sizeof...(K)>());
 }
 
 typedef void (*SpecGrid32)(FastArgs, FGridIn);
@@ -441,132 +489,169 @@ int32_t launch(const KernelSet<In> &ks, bool special, const optk_system *sys, co
 
 // batched persistent trace, float32 form ------------------------------------
 
+// a batched path whose multilayers are left to the float64 routine: the
+// final ray, written out and returned (kernels with the arguments
+// (BatchArgs, FGridIn, FRaysOut))
+struct FastBatchEnd {
+  float x, y, intensity;
+  bool unvignetted;
+};
+template <int F> OPTK_RARE_PATH FastBatchEnd fast_rare_batch_path(const void *args, int instance, int64_t i, int path);
+
 template <int F> struct Tracer32 {
   const BatchArgs &A;
   const FGridIn &in;
   const FRaysOut &out;
-  FastSpec *s_spec;
-  FastSurface *s_fast;
-  optk_surface *s_surf;
+  const FastSpec *spec = nullptr;  // of the current instance, constant address space
+  const FastSurface *fast = nullptr;
+  const optk_surface *surf = nullptr;
+  int instance = 0;
+
+  __device__ Tracer32(const BatchArgs &a, const FGridIn &g, const FRaysOut &o) : A(a), in(g), out(o) {}
 
   __device__ int num_paths() const { return (F & FEAT_RULINGS) ? A.num_paths : 1; }
 
-  __device__ __forceinline__ void stage(int instance) {
-    stage_words(s_spec, A.fast_specs + instance, sizeof(FastSpec));
-    stage_words(s_fast, A.fast + (int64_t)instance * A.num_surfaces,
-                sizeof(FastSurface) * (size_t)A.num_surfaces);
-    stage_words(s_surf, A.surfaces + (int64_t)instance * A.num_surfaces,
-                sizeof(optk_surface) * (size_t)A.num_surfaces);
+  __device__ __forceinline__ void select(int k) {
+    instance = k;
+    const int64_t first_surface = (int64_t)instance * A.num_surfaces;
+    spec = (const FastSpec *)((ConstFastSpec *)A.fast_specs + instance);
+    fast = (const FastSurface *)((ConstFastSurface *)A.fast + first_surface);
+    surf = (const optk_surface *)((ConstSurface *)A.surfaces + first_surface);
   }
 
-  __device__ __forceinline__ FRay start(int64_t i) {
+  __device__ __forceinline__ FastView view() const {
+    FastView v;
+    v.surfaces = surf;
+    v.fast = fast;
+    v.sv = A.sv;
+    v.tables32 = A.tables32;
+    return v;
+  }
+
+  // a pass-through surface 0 is elided as in the grid kernels
+  __device__ __forceinline__ int first() const { return spec->skip_first != 0 ? 1 : 0; }
+
+  __device__ __forceinline__ FRay start(int64_t i) const {
     FRay r = load_fray(in, i);
-    if (s_spec->skip_first != 0) {
+    if (spec->skip_first != 0) {
       const bool parallel = r.dz == 0.0;
-      fast_xf(s_spec->first_skip, r);
+      fast_xf(spec->first_skip, r);
       if (parallel) {
         r.px = r.py = r.pz = NAN;
         r.intensity = NAN;
       }
     } else {
-      fast_xf(s_spec->first_hop[1], r);
+      fast_xf(spec->first_hop[1], r);
     }
     return r;
   }
 
-  // the whole path with the float64 multilayer (FRay::rare)
-  __device__ __forceinline__ void reference(const FastView &v, int64_t i, int path, FRay &r) {
-    const int k0 = s_spec->skip_first != 0 ? 1 : 0;
-    r = start(i);
-    for (int k = k0; k < A.num_surfaces; ++k) {
-      if (k > k0) fast_xf(s_fast[k].hop, r);
-      fast_propagate<F | FEAT_REFERENCE>(s_fast[k], s_surf[k], v, path, r);
-    }
+  // a path by the float64 routine: fast_rare_batch_path
+  template <int G, typename Emit> __device__ __forceinline__ void rare(int64_t i, int path, Emit emit) const {
+    const FastBatchEnd e = fast_rare_batch_path<G>(kernel_args(), instance, i, path);
+    emit(path, (double)e.x, (double)e.y, (double)e.intensity, e.unvignetted);
   }
 
-  __device__ __forceinline__ void trace(int64_t i, int path, double &x, double &y, double &inten,
-                                        bool &unv) {
-    FastView v;
-    v.surfaces = s_surf;
-    v.fast = s_fast;
-    v.sv = A.sv;
-    v.tables32 = A.tables32;
-    // a pass-through surface 0 is elided as in the grid kernels
-    const int k0 = s_spec->skip_first != 0 ? 1 : 0;
-    FRay r = start(i);
-    for (int k = k0; k < A.num_surfaces; ++k) {
-      if (k > k0) fast_xf(s_fast[k].hop, r);
-      fast_propagate<F | FEAT_DEFER>(s_fast[k], s_surf[k], v, path, r);
-    }
-    if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) reference(v, i, path, r);
-    const optk_affine &last = s_spec->last[A.apply_post];
-    fast_xf(last, r);
+  template <typename Emit>
+  __device__ __forceinline__ void finish(int64_t i, int path, FRay &r, Emit emit) const {
+    fast_xf(spec->last[A.apply_post], r);
     store_f(out, (int64_t)path * A.n + i, r);
     // statistics of the float32 result, as a caller reading the outputs sees it
-    x = (double)(float)r.px;
-    y = (double)(float)r.py;
-    inten = r.intensity;
-    unv = r.unvignetted;
+    emit(path, (double)(float)r.px, (double)(float)r.py, (double)r.intensity, r.unvignetted);
+  }
+
+  template <typename Emit>
+  __device__ __forceinline__ void trace(int64_t i, int path0, int path1, Emit emit) {
+    const FastView v = view();
+    const int k0 = first();
+    const int split = num_paths() > 1 ? first_split(surf, A.num_surfaces) : A.num_surfaces;
+    FRay r = start(i), at_split;
+    FastHit hit_split = {};
+    for (int path = path0; path < path1; ++path) {
+      if (path > path0) r = at_split;
+      for (int k = path > path0 ? split : k0; k < A.num_surfaces; ++k) {
+        FastHit hit = hit_split;
+        if (path == path0 || k != split) {
+          if (k > k0) fast_xf(fast[k].hop, r);
+          hit = fast_arrive<F>(fast[k], r);
+        }
+        if (k == split && path == path0) {
+          at_split = r;
+          hit_split = hit;
+        }
+        fast_leave<F | FEAT_DEFER>(fast[k], surf[k], v, path, hit, r);
+      }
+      if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
+        this->template rare<F>(i, path, emit);
+        continue;
+      }
+      finish(i, path, r, emit);
+    }
   }
 };
 
 // the same with the instances' surface kinds fixed at compile time (every
 // instance of a batch matching one signature), the surfaces unrolled
-template <int F, uint32_t K>
-__device__ __forceinline__ void batch_fast_step(int k, int k0, const FastSurface *s_fast,
-                                                const optk_surface *s_surf, const FastView &v, int path,
-                                                FRay &r) {
-  if (k < k0) return;
-  if (k > k0) fast_xf(s_fast[k].hop, r);
-  fast_propagate<F, K>(s_fast[k], s_surf[k], v, path, r);
-}
-
 template <int F, uint32_t... K> struct Tracer32Spec : Tracer32<F> {
-  __device__ __forceinline__ void trace(int64_t i, int path, double &x, double &y, double &inten,
-                                        bool &unv) {
-    FastView v;
-    v.surfaces = this->s_surf;
-    v.fast = this->s_fast;
-    v.sv = this->A.sv;
-    v.tables32 = this->A.tables32;
-    const int k0 = this->s_spec->skip_first != 0 ? 1 : 0;
-    FRay r = this->start(i);
-    int k = 0;
-    (batch_fast_step<F | FEAT_DEFER | FEAT_BILAYER, K>(k++, k0, this->s_fast, this->s_surf, v, path, r), ...);
-    if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
-      r = this->start(i);
-      k = 0;
-      (batch_fast_step<F | FEAT_REFERENCE | FEAT_BILAYER, K>(k++, k0, this->s_fast, this->s_surf, v, path, r), ...);
+  using Tracer32<F>::Tracer32;
+
+  template <typename Emit>
+  __device__ __forceinline__ void trace(int64_t i, int path0, int path1, Emit emit) {
+    trace_each(i, path0, path1, emit, std::make_integer_sequence<int, sizeof...(K)>());
+  }
+
+  template <typename Emit, int... I>
+  __device__ __forceinline__ void trace_each(int64_t i, int path0, int path1, Emit emit,
+                                             std::integer_sequence<int, I...>) {
+    constexpr int FAST = F | FEAT_DEFER | FEAT_BILAYER;
+    constexpr int SPLIT = (F & FEAT_RULINGS) ? first_ruled<K...>() : (int)sizeof...(K);
+    const FastView v = this->view();
+    const int k0 = this->first();
+    FRay r0 = this->start(i);
+    FastHit hit = {};
+    (fast_spec_before<FAST, K, I, SPLIT>(k0, this->fast[I], this->surf[I], v, hit, r0), ...);
+    for (int path = path0; path < path1; ++path) {
+      FRay r = r0;
+      (fast_spec_after<FAST, K, I, SPLIT>(k0, this->fast[I], this->surf[I], v, path, hit, r), ...);
+      if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
+        this->template rare<F | FEAT_BILAYER>(i, path, emit);
+        continue;
+      }
+      this->finish(i, path, r, emit);
     }
-    const optk_affine &last = this->s_spec->last[this->A.apply_post];
-    fast_xf(last, r);
-    store_f(this->out, (int64_t)path * this->A.n + i, r);
-    x = (double)(float)r.px;
-    y = (double)(float)r.py;
-    inten = r.intensity;
-    unv = r.unvignetted;
   }
 };
+
+template <int F> OPTK_RARE_PATH FastBatchEnd fast_rare_batch_path(const void *args, int instance, int64_t i, int path) {
+  const char *base = uniform_address(args);
+  Tracer32<F> tr(kernel_arg<BatchArgs>(base, 0), kernel_arg<FGridIn>(base, sizeof(BatchArgs)),
+                 kernel_arg<FRaysOut>(base, sizeof(BatchArgs) + sizeof(FGridIn)));
+  tr.select(__builtin_amdgcn_readfirstlane(instance));
+  const FastView v = tr.view();
+  const int k0 = tr.first();
+  FRay r = tr.start(i);
+  for (int k = k0; k < tr.A.num_surfaces; ++k) {
+    if (k > k0) fast_xf(tr.fast[k].hop, r);
+    fast_propagate<F | FEAT_REFERENCE>(tr.fast[k], tr.surf[k], v, path, r);
+  }
+  FastBatchEnd end;
+  tr.finish(i, path, r, [&](int, double x, double y, double inten, bool unv) {
+    end = {(float)x, (float)y, (float)inten, unv};
+  });
+  return end;
+}
 
 template <int F>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(BatchWaves<F>::value)))
 void batch_grid_f32(const BatchArgs A, const FGridIn in, const FRaysOut out) {
-  extern __shared__ double staged[];
-  FastSpec *spec = reinterpret_cast<FastSpec *>(staged);
-  FastSurface *fast = reinterpret_cast<FastSurface *>(spec + 1);
-  optk_surface *surf = reinterpret_cast<optk_surface *>(fast + A.num_surfaces);
-  Tracer32<F> tr{A, in, out, spec, fast, surf};
+  Tracer32<F> tr(A, in, out);
   batch_loop(A, tr);
 }
 
 template <int F, uint32_t... K>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(FastSpecWaves<F>::value)))
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(BatchSpecWaves<F>::value)))
 void batch_grid_f32_spec(const BatchArgs A, const FGridIn in, const FRaysOut out) {
-  extern __shared__ double staged[];
-  FastSpec *spec = reinterpret_cast<FastSpec *>(staged);
-  FastSurface *fast = reinterpret_cast<FastSurface *>(spec + 1);
-  optk_surface *surf = reinterpret_cast<optk_surface *>(fast + A.num_surfaces);
-  Tracer32Spec<F, K...> tr{{A, in, out, spec, fast, surf}};
+  Tracer32Spec<F, K...> tr(A, in, out);
   batch_loop(A, tr);
 }
 
@@ -615,28 +700,18 @@ int32_t fast_trace_grid(const optk_system *sys, const FGridIn &in, const FRaysOu
                          stream);
 }
 
-size_t batch_lds_f32(int num_surfaces) { return fast_staged_bytes(num_surfaces); }
-
-int batch_occupancy_f32(int features, int signature, int block, size_t lds) {
+int batch_occupancy_f32(int features, int signature, int block) {
   int nb = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_kernel_f32(features, signature), block,
-                                                   lds) != hipSuccess)
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_kernel_f32(features, signature), block, 0) !=
+      hipSuccess)
     return 0;
   return nb;
 }
 
 hipError_t batch_launch_f32(int features, int signature, int blocks, int block, const BatchArgs &A,
                             const FGridIn &in, const FRaysOut &out, hipStream_t stream) {
-  size_t lds = fast_staged_bytes(A.num_surfaces);
-  if (signature >= 0 && signature < NUM_SIGNATURES && BATCH_SPEC32[signature])
-    hipLaunchKernelGGL(BATCH_SPEC32[signature], dim3(blocks), dim3(block), lds, stream, A, in, out);
-  else if (features == 0)
-    hipLaunchKernelGGL(batch_grid_f32<0>, dim3(blocks), dim3(block), lds, stream, A, in, out);
-  else if (features == (FEAT_TOROID | FEAT_RULINGS))
-    hipLaunchKernelGGL(batch_grid_f32<FEAT_TOROID | FEAT_RULINGS>, dim3(blocks), dim3(block), lds,
-                       stream, A, in, out);
-  else
-    hipLaunchKernelGGL(batch_grid_f32<FEAT_ALL>, dim3(blocks), dim3(block), lds, stream, A, in, out);
+  typedef void (*Kernel)(BatchArgs, FGridIn, FRaysOut);
+  hipLaunchKernelGGL((Kernel)batch_kernel_f32(features, signature), dim3(blocks), dim3(block), 0, stream, A, in, out);
   return hipGetLastError();
 }
 

@@ -153,16 +153,44 @@ struct BatchArgs {
   int64_t n;                       // rays in the batch (output stride per path)
 };
 
-size_t batch_lds_f64(int num_surfaces);
-size_t batch_lds_f32(int num_surfaces);
 // resident blocks per CU of the kernel covering `features` (0 on error);
 // signature >= 0: the instances' common surface-kind signature
 // (optk_signatures.h), whose specialised kernel runs where one exists
-int batch_occupancy_f64(int features, int signature, int block, size_t lds);
-int batch_occupancy_f32(int features, int signature, int block, size_t lds);
+int batch_occupancy_f64(int features, int signature, int block);
+int batch_occupancy_f32(int features, int signature, int block);
 hipError_t batch_launch_f64(int features, int signature, int blocks, int block, const BatchArgs &A,
                             const GridIn &in, const RaysOut &out, hipStream_t stream);
 hipError_t batch_launch_f32(int features, int signature, int blocks, int block, const BatchArgs &A,
                             const FGridIn &in, const FRaysOut &out, hipStream_t stream);
+
+#if defined(__HIPCC__)
+// The rare paths of the trace kernels (rays whose multilayers are evaluated
+// by the reference's operations) are out-of-line functions: inlined, their
+// registers crowded every ray's -- the float32 spectrograph kernel's main
+// path had 870 register-lane spills and up to 280 scratch accesses with them
+// and has 70 and none without (8.4M rays: 1.63 to 1.87 ms, by the
+// allocator's mood, against 1.33 ms at 3 waves).  They read the kernel's arguments
+// through the kernarg segment's address, which the kernel passes on (passed
+// by reference, the arguments would be copied to scratch at its start), made
+// uniform again so that the records stay scalar loads.
+__device__ __forceinline__ const char *uniform_address(const void *p) {
+  const uint64_t v = (uint64_t)p;
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+  return (const char *)(((uint64_t)hi << 32) | lo);
+}
+
+// the argument of type T at byte `offset` of the kernarg segment
+template <typename T> __device__ __forceinline__ const T &kernel_arg(const char *args, size_t offset) {
+  static_assert(alignof(T) == 8 && sizeof(T) % 8 == 0, "kernel arguments are packed at 8 bytes");
+  typedef __attribute__((address_space(4))) const T ConstT;
+  return *(const T *)(ConstT *)(args + offset);
+}
+
+__device__ __forceinline__ const void *kernel_args() {
+  return (const void *)__builtin_amdgcn_kernarg_segment_ptr();
+}
+#define OPTK_RARE_PATH __device__ __attribute__((noinline))
+#endif
 
 }  // namespace optk

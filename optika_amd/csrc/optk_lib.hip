@@ -281,6 +281,29 @@ template <int IO> __device__ __forceinline__ void store_io32(const RaysOut &o, u
 typedef __attribute__((address_space(4))) const TraceSpec ConstTraceSpec;
 typedef __attribute__((address_space(4))) const optk_surface ConstSurface;
 
+// a path whose multilayers are left to the reference's operations, from its
+// input (kernels with the arguments (TraceArgs, In, RaysOut))
+template <int F, bool ACCUM, int IO, typename In>
+OPTK_RARE_PATH void rare_path(const void *args, int64_t i, int path) {
+  const char *base = uniform_address(args);
+  const TraceArgs &A = kernel_arg<TraceArgs>(base, 0);
+  const In &in = kernel_arg<In>(base, sizeof(TraceArgs));
+  const TraceSpec &spec = *(const TraceSpec *)(ConstTraceSpec *)A.spec;
+  ConstSurface *c_surf = (ConstSurface *)A.surfaces;
+  SystemView sys = spec.sys;
+  sys.surfaces = A.surfaces;
+  Ray<double> r = load_io<IO>(in, i);
+  apply_pre(spec, r);
+  for (int k = 0; k < A.num_surfaces; ++k) {
+    propagate_surface<F | FEAT_REFERENCE>(*(const optk_surface *)&c_surf[k], sys, path, r);
+    if (ACCUM)
+      store(kernel_arg<RaysOut>(base, sizeof(TraceArgs) + sizeof(In)),
+            ((int64_t)k * sys.num_paths + path) * A.n + i, r);
+  }
+  if (A.apply_post) xf_inverse_ray(spec.post, r.px, r.py, r.pz, r.dx, r.dy, r.dz);
+  store_io<IO>(A.out, (int64_t)path * A.n + i, r);
+}
+
 template <int F, bool ACCUM, int IO, typename In>
 __device__ __forceinline__ void trace_body(const TraceArgs &A, const In &in, const RaysOut &accum) {
   ConstTraceSpec *c_spec = (ConstTraceSpec *)A.spec;
@@ -291,27 +314,33 @@ __device__ __forceinline__ void trace_body(const TraceArgs &A, const In &in, con
   // only rulings create diffraction-order paths: without them one path
   const int num_paths = (F & FEAT_RULINGS) ? sys.num_paths : 1;
   const int num_surfaces = A.num_surfaces;
+  const int split = num_paths > 1 ? first_split((const optk_surface *)c_surf, num_surfaces) : num_surfaces;
   const int64_t n = A.n;
   // the launch block is TRACE_BLOCK threads: a compile-time stride keeps
   // it in scalar registers (blockDim.x would be a per-lane load)
   const int64_t stride = (int64_t)gridDim.x * TRACE_BLOCK;
   for (int64_t i = (int64_t)blockIdx.x * TRACE_BLOCK + threadIdx.x; i < n; i += stride) {
-    Ray<double> r0 = load_io<IO>(in, i);
-    apply_pre(spec, r0);
+    Ray<double> r = load_io<IO>(in, i), at_split;
+    V3<double> normal_split = {0.0, 0.0, 0.0};
+    apply_pre(spec, r);
     for (int path = 0; path < num_paths; ++path) {
-      Ray<double> r = r0;
-      for (int k = 0; k < num_surfaces; ++k) {
-        propagate_surface<F | FEAT_DEFER>(*(const optk_surface *)&c_surf[k], sys, path, r);
-        if (ACCUM) store(accum, ((int64_t)k * num_paths + path) * n + i, r);
+      if (path > 0) r = at_split;
+      for (int k = path > 0 ? split : 0; k < num_surfaces; ++k) {
+        const optk_surface &sk = *(const optk_surface *)&c_surf[k];
+        V3<double> normal = normal_split;
+        if (path == 0 || k != split) normal = surface_arrive<F>(sk, r);
+        if (k == split && path == 0) {
+          at_split = r;
+          normal_split = normal;
+        }
+        surface_leave<F | FEAT_DEFER>(sk, sys, path, normal, r);
+        if (ACCUM)
+          for (int q = path; q < (k < split ? num_paths : path + 1); ++q)
+            store(accum, ((int64_t)k * num_paths + q) * n + i, r);
       }
       if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
-        // the whole path again, so that nothing is kept live for it above
-        r = load_io<IO>(in, i);
-        apply_pre(spec, r);
-        for (int k = 0; k < num_surfaces; ++k) {
-          propagate_surface<F | FEAT_REFERENCE>(*(const optk_surface *)&c_surf[k], sys, path, r);
-          if (ACCUM) store(accum, ((int64_t)k * num_paths + path) * n + i, r);
-        }
+        rare_path<F, ACCUM, IO, In>(kernel_args(), i, path);
+        continue;
       }
       if (A.apply_post) {
         xf_inverse_ray(spec.post, r.px, r.py, r.pz, r.dx, r.dy, r.dz);
@@ -347,14 +376,29 @@ static void launch_trace(void (*k0)(TraceArgs, In, RaysOut), void (*k3)(TraceArg
 }
 
 
+// surface I of a specialised kernel: up to the split (before it whole, the
+// split surface up to its intercept), and from the split on
+template <int F, uint32_t K, int I, int SPLIT>
+__device__ __forceinline__ void spec_before(const optk_surface &s, const SystemView &sys, V3<double> &normal,
+                                            Ray<double> &r) {
+  if (I < SPLIT) propagate_surface<F, K>(s, sys, 0, r);
+  if (I == SPLIT) normal = surface_arrive<F, K>(s, r);
+}
+template <int F, uint32_t K, int I, int SPLIT>
+__device__ __forceinline__ void spec_after(const optk_surface &s, const SystemView &sys, int path,
+                                           V3<double> normal, Ray<double> &r) {
+  if (I == SPLIT) surface_leave<F, K>(s, sys, path, normal, r);
+  if (I > SPLIT) propagate_surface<F, K>(s, sys, path, r);
+}
+
 // Kernels specialised on a system's surface kinds (optk_signatures.h): the
 // surfaces unrolled in order, each with its kinds fixed at compile time, one
 // ray per thread.  (A grid-stride loop would keep every surface's record
 // fields live in scalar registers across its iterations, more than the
 // scalar register file holds; the compiler then spills them into VGPR
 // lanes.)  The arithmetic is that of the generic kernels.
-template <typename In, int F, int IO, uint32_t... K>
-__device__ __forceinline__ void spec_body(const TraceArgs &A, const In &in) {
+template <typename In, int F, int IO, uint32_t... K, int... I>
+__device__ __forceinline__ void spec_body(const TraceArgs &A, const In &in, std::integer_sequence<int, I...>) {
   // the host launches these kernels with n * paths < 2^29: indices and
   // every element offset fit 32 bits
   const uint32_t i32 = blockIdx.x * (uint32_t)TRACE_BLOCK + threadIdx.x, n32 = (uint32_t)A.n;
@@ -365,18 +409,18 @@ __device__ __forceinline__ void spec_body(const TraceArgs &A, const In &in) {
   SystemView sys = spec.sys;
   sys.surfaces = A.surfaces;
   const int num_paths = (F & FEAT_RULINGS) ? sys.num_paths : 1;
+  constexpr int FAST = F | FEAT_DEFER | FEAT_BILAYER;
+  constexpr int SPLIT = (F & FEAT_RULINGS) ? first_ruled<K...>() : (int)sizeof...(K);
   Ray<double> r0 = load_io32<IO>(in, i32);
+  V3<double> normal = {0.0, 0.0, 0.0};
   apply_pre(spec, r0);
+  (spec_before<FAST, K, I, SPLIT>(*(const optk_surface *)&c_surf[I], sys, normal, r0), ...);
   for (int path = 0; path < num_paths; ++path) {
     Ray<double> r = r0;
-    int k = 0;
-    (propagate_surface<F | FEAT_DEFER | FEAT_BILAYER, K>(*(const optk_surface *)&c_surf[k++], sys, path, r), ...);
+    (spec_after<FAST, K, I, SPLIT>(*(const optk_surface *)&c_surf[I], sys, path, normal, r), ...);
     if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
-      // the whole path again, so that nothing is kept live for it above
-      r = load_io32<IO>(in, i32);
-      apply_pre(spec, r);
-      k = 0;
-      (propagate_surface<F | FEAT_REFERENCE | FEAT_BILAYER, K>(*(const optk_surface *)&c_surf[k++], sys, path, r), ...);
+      rare_path<F | FEAT_BILAYER, false, IO, In>(kernel_args(), i32, path);
+      continue;
     }
     if (A.apply_post) xf_inverse_ray(spec.post, r.px, r.py, r.pz, r.dx, r.dy, r.dz);
     store_io32<IO>(A.out, (uint32_t)path * n32 + i32, r);
@@ -386,13 +430,13 @@ __device__ __forceinline__ void spec_body(const TraceArgs &A, const In &in) {
 template <int F, int IO, uint32_t... K>
 __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(SpecWaves<F>::value)))
 void trace_grid_f64_spec(const TraceArgs A, const GridIn g) {
-  spec_body<GridIn, F, IO, K...>(A, g);
+  spec_body<GridIn, F, IO, K...>(A, g, std::make_integer_sequence<int, sizeof...(K)>());
 }
 
 template <int F, int IO, uint32_t... K>
 __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(SpecWaves<F>::value)))
 void trace_rays_f64_spec(const TraceArgs A, const RaysIn in) {
-  spec_body<RaysIn, F, IO, K...>(A, in);
+  spec_body<RaysIn, F, IO, K...>(A, in, std::make_integer_sequence<int, sizeof...(K)>());
 }
 
 // the specialised kernels by signature (the order of SIGNATURES): grid
@@ -574,41 +618,79 @@ __global__ __launch_bounds__(256) void expose_kernel(const optk_expose_args a, i
 
 // batched persistent trace, float64 form ------------------------------------
 
+// a batched path whose multilayers are left to the reference's operations:
+// the final ray, written out and returned (kernels with the arguments
+// (BatchArgs, GridIn, RaysOut))
+struct BatchEnd {
+  double x, y, intensity;
+  bool unvignetted;
+};
+template <int F> OPTK_RARE_PATH BatchEnd rare_batch_path(const void *args, int instance, int64_t i, int path);
+
 template <int F> struct Tracer64 {
   const BatchArgs &A;
   const GridIn &in;
   const RaysOut &out;
-  TraceSpec *s_spec;
-  optk_surface *s_surf;
+  const TraceSpec *spec = nullptr;  // of the current instance, constant address space
+  const optk_surface *surf = nullptr;
+  int instance = 0;
+
+  __device__ Tracer64(const BatchArgs &a, const GridIn &g, const RaysOut &o) : A(a), in(g), out(o) {}
 
   __device__ int num_paths() const { return (F & FEAT_RULINGS) ? A.num_paths : 1; }
 
-  __device__ __forceinline__ void stage(int instance) {
-    stage_words(s_spec, A.specs64 + instance, sizeof(TraceSpec));
-    stage_words(s_surf, A.surfaces + (int64_t)instance * A.num_surfaces,
-                sizeof(optk_surface) * (size_t)A.num_surfaces);
+  __device__ __forceinline__ void select(int k) {
+    instance = k;
+    spec = (const TraceSpec *)((ConstTraceSpec *)A.specs64 + instance);
+    surf = (const optk_surface *)((ConstSurface *)A.surfaces + (int64_t)instance * A.num_surfaces);
   }
 
-  __device__ __forceinline__ void trace(int64_t i, int path, double &x, double &y, double &inten,
-                                        bool &unv) {
+  __device__ __forceinline__ SystemView view() const {
+    return {surf, A.num_surfaces, A.num_paths, A.sv};
+  }
+
+  __device__ __forceinline__ Ray<double> start(int64_t i) const {
     Ray<double> r = load_ray(in, i);
-    apply_pre(*s_spec, r);
-    SystemView sys = s_spec->sys;
-    sys.surfaces = s_surf;
-    for (int k = 0; k < A.num_surfaces; ++k) propagate_surface<F | FEAT_DEFER>(s_surf[k], sys, path, r);
-    if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
-      r = load_ray(in, i);
-      apply_pre(*s_spec, r);
-      for (int k = 0; k < A.num_surfaces; ++k) propagate_surface<F | FEAT_REFERENCE>(s_surf[k], sys, path, r);
-    }
-    if (A.apply_post) {
-      xf_inverse_ray(s_spec->post, r.px, r.py, r.pz, r.dx, r.dy, r.dz);
-    }
+    apply_pre(*spec, r);
+    return r;
+  }
+
+  // a path by the reference's operations: rare_batch_path
+  template <int G, typename Emit> __device__ __forceinline__ void rare(int64_t i, int path, Emit emit) const {
+    const BatchEnd e = rare_batch_path<G>(kernel_args(), instance, i, path);
+    emit(path, e.x, e.y, e.intensity, e.unvignetted);
+  }
+
+  template <typename Emit>
+  __device__ __forceinline__ void finish(int64_t i, int path, Ray<double> &r, Emit emit) const {
+    if (A.apply_post) xf_inverse_ray(spec->post, r.px, r.py, r.pz, r.dx, r.dy, r.dz);
     store(out, (int64_t)path * A.n + i, r);
-    x = r.px;
-    y = r.py;
-    inten = r.intensity;
-    unv = r.unvignetted;
+    emit(path, r.px, r.py, r.intensity, r.unvignetted);
+  }
+
+  template <typename Emit>
+  __device__ __forceinline__ void trace(int64_t i, int path0, int path1, Emit emit) {
+    const SystemView sys = view();
+    const int split = num_paths() > 1 ? first_split(surf, A.num_surfaces) : A.num_surfaces;
+    Ray<double> r = start(i), at_split;
+    V3<double> normal_split = {0.0, 0.0, 0.0};
+    for (int path = path0; path < path1; ++path) {
+      if (path > path0) r = at_split;
+      for (int k = path > path0 ? split : 0; k < A.num_surfaces; ++k) {
+        V3<double> normal = normal_split;
+        if (path == path0 || k != split) normal = surface_arrive<F>(surf[k], r);
+        if (k == split && path == path0) {
+          at_split = r;
+          normal_split = normal;
+        }
+        surface_leave<F | FEAT_DEFER>(surf[k], sys, path, normal, r);
+      }
+      if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
+        this->template rare<F>(i, path, emit);
+        continue;
+      }
+      finish(i, path, r, emit);
+    }
   }
 };
 
@@ -616,51 +698,60 @@ template <int F> struct Tracer64 {
 // instance of a batch matching one signature): the surfaces unroll as in
 // the specialised single-system kernels, the records are read from LDS
 template <int F, uint32_t... K> struct Tracer64Spec : Tracer64<F> {
-  __device__ __forceinline__ void trace(int64_t i, int path, double &x, double &y, double &inten,
-                                        bool &unv) {
-    Ray<double> r = load_ray(this->in, i);
-    apply_pre(*this->s_spec, r);
-    SystemView sys = this->s_spec->sys;
-    sys.surfaces = this->s_surf;
-    int k = 0;
-    (propagate_surface<F | FEAT_DEFER | FEAT_BILAYER, K>(this->s_surf[k++], sys, path, r), ...);
-    if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
-      r = load_ray(this->in, i);
-      apply_pre(*this->s_spec, r);
-      k = 0;
-      (propagate_surface<F | FEAT_REFERENCE | FEAT_BILAYER, K>(this->s_surf[k++], sys, path, r), ...);
+  using Tracer64<F>::Tracer64;
+
+  template <typename Emit>
+  __device__ __forceinline__ void trace(int64_t i, int path0, int path1, Emit emit) {
+    trace_each(i, path0, path1, emit, std::make_integer_sequence<int, sizeof...(K)>());
+  }
+
+  template <typename Emit, int... I>
+  __device__ __forceinline__ void trace_each(int64_t i, int path0, int path1, Emit emit,
+                                             std::integer_sequence<int, I...>) {
+    constexpr int FAST = F | FEAT_DEFER | FEAT_BILAYER;
+    constexpr int SPLIT = (F & FEAT_RULINGS) ? first_ruled<K...>() : (int)sizeof...(K);
+    const SystemView sys = this->view();
+    Ray<double> r0 = this->start(i);
+    V3<double> normal = {0.0, 0.0, 0.0};
+    (spec_before<FAST, K, I, SPLIT>(this->surf[I], sys, normal, r0), ...);
+    for (int path = path0; path < path1; ++path) {
+      Ray<double> r = r0;
+      (spec_after<FAST, K, I, SPLIT>(this->surf[I], sys, path, normal, r), ...);
+      if ((F & FEAT_MULTILAYER) && __builtin_expect(r.rare, 0)) {
+        this->template rare<F | FEAT_BILAYER>(i, path, emit);
+        continue;
+      }
+      this->finish(i, path, r, emit);
     }
-    if (this->A.apply_post) {
-      xf_inverse_ray(this->s_spec->post, r.px, r.py, r.pz, r.dx, r.dy, r.dz);
-    }
-    store(this->out, (int64_t)path * this->A.n + i, r);
-    x = r.px;
-    y = r.py;
-    inten = r.intensity;
-    unv = r.unvignetted;
   }
 };
+
+template <int F> OPTK_RARE_PATH BatchEnd rare_batch_path(const void *args, int instance, int64_t i, int path) {
+  const char *base = uniform_address(args);
+  Tracer64<F> tr(kernel_arg<BatchArgs>(base, 0), kernel_arg<GridIn>(base, sizeof(BatchArgs)),
+                 kernel_arg<RaysOut>(base, sizeof(BatchArgs) + sizeof(GridIn)));
+  tr.select(__builtin_amdgcn_readfirstlane(instance));
+  const SystemView sys = tr.view();
+  Ray<double> r = tr.start(i);
+  for (int k = 0; k < tr.A.num_surfaces; ++k) propagate_surface<F | FEAT_REFERENCE>(tr.surf[k], sys, path, r);
+  BatchEnd end;
+  tr.finish(i, path, r, [&](int, double x, double y, double inten, bool unv) { end = {x, y, inten, unv}; });
+  return end;
+}
 
 template <int F>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(Waves<F>::value)))
 void batch_grid_f64(const BatchArgs A, const GridIn in, const RaysOut out) {
-  extern __shared__ double staged[];
-  Tracer64<F> tr{A, in, out, reinterpret_cast<TraceSpec *>(staged),
-                 reinterpret_cast<optk_surface *>(reinterpret_cast<TraceSpec *>(staged) + 1)};
+  Tracer64<F> tr(A, in, out);
   batch_loop(A, tr);
 }
 
 // 2 waves per SIMD (256 VGPRs) for the multilayer layouts, as the generic
-// batch kernel: built for 3 or 4 waves (168 / 128 VGPRs, about twice the
-// spill slots) this kernel returned every ray vignetted on the tolerance
-// batch, while the same source at 256 VGPRs, and with the trace left as a
-// call, matches the single-system traces; the narrower builds are not used
+// batch kernel
 template <int F, uint32_t... K>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(Waves<F>::value)))
 void batch_grid_f64_spec(const BatchArgs A, const GridIn in, const RaysOut out) {
-  extern __shared__ double staged[];
-  Tracer64Spec<F, K...> tr{{A, in, out, reinterpret_cast<TraceSpec *>(staged),
-                            reinterpret_cast<optk_surface *>(reinterpret_cast<TraceSpec *>(staged) + 1)}};
+  Tracer64Spec<F, K...> tr(A, in, out);
   batch_loop(A, tr);
 }
 
@@ -674,8 +765,6 @@ static const BatchSpec64 BATCH_SPEC64[NUM_SIGNATURES] = {
 
 namespace optk {
 
-size_t batch_lds_f64(int num_surfaces) { return staged_bytes(num_surfaces); }
-
 static void *batch_kernel_f64(int features, int signature) {
   if (signature >= 0 && signature < NUM_SIGNATURES && BATCH_SPEC64[signature])
     return (void *)BATCH_SPEC64[signature];
@@ -684,26 +773,18 @@ static void *batch_kernel_f64(int features, int signature) {
   return (void *)batch_grid_f64<FEAT_ALL>;
 }
 
-int batch_occupancy_f64(int features, int signature, int block, size_t lds) {
+int batch_occupancy_f64(int features, int signature, int block) {
   int nb = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_kernel_f64(features, signature), block,
-                                                   lds) != hipSuccess)
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_kernel_f64(features, signature), block, 0) !=
+      hipSuccess)
     return 0;
   return nb;
 }
 
 hipError_t batch_launch_f64(int features, int signature, int blocks, int block, const BatchArgs &A,
                             const GridIn &in, const RaysOut &out, hipStream_t stream) {
-  size_t lds = staged_bytes(A.num_surfaces);
-  if (signature >= 0 && signature < NUM_SIGNATURES && BATCH_SPEC64[signature])
-    hipLaunchKernelGGL(BATCH_SPEC64[signature], dim3(blocks), dim3(block), lds, stream, A, in, out);
-  else if (features == 0)
-    hipLaunchKernelGGL(batch_grid_f64<0>, dim3(blocks), dim3(block), lds, stream, A, in, out);
-  else if (features == (FEAT_TOROID | FEAT_RULINGS))
-    hipLaunchKernelGGL(batch_grid_f64<FEAT_TOROID | FEAT_RULINGS>, dim3(blocks), dim3(block), lds,
-                       stream, A, in, out);
-  else
-    hipLaunchKernelGGL(batch_grid_f64<FEAT_ALL>, dim3(blocks), dim3(block), lds, stream, A, in, out);
+  typedef void (*Kernel)(BatchArgs, GridIn, RaysOut);
+  hipLaunchKernelGGL((Kernel)batch_kernel_f64(features, signature), dim3(blocks), dim3(block), 0, stream, A, in, out);
   return hipGetLastError();
 }
 

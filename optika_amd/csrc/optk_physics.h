@@ -567,27 +567,33 @@ OPTK_HD C<T> layer_index(const optk_layer &L, const StackView &sv, T wavelength)
                             sv.grids ? sv.grids + L.chemical : nullptr, sv.grid_lo));
 }
 
+// the indices of a block's first 4 layers (named fields: an array would be
+// promoted to LDS, 64 bytes a thread)
+template <typename T> struct LayerIndices {
+  C<T> n0, n1, n2, n3;
+};
+
 // LayerSequence.transfer over layers first .. first + count - 1, both
 // polarizations; `n_cache` holds the indices of the first 4 layers when
 // `cached` (a periodic block's second pass reuses its first pass's lookups)
 template <typename T, bool SMOOTH = false>
 OPTK_HD M2Pair<T> sequence_transfer2(const StackView &sv, int first, int count, T wavelength,
-                                     LayerState<T> &st, C<T> n_cache[4], bool cached) {
+                                     LayerState<T> &st, LayerIndices<T> &n_cache, bool cached) {
   M2Pair<T> result = {midentity<T>(), midentity<T>()};
   for (int i = 0; i < count; ++i) {
     const optk_layer &L = sv.layers[first + i];
     C<T> n_int;
     if (i < 4 && cached) {
-      n_int = n_cache[0];
-      if (i == 1) n_int = n_cache[1];
-      if (i == 2) n_int = n_cache[2];
-      if (i == 3) n_int = n_cache[3];
+      n_int = n_cache.n0;
+      if (i == 1) n_int = n_cache.n1;
+      if (i == 2) n_int = n_cache.n2;
+      if (i == 3) n_int = n_cache.n3;
     } else {
       n_int = layer_index<T>(L, sv, wavelength);
-      if (i == 0) n_cache[0] = n_int;
-      if (i == 1) n_cache[1] = n_int;
-      if (i == 2) n_cache[2] = n_int;
-      if (i == 3) n_cache[3] = n_int;
+      if (i == 0) n_cache.n0 = n_int;
+      if (i == 1) n_cache.n1 = n_int;
+      if (i == 2) n_cache.n2 = n_int;
+      if (i == 3) n_cache.n3 = n_int;
     }
     M2Pair<T> x = layer_transfer2<T, SMOOTH>(L, n_int, wavelength, st, T(L.thickness));
     result.s = mmul(result.s, x.s);
@@ -613,7 +619,7 @@ OPTK_HD MultilayerOut<T> multilayer_rt(const StackView &sv, int stack_index, T w
   bool first_block = true;
   for (int b = 0; b < stk.num_blocks; ++b) {
     const optk_block &blk = stk.blocks[b];
-    C<T> n_cache[4];
+    LayerIndices<T> n_cache = {};
     M2Pair<T> x;
     if (blk.kind == OPTK_BLOCK_PERIODIC) {
       M2Pair<T> start =
@@ -730,7 +736,15 @@ OPTK_HD double ml_rcp(double x) {
   return 1.0 / x;
 #endif
 }
-OPTK_HD float ml_rcp(float x) { return 1.0f / x; }
+// float32: the hardware reciprocal (1 ulp) and one Newton step
+OPTK_HD float ml_rcp(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float r = __builtin_amdgcn_rcpf(x);
+  return ml_fma(r, ml_fma(-x, r, 1.0f), r);
+#else
+  return 1.0f / x;
+#endif
+}
 
 // square root of a finite value >= 0: hardware reciprocal square root
 // (2^-24.2), one coupled Newton step for the root and its half reciprocal

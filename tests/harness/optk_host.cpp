@@ -266,12 +266,11 @@ void host_multilayer_column(const optk_system_desc *d, const double *wl, const d
                             const double *n_im, int64_t n, int film, int general, double *eff64, double *eff32, uint8_t *ok) {
   SystemView v = view_of(d);
   const bool two = !general && is_bilayer(v.sv.layers, v.sv.stacks[0]);
-  std::vector<float> t32(d->tables, d->tables + d->num_tables);
   for (int64_t i = 0; i < n; ++i) {
     const C<double> c64 = {cosine[i], 0.0}, n64 = {n_re[i], n_im[i]};
     const Cf c32 = {(float)cosine[i], 0.0f}, n32 = {(float)n_re[i], (float)n_im[i]};
     const LayerIndex64 at64{v.sv, wl[i]};
-    const LayerIndex32 at32{v.sv, t32.data(), (float)wl[i]};
+    const LayerIndex32 at32{v.sv, (float)wl[i]};
     const MLResult<double> a = two ? multilayer_bilayer<double>(v.sv, 0, wl[i], c64, n64, film != 0, at64)
                                    : multilayer_column<double>(v.sv, 0, wl[i], c64, n64, film != 0, at64);
     const MLResult<float> b = two ? multilayer_bilayer<float>(v.sv, 0, (float)wl[i], c32, n32, film != 0, at32)
