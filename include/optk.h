@@ -426,7 +426,7 @@ int32_t optk_expose(const optk_expose_args *args, int64_t n, void *hip_stream);
 
 /* Batched trace: many instances of one system layout (the same surface
  * kinds, layer stacks and tables; different parameters: tolerance
- * perturbations), each with its own number of rays, in ONE persistent
+ * perturbations), each with its own number of rays, in ONE
  * launch.  Replaces the reference's n-dimensional configurations, where
  * surface parameters broadcast along named axes of the ray arrays
  * (SequentialSystem.shape, optika/systems/_sequential.py:2125-2132;
@@ -445,9 +445,10 @@ typedef struct optk_batch_desc {
   int32_t pad;
 } optk_batch_desc;
 
-/* launch shape of the persistent kernel: threads per block, rays per thread
- * per work tile (a tile is block * rays_per_thread rays of one instance),
- * blocks resident per CU (0: as many as fit) */
+/* launch shape: threads per block, rays per thread per work tile (a tile is
+ * block * rays_per_thread rays of one instance, and a block traces one);
+ * blocks_per_cu must be >= 0 and changes nothing (the hardware keeps as many
+ * blocks as fit) */
 typedef struct optk_tune {
   int32_t block;
   int32_t rays_per_thread;

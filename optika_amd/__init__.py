@@ -7,7 +7,7 @@ path: ``systems.SequentialSystem`` (``raytrace``, ``rayfunction``),
 ``accumulate_rays``, the ``sags``, ``rulings``, ``apertures`` and
 ``materials`` operators and ``sensors.ImagingSensor.collect`` keep their
 names and arguments.  ``BatchedSystem`` traces many perturbed instances of
-one layout, each with its own ray count, in one persistent launch.  Units are fixed instead of carried: millimetres,
+one layout, each with its own ray count, in one launch.  Units are fixed instead of carried: millimetres,
 nanometres, degrees, 1/mm.
 
 All of them run on the GPU through ``liboptk.so`` (hand-written gfx950 HIP

@@ -1,5 +1,5 @@
 """Batched traces of many instances of one system layout (tolerance
-analysis), each instance with its own number of rays, in one persistent
+analysis), each instance with its own number of rays, in one
 launch (``optk_batch_*``).
 
 The reference expresses such ensembles as n-dimensional configurations:

@@ -1,6 +1,6 @@
-// optk_batch.hip -- host side of the batched persistent trace (optk_batch_*):
+// optk_batch.hip -- host side of the batched trace (optk_batch_*):
 // per-instance records, the work-tile table, the launch-shape autotuner and
-// hipGraph capture/replay.  The persistent kernels themselves live with
+// hipGraph capture/replay.  The kernels themselves live with
 // their forms (optk_lib.hip: float64, optk_fast.hip: float32).
 
 #include <cstring>
@@ -14,9 +14,8 @@ using namespace optk;
 
 namespace {
 
-__global__ __launch_bounds__(256) void batch_zero(double *stats, int64_t count, int32_t *counter) {
+__global__ __launch_bounds__(256) void batch_zero(double *stats, int64_t count) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) *counter = 0;
   for (; i < count; i += (int64_t)gridDim.x * blockDim.x) stats[i] = 0.0;
 }
 
@@ -36,7 +35,7 @@ __global__ __launch_bounds__(256) void batch_finalize(double *stats, const int64
 }
 
 struct LaunchShape {
-  int block, rays_per_thread, blocks;
+  int block, rays_per_thread;
 };
 
 }  // namespace
@@ -47,7 +46,6 @@ struct optk_batch {
   int32_t num_paths = 1;
   int32_t features = 0;
   int32_t signature = -1;  // the instances' common surface-kind signature, or -1
-  int32_t num_cus = 0;
   // shared by every instance
   optk_layer *layers = nullptr;
   optk_stack *stacks = nullptr;
@@ -61,8 +59,7 @@ struct optk_batch {
   TraceSpec *specs64 = nullptr;
   FastSurface *fast = nullptr;
   FastSpec *fast_specs = nullptr;
-  // work queue and tiles
-  int32_t *counter = nullptr;
+  // work tiles
   int64_t *counts = nullptr;  // rays per instance (device)
   BatchTile *tiles = nullptr;
   int64_t tiles_capacity = 0;
@@ -102,7 +99,6 @@ void release(optk_batch *b) {
   (void)hipFree(b->specs64);
   (void)hipFree(b->fast);
   (void)hipFree(b->fast_specs);
-  (void)hipFree(b->counter);
   (void)hipFree(b->counts);
   (void)hipFree(b->tiles);
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
@@ -221,26 +217,18 @@ int call_signature(const optk_batch *b, int32_t flags) {
   return (flags & OPTK_TRACE_GENERIC) ? -1 : b->signature;
 }
 
-int resident_blocks(const optk_batch *b, int32_t precision, int block, int32_t flags) {
-  const int sig = call_signature(b, flags);
-  if (precision == OPTK_F64)
-    return batch_occupancy_f64(b->features, sig, block);
-  return batch_occupancy_f32(b->features, sig, block);
-}
-
-// zero the statistics and the queue head, run the persistent kernel, reduce
-// the statistics: three launches on `stream`, no host synchronisation
+// zero the statistics, trace every tile, reduce the statistics: launches on
+// `stream` (three, up to 2^22 tiles), no host synchronisation
 int32_t enqueue(optk_batch *b, int32_t precision, const Inputs &io, double *stats,
                 const LaunchShape &shape, int32_t flags, int64_t n, hipStream_t stream) {
   const int64_t nstats = (int64_t)b->num_instances * b->num_paths * OPTK_BATCH_STATS;
-  hipLaunchKernelGGL(batch_zero, dim3(64), dim3(256), 0, stream, stats, nstats, b->counter);
+  hipLaunchKernelGGL(batch_zero, dim3(64), dim3(256), 0, stream, stats, nstats);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(OPTK_EDEVICE, std::string("batch zero: ") + hipGetErrorString(e));
   BatchArgs A;
   std::memset(&A, 0, sizeof(A));
   A.tiles = b->tiles;
   A.num_tiles = b->num_tiles;
-  A.counter = b->counter;
   A.rays_per_thread = shape.rays_per_thread;
   A.num_surfaces = b->num_surfaces;
   A.num_paths = b->num_paths;
@@ -258,11 +246,14 @@ int32_t enqueue(optk_batch *b, int32_t precision, const Inputs &io, double *stat
   A.tables32 = b->tables32;
   A.stats = stats;
   A.n = n;
-  if (b->num_tiles > 0) {
-    const int sig = call_signature(b, flags);
-    e = precision == OPTK_F64
-            ? batch_launch_f64(b->features, sig, shape.blocks, shape.block, A, io.g64, io.o64, stream)
-            : batch_launch_f32(b->features, sig, shape.blocks, shape.block, A, io.g32, io.o32, stream);
+  const int sig = call_signature(b, flags);
+  const int64_t most = (int64_t)1 << 22;  // tiles a launch (2^31 threads at 512)
+  for (int64_t first = 0; first < b->num_tiles; first += most) {
+    A.first_tile = first;
+    const dim3 grid((unsigned)(b->num_tiles - first < most ? b->num_tiles - first : most),
+                    (unsigned)((b->num_paths + 1) / 2));
+    e = precision == OPTK_F64 ? batch_launch_f64(b->features, sig, grid, shape.block, A, io.g64, io.o64, stream)
+                              : batch_launch_f32(b->features, sig, grid, shape.block, A, io.g32, io.o32, stream);
     if (e != hipSuccess) return fail(OPTK_EDEVICE, std::string("batch trace: ") + hipGetErrorString(e));
   }
   const int64_t pairs = (int64_t)b->num_instances * b->num_paths;
@@ -284,16 +275,11 @@ int32_t check_call(const optk_batch *b, int32_t precision, const optk_grid *in,
   return OPTK_OK;
 }
 
-int32_t shape_for(optk_batch *b, int32_t precision, const optk_tune &t, int32_t flags,
-                  LaunchShape &shape) {
+int32_t shape_for(const optk_tune &t, LaunchShape &shape) {
   int32_t rc = check_tune(t);
   if (rc) return rc;
-  int fit = resident_blocks(b, precision, t.block, flags);
-  if (fit <= 0) return fail(OPTK_EDEVICE, "the batched kernel does not fit on a CU at this block size");
-  int per_cu = (t.blocks_per_cu > 0 && t.blocks_per_cu < fit) ? t.blocks_per_cu : fit;
   shape.block = t.block;
   shape.rays_per_thread = t.rays_per_thread;
-  shape.blocks = per_cu * b->num_cus;
   return OPTK_OK;
 }
 
@@ -352,10 +338,7 @@ int32_t optk_batch_create(const optk_batch_desc *desc, optk_batch **out) {
   b->num_paths = base.num_paths;
   b->features = features;
   b->signature = signature;
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e == hipSuccess) e = hipDeviceGetAttribute(&b->num_cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (e == hipSuccess) e = hipStreamCreate(&b->capture);
+  hipError_t e = hipStreamCreate(&b->capture);
   if (e != hipSuccess) {
     release(b);
     delete b;
@@ -406,8 +389,7 @@ int32_t optk_batch_create(const optk_batch_desc *desc, optk_batch **out) {
     delete b;
     return rc;
   }
-  e = hipMalloc((void **)&b->counter, sizeof(int32_t));
-  if (e == hipSuccess) e = hipMalloc((void **)&b->counts, sizeof(int64_t) * N);
+  e = hipMalloc((void **)&b->counts, sizeof(int64_t) * N);
   if (e != hipSuccess) {
     release(b);
     delete b;
@@ -429,9 +411,9 @@ int32_t optk_batch_trace(optk_batch *b, int32_t precision, const optk_grid *in,
   else if (b->have_tuned[precision])
     t = b->tuned[precision];
   else
-    t = optk_tune{256, 2, 0, 0, 0.0};
+    t = optk_tune{128, 1, 0, 0, 0.0};
   LaunchShape shape;
-  if ((rc = shape_for(b, precision, t, flags, shape))) return rc;
+  if ((rc = shape_for(t, shape))) return rc;
   if ((rc = prepare_tiles(b, offsets, (int64_t)shape.block * shape.rays_per_thread))) return rc;
   const int64_t n = offsets[b->num_instances];
   Inputs io;
@@ -498,7 +480,7 @@ int32_t optk_batch_autotune(optk_batch *b, int32_t precision, const optk_grid *i
     for (int ri = 0; ri < 4 && rc == OPTK_OK; ++ri) {
       optk_tune t = {blocks[bi], rpts[ri], 0, 0, 0.0};
       LaunchShape shape;
-      if (shape_for(b, precision, t, flags, shape) != OPTK_OK) continue;  // does not fit: skip
+      if (shape_for(t, shape) != OPTK_OK) continue;  // does not fit: skip
       if ((rc = prepare_tiles(b, offsets, (int64_t)shape.block * shape.rays_per_thread))) break;
       if ((rc = enqueue(b, precision, io, stats, shape, flags, n, stream))) break;  // warm-up
       float best_ms = INFINITY;

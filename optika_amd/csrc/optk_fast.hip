@@ -194,8 +194,11 @@ template <int F> struct FastSpecWaves {
 template <int F> struct BatchWaves {
   static constexpr int value = (F & FEAT_MULTILAYER) ? 2 : 4;
 };
-template <int F> struct BatchSpecWaves {
-  static constexpr int value = 3;
+// the specialised ones with several rays per thread 3 (at 4 the loop over
+// rays spills: 4.1 ms against 1.1 on the tolerance batch), with one ray per
+// thread 4 (782 us, at 3 waves 815)
+template <bool ONE> struct BatchSpecWaves {
+  static constexpr int value = ONE ? 4 : 3;
 };
 
 // The system's records are read through the constant address space: every
@@ -487,7 +490,7 @@ int32_t launch(const KernelSet<In> &ks, bool special, const optk_system *sys, co
   return OPTK_OK;
 }
 
-// batched persistent trace, float32 form ------------------------------------
+// batched trace, float32 form ------------------------------------
 
 // a batched path whose multilayers are left to the float64 routine: the
 // final ray, written out and returned (kernels with the arguments
@@ -645,27 +648,30 @@ template <int F>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(BatchWaves<F>::value)))
 void batch_grid_f32(const BatchArgs A, const FGridIn in, const FRaysOut out) {
   Tracer32<F> tr(A, in, out);
-  batch_loop(A, tr);
+  batch_tile<false>(A, tr);
 }
 
-template <int F, uint32_t... K>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(BatchSpecWaves<F>::value)))
+template <bool ONE, int F, uint32_t... K>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(BatchSpecWaves<ONE>::value)))
 void batch_grid_f32_spec(const BatchArgs A, const FGridIn in, const FRaysOut out) {
   Tracer32Spec<F, K...> tr(A, in, out);
-  batch_loop(A, tr);
+  batch_tile<ONE>(A, tr);
 }
 
 typedef void (*BatchSpec32)(BatchArgs, FGridIn, FRaysOut);
-// by signature; the geometric Newtonian layout keeps the generic kernel
-const BatchSpec32 BATCH_SPEC32[NUM_SIGNATURES] = {
-    nullptr,
-    batch_grid_f32_spec<SIGNATURES[SIG_SPECTROGRAPH].features, OPTK_SIGNATURE_SPECTROGRAPH>,
-    batch_grid_f32_spec<SIGNATURES[SIG_SPECTROGRAPH_TILTED].features, OPTK_SIGNATURE_SPECTROGRAPH_TILTED>,
+// by signature and by whether each thread traces one ray; the geometric
+// Newtonian layout keeps the generic kernel
+const BatchSpec32 BATCH_SPEC32[NUM_SIGNATURES][2] = {
+    {nullptr, nullptr},
+    {batch_grid_f32_spec<false, SIGNATURES[SIG_SPECTROGRAPH].features, OPTK_SIGNATURE_SPECTROGRAPH>,
+     batch_grid_f32_spec<true, SIGNATURES[SIG_SPECTROGRAPH].features, OPTK_SIGNATURE_SPECTROGRAPH>},
+    {batch_grid_f32_spec<false, SIGNATURES[SIG_SPECTROGRAPH_TILTED].features, OPTK_SIGNATURE_SPECTROGRAPH_TILTED>,
+     batch_grid_f32_spec<true, SIGNATURES[SIG_SPECTROGRAPH_TILTED].features, OPTK_SIGNATURE_SPECTROGRAPH_TILTED>},
 };
 
-void *batch_kernel_f32(int features, int signature) {
-  if (signature >= 0 && signature < NUM_SIGNATURES && BATCH_SPEC32[signature])
-    return (void *)BATCH_SPEC32[signature];
+void *batch_kernel_f32(int features, int signature, bool one) {
+  if (signature >= 0 && signature < NUM_SIGNATURES && BATCH_SPEC32[signature][one])
+    return (void *)BATCH_SPEC32[signature][one];
   if (features == 0) return (void *)batch_grid_f32<0>;
   if (features == (FEAT_TOROID | FEAT_RULINGS)) return (void *)batch_grid_f32<FEAT_TOROID | FEAT_RULINGS>;
   return (void *)batch_grid_f32<FEAT_ALL>;
@@ -700,18 +706,11 @@ int32_t fast_trace_grid(const optk_system *sys, const FGridIn &in, const FRaysOu
                          stream);
 }
 
-int batch_occupancy_f32(int features, int signature, int block) {
-  int nb = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_kernel_f32(features, signature), block, 0) !=
-      hipSuccess)
-    return 0;
-  return nb;
-}
-
-hipError_t batch_launch_f32(int features, int signature, int blocks, int block, const BatchArgs &A,
+hipError_t batch_launch_f32(int features, int signature, dim3 grid, int block, const BatchArgs &A,
                             const FGridIn &in, const FRaysOut &out, hipStream_t stream) {
   typedef void (*Kernel)(BatchArgs, FGridIn, FRaysOut);
-  hipLaunchKernelGGL((Kernel)batch_kernel_f32(features, signature), dim3(blocks), dim3(block), 0, stream, A, in, out);
+  hipLaunchKernelGGL((Kernel)batch_kernel_f32(features, signature, A.rays_per_thread == 1), grid, dim3(block), 0, stream,
+                     A, in, out);
   return hipGetLastError();
 }
 

@@ -125,7 +125,7 @@ int32_t fast_trace_grid(const optk_system *sys, const FGridIn &in, const FRaysOu
                         hipStream_t stream);
 
 // ---------------------------------------------------------------------------
-// batched persistent trace (optk_batch_*)
+// batched trace (optk_batch_*)
 // ---------------------------------------------------------------------------
 
 // a work tile: `count` consecutive rays of one instance
@@ -138,7 +138,7 @@ struct BatchTile {
 struct BatchArgs {
   const BatchTile *tiles;
   int64_t num_tiles;
-  int32_t *counter;                // work-queue head, zeroed before each launch
+  int64_t first_tile;              // of this launch
   int32_t rays_per_thread;
   int32_t num_surfaces;
   int32_t num_paths;
@@ -153,14 +153,12 @@ struct BatchArgs {
   int64_t n;                       // rays in the batch (output stride per path)
 };
 
-// resident blocks per CU of the kernel covering `features` (0 on error);
+// the kernel covering `features` over a grid of (tiles, pairs of paths);
 // signature >= 0: the instances' common surface-kind signature
 // (optk_signatures.h), whose specialised kernel runs where one exists
-int batch_occupancy_f64(int features, int signature, int block);
-int batch_occupancy_f32(int features, int signature, int block);
-hipError_t batch_launch_f64(int features, int signature, int blocks, int block, const BatchArgs &A,
+hipError_t batch_launch_f64(int features, int signature, dim3 grid, int block, const BatchArgs &A,
                             const GridIn &in, const RaysOut &out, hipStream_t stream);
-hipError_t batch_launch_f32(int features, int signature, int blocks, int block, const BatchArgs &A,
+hipError_t batch_launch_f32(int features, int signature, dim3 grid, int block, const BatchArgs &A,
                             const FGridIn &in, const FRaysOut &out, hipStream_t stream);
 
 #if defined(__HIPCC__)

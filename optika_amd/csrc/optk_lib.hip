@@ -616,7 +616,7 @@ __global__ __launch_bounds__(256) void expose_kernel(const optk_expose_args a, i
   }
 }
 
-// batched persistent trace, float64 form ------------------------------------
+// batched trace, float64 form ------------------------------------
 
 // a batched path whose multilayers are left to the reference's operations:
 // the final ray, written out and returned (kernels with the arguments
@@ -743,48 +743,44 @@ template <int F>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(Waves<F>::value)))
 void batch_grid_f64(const BatchArgs A, const GridIn in, const RaysOut out) {
   Tracer64<F> tr(A, in, out);
-  batch_loop(A, tr);
+  batch_tile<false>(A, tr);
 }
 
 // 2 waves per SIMD (256 VGPRs) for the multilayer layouts, as the generic
 // batch kernel
-template <int F, uint32_t... K>
+template <bool ONE, int F, uint32_t... K>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(Waves<F>::value)))
 void batch_grid_f64_spec(const BatchArgs A, const GridIn in, const RaysOut out) {
   Tracer64Spec<F, K...> tr(A, in, out);
-  batch_loop(A, tr);
+  batch_tile<ONE>(A, tr);
 }
 
 typedef void (*BatchSpec64)(BatchArgs, GridIn, RaysOut);
-// by signature; the geometric Newtonian layout keeps the generic kernel
-static const BatchSpec64 BATCH_SPEC64[NUM_SIGNATURES] = {
-    nullptr,
-    batch_grid_f64_spec<SIGNATURES[SIG_SPECTROGRAPH].features, OPTK_SIGNATURE_SPECTROGRAPH>,
-    batch_grid_f64_spec<SIGNATURES[SIG_SPECTROGRAPH_TILTED].features, OPTK_SIGNATURE_SPECTROGRAPH_TILTED>,
+// by signature and by whether each thread traces one ray; the geometric
+// Newtonian layout keeps the generic kernel
+static const BatchSpec64 BATCH_SPEC64[NUM_SIGNATURES][2] = {
+    {nullptr, nullptr},
+    {batch_grid_f64_spec<false, SIGNATURES[SIG_SPECTROGRAPH].features, OPTK_SIGNATURE_SPECTROGRAPH>,
+     batch_grid_f64_spec<true, SIGNATURES[SIG_SPECTROGRAPH].features, OPTK_SIGNATURE_SPECTROGRAPH>},
+    {batch_grid_f64_spec<false, SIGNATURES[SIG_SPECTROGRAPH_TILTED].features, OPTK_SIGNATURE_SPECTROGRAPH_TILTED>,
+     batch_grid_f64_spec<true, SIGNATURES[SIG_SPECTROGRAPH_TILTED].features, OPTK_SIGNATURE_SPECTROGRAPH_TILTED>},
 };
 
 namespace optk {
 
-static void *batch_kernel_f64(int features, int signature) {
-  if (signature >= 0 && signature < NUM_SIGNATURES && BATCH_SPEC64[signature])
-    return (void *)BATCH_SPEC64[signature];
+static void *batch_kernel_f64(int features, int signature, bool one) {
+  if (signature >= 0 && signature < NUM_SIGNATURES && BATCH_SPEC64[signature][one])
+    return (void *)BATCH_SPEC64[signature][one];
   if (features == 0) return (void *)batch_grid_f64<0>;
   if (features == (FEAT_TOROID | FEAT_RULINGS)) return (void *)batch_grid_f64<FEAT_TOROID | FEAT_RULINGS>;
   return (void *)batch_grid_f64<FEAT_ALL>;
 }
 
-int batch_occupancy_f64(int features, int signature, int block) {
-  int nb = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_kernel_f64(features, signature), block, 0) !=
-      hipSuccess)
-    return 0;
-  return nb;
-}
-
-hipError_t batch_launch_f64(int features, int signature, int blocks, int block, const BatchArgs &A,
+hipError_t batch_launch_f64(int features, int signature, dim3 grid, int block, const BatchArgs &A,
                             const GridIn &in, const RaysOut &out, hipStream_t stream) {
   typedef void (*Kernel)(BatchArgs, GridIn, RaysOut);
-  hipLaunchKernelGGL((Kernel)batch_kernel_f64(features, signature), dim3(blocks), dim3(block), 0, stream, A, in, out);
+  hipLaunchKernelGGL((Kernel)batch_kernel_f64(features, signature, A.rays_per_thread == 1), grid, dim3(block), 0, stream,
+                     A, in, out);
   return hipGetLastError();
 }
 
