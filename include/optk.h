@@ -33,6 +33,7 @@
  *                    area_effective (optika/systems/_sequential.py:1208-1512)
  *   optk_denormalize the normalized grid's denormalization
  *                    (optika/systems/_sequential.py:748-789)
+ *   optk_scene_rays  the rays of SequentialSystem.image (one per cell)
  *   optk_expose      AbstractImagingSensor.expose with the ideal sensor
  *                    material (optika/sensors/_sensors.py:173-252)
  */
@@ -423,6 +424,32 @@ typedef struct optk_expose_args {
 } optk_expose_args;
 
 int32_t optk_expose(const optk_expose_args *args, int64_t n, void *hip_stream);
+
+/* Rays of the forward model, one per (wavelength, field, pupil) cell of a
+ * scene: _rayfunction_from_vertices and ObjectVectorArray.cell_area
+ * (optika/systems/_sequential.py:1002-1083,
+ * optika/vectors/_vectors_object.py:52-133).  A ray sits at uniform weights
+ * u[0..4] (wavelength, field x, y, pupil x, y; each [rays]) of its cell,
+ * every coordinate interpolated between the cell's vertices, and carries
+ * radiance x wavelength step x field cell measure x pupil cell measure (a
+ * solid angle in steradians, or an area in mm^2), the measures averaged over
+ * the cell's two wavelength vertices.  Rays are ordered [wavelength][field
+ * x][field y][pupil x][pupil y].  Device pointers, float64. */
+typedef struct optk_scene_args {
+  const double *wavelength;     /* [nw + 1] vertices, nm */
+  const double *axis[4];        /* field x, y, pupil x, y: [nw + 1][n + 1] */
+  const double *radiance;       /* [nw][nx][ny] */
+  const double *u[5];           /* [rays] each */
+  double *measure_field;        /* workspace, [nw][nx][ny] */
+  double *measure_pupil;        /* workspace, [nw][npx][npy] */
+  double *out_wavelength;       /* [rays] */
+  double *out[4];               /* field x, y, pupil x, y: [rays] each */
+  double *flux;                 /* [rays] */
+  int32_t nw, n[4];             /* cells: wavelength; field x, y, pupil x, y */
+  int32_t field_is_angle;       /* 1: field in degrees and pupil in mm, else the other way round */
+} optk_scene_args;
+
+int32_t optk_scene_rays(const optk_scene_args *args, void *hip_stream);
 
 /* Batched trace: many instances of one system layout (the same surface
  * kinds, layer stacks and tables; different parameters: tolerance

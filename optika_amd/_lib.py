@@ -223,6 +223,13 @@ class ExposeArgs(ctypes.Structure):
                 ("pad", c_int32)]
 
 
+class SceneArgs(ctypes.Structure):
+    _fields_ = [("wavelength", c_void_p), ("axis", c_void_p * 4), ("radiance", c_void_p),
+                ("u", c_void_p * 5), ("measure_field", c_void_p), ("measure_pupil", c_void_p),
+                ("out_wavelength", c_void_p), ("out", c_void_p * 4), ("flux", c_void_p),
+                ("nw", c_int32), ("n", c_int32 * 4), ("field_is_angle", c_int32)]
+
+
 class PupilArgs(ctypes.Structure):
     _fields_ = [("x", c_void_p), ("y", c_void_p), ("intensity", c_void_p), ("unvignetted", c_void_p),
                 ("weight", c_void_p), ("per_segment", c_int64), ("count", c_void_p),
@@ -355,6 +362,8 @@ def lib() -> ctypes.CDLL:
     L.optk_surrogate_infer.restype = c_int32
     L.optk_surrogate_infer.argtypes = [ctypes.POINTER(SurrogateDesc), ctypes.POINTER(SurrogateIO),
                                        c_void_p]
+    L.optk_scene_rays.restype = c_int32
+    L.optk_scene_rays.argtypes = [ctypes.POINTER(SceneArgs), c_void_p]
     L.optk_expose.restype = c_int32
     L.optk_expose.argtypes = [ctypes.POINTER(ExposeArgs), c_int64, c_void_p]
     L.optk_pupil_reduce.restype = c_int32
@@ -380,7 +389,7 @@ def lib() -> ctypes.CDLL:
                       ("optk_mlp_args", MlpArgs), ("optk_surrogate_desc", SurrogateDesc),
                       ("optk_surrogate_io", SurrogateIO), ("optk_stop_args", StopArgs),
                       ("optk_pupil_args", PupilArgs), ("optk_denormalize_args", DenormalizeArgs),
-                      ("optk_expose_args", ExposeArgs)]:
+                      ("optk_expose_args", ExposeArgs), ("optk_scene_args", SceneArgs)]:
         size = L.optk_sizeof(name.encode())
         if size != ctypes.sizeof(cls):
             raise OptkError(f"record {name}: C size {size} != binding size {ctypes.sizeof(cls)}")

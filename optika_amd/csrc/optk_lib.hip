@@ -616,6 +616,99 @@ __global__ __launch_bounds__(256) void expose_kernel(const optk_expose_args a, i
   }
 }
 
+// rays of a scene (optk_scene_rays) -----------------------------------------
+//
+// Two kernels in place of host numpy (the cells' solid angles: 11 ms for 4
+// bands of 128 x 128 cells) and about forty elementwise kernels over the
+// rays: the measures, a thread per cell, and the rays, a thread per ray
+// (40 bytes of weights in, 48 out; HBM-bound).
+
+struct Unit3 {
+  double x, y, z;
+};
+
+__device__ __forceinline__ Unit3 unit_direction(double ax_deg, double ay_deg) {  // optika/_util.py:41-73
+  const double deg = 0.017453292519943295;
+  double sx, cx, sy, cy;
+  sincos(ax_deg * deg, &sx, &cx);
+  sincos(ay_deg * deg, &sy, &cy);
+  return {-cy * sx, -sy, cy * cx};
+}
+
+// signed solid angle of the spherical triangle of unit vectors a, b, c: tan
+// (omega / 2) = a . (b x c) / (1 + a.b + b.c + c.a) (Van Oosterom and
+// Strackee, IEEE Trans. Biomed. Eng. 30, 125 (1983)).  The triple product is
+// taken of the sides b - a and c - a, which is the same value: of the unit
+// vectors themselves it cancels to the square of the cell's size (relative
+// error 5e-7 for cells of 1e-5 rad, against 1e-11).
+__device__ __forceinline__ double triangle_solid_angle(Unit3 a, Unit3 b, Unit3 c) {
+  const double ux = b.x - a.x, uy = b.y - a.y, uz = b.z - a.z;
+  const double vx = c.x - a.x, vy = c.y - a.y, vz = c.z - a.z;
+  const double triple = a.x * (uy * vz - uz * vy) + a.y * (uz * vx - ux * vz) + a.z * (ux * vy - uy * vx);
+  const double den = 1.0 + (a.x * b.x + a.y * b.y + a.z * b.z) + (b.x * c.x + b.y * c.y + b.z * c.z) +
+                     (c.x * a.x + c.y * a.y + c.z * a.z);
+  return 2.0 * atan2(triple, den);
+}
+
+// measure of the cell of vertices x0, x1 by y0, y1
+__device__ __forceinline__ double cell_measure(double x0, double x1, double y0, double y1, bool angle) {
+  if (!angle) return fabs((x1 - x0) * (y1 - y0));
+  const Unit3 v00 = unit_direction(x0, y0), v10 = unit_direction(x1, y0);
+  const Unit3 v11 = unit_direction(x1, y1), v01 = unit_direction(x0, y1);
+  return fabs(triangle_solid_angle(v00, v10, v11) + triangle_solid_angle(v00, v11, v01));
+}
+
+__global__ __launch_bounds__(256) void scene_measures(const optk_scene_args a, int64_t cells) {
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= cells) return;
+  const int64_t field_cells = (int64_t)a.nw * a.n[0] * a.n[1];
+  const int pupil = i >= field_cells ? 1 : 0;
+  double *out = pupil ? a.measure_pupil : a.measure_field;
+  if (pupil) i -= field_cells;
+  const double *vx = a.axis[2 * pupil], *vy = a.axis[2 * pupil + 1];
+  const int64_t nx = a.n[2 * pupil], ny = a.n[2 * pupil + 1];
+  const int64_t w = i / (nx * ny), x = i / ny % nx, y = i % ny;
+  const bool angle = (a.field_is_angle != 0) != (pupil != 0);
+  double m[2];
+  for (int k = 0; k < 2; ++k) {
+    const double *px = vx + (w + k) * (nx + 1) + x, *py = vy + (w + k) * (ny + 1) + y;
+    m[k] = cell_measure(px[0], px[1], py[0], py[1], angle);
+  }
+  out[i] = (m[0] + m[1]) / 2.0;
+}
+
+// the coordinate at weight uw between wavelength vertices and uc between the
+// cell's two vertices along its own axis
+__device__ __forceinline__ double between(const double *v, int64_t w, int64_t count, int64_t c, double uw, double uc) {
+  const double *lo = v + w * (count + 1) + c, *hi = lo + count + 1;
+  const double p = lo[0] + (hi[0] - lo[0]) * uw;
+  const double q = lo[1] + (hi[1] - lo[1]) * uw;
+  return p + (q - p) * uc;
+}
+
+template <typename I> __global__ __launch_bounds__(256) void scene_rays(const optk_scene_args a, int64_t rays) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= rays) return;
+  I rest = (I)i;
+  const I py = rest % (I)a.n[3];
+  rest /= (I)a.n[3];
+  const I px = rest % (I)a.n[2];
+  const I cell = rest / (I)a.n[2];
+  const I y = cell % (I)a.n[1];
+  rest = cell / (I)a.n[1];
+  const I x = rest % (I)a.n[0];
+  const I w = rest / (I)a.n[0];
+  const double uw = a.u[0][i];
+  const double w0 = a.wavelength[w], w1 = a.wavelength[w + 1];
+  put<double>(a.out_wavelength[i], w0 + (w1 - w0) * uw);
+  put<double>(a.out[0][i], between(a.axis[0], w, a.n[0], x, uw, a.u[1][i]));
+  put<double>(a.out[1][i], between(a.axis[1], w, a.n[1], y, uw, a.u[2][i]));
+  put<double>(a.out[2][i], between(a.axis[2], w, a.n[2], px, uw, a.u[3][i]));
+  put<double>(a.out[3][i], between(a.axis[3], w, a.n[3], py, uw, a.u[4][i]));
+  const double volume = fabs(w1 - w0) * a.measure_field[cell] * a.measure_pupil[(w * (I)a.n[2] + px) * (I)a.n[3] + py];
+  put<double>(a.flux[i], a.radiance[cell] * volume);
+}
+
 // batched trace, float64 form ------------------------------------
 
 // a batched path whose multilayers are left to the reference's operations:
@@ -1579,6 +1672,7 @@ int64_t optk_sizeof(const char *name) {
   if (s == "optk_stop_args") return sizeof(optk_stop_args);
   if (s == "optk_pupil_args") return sizeof(optk_pupil_args);
   if (s == "optk_denormalize_args") return sizeof(optk_denormalize_args);
+  if (s == "optk_scene_args") return sizeof(optk_scene_args);
   if (s == "optk_expose_args") return sizeof(optk_expose_args);
   return -1;
 }
@@ -1944,6 +2038,34 @@ int32_t optk_denormalize(const optk_denormalize_args *args, int64_t n, void *hip
   if ((n + 255) / 256 > INT32_MAX) return fail(OPTK_EINVAL, "too many values");
   hipLaunchKernelGGL(denormalize_kernel, grid_for(n), dim3(256), 0, (hipStream_t)hip_stream, *args,
                      ncomp, n);
+  OPTK_HIP_CHECK(hipGetLastError());
+  return OPTK_OK;
+}
+
+int32_t optk_scene_rays(const optk_scene_args *args, void *hip_stream) {
+  if (!args) return fail(OPTK_EINVAL, "null argument");
+  const optk_scene_args &a = *args;
+  int64_t rays = a.nw;
+  bool none = a.nw == 0;
+  if (a.nw < 0) return fail(OPTK_EINVAL, "negative count");
+  for (int k = 0; k < 4; ++k) {
+    if (a.n[k] < 0) return fail(OPTK_EINVAL, "negative count");
+    none = none || a.n[k] == 0;
+    if (a.n[k] > 0 && rays > ((int64_t)1 << 40) / a.n[k]) return fail(OPTK_EINVAL, "too many cells");
+    rays *= a.n[k];
+  }
+  if (none) return OPTK_OK;
+  bool missing = !a.wavelength || !a.radiance || !a.measure_field || !a.measure_pupil || !a.out_wavelength || !a.flux;
+  for (int k = 0; k < 4; ++k) missing = missing || !a.axis[k] || !a.out[k];
+  for (int k = 0; k < 5; ++k) missing = missing || !a.u[k];
+  if (missing) return fail(OPTK_EINVAL, "missing scene array");
+  hipStream_t s = (hipStream_t)hip_stream;
+  const int64_t cells = (int64_t)a.nw * ((int64_t)a.n[0] * a.n[1] + (int64_t)a.n[2] * a.n[3]);
+  hipLaunchKernelGGL(scene_measures, grid_for(cells), dim3(256), 0, s, a, cells);
+  if (rays <= INT32_MAX)
+    hipLaunchKernelGGL(scene_rays<uint32_t>, grid_for(rays), dim3(256), 0, s, a, rays);
+  else
+    hipLaunchKernelGGL(scene_rays<uint64_t>, grid_for(rays), dim3(256), 0, s, a, rays);
   OPTK_HIP_CHECK(hipGetLastError());
   return OPTK_OK;
 }

@@ -344,79 +344,41 @@ class AbstractSequentialSystem:
         device, binned on the sensor's pixels over the wavelength cells and
         exposed (``measure``).  Returns [W][Nx][Ny] electrons, or [Nx][Ny]
         with ``integrate``."""
-        from .pupil import solid_angle_cells
+        import torch
+
+        from . import _scene, _trace
 
         h = lambda v: np.asarray(v.detach().cpu().numpy() if hasattr(v, "detach") else v,  # noqa: E731
                                  np.float64).reshape(-1)
         wv, fxv, fyv = h(wavelength), h(field_x), h(field_y)
         W, X, Y = wv.size - 1, fxv.size - 1, fyv.size - 1
-        R = h(radiance).reshape(W, X, Y)
+        R = radiance if isinstance(radiance, torch.Tensor) else np.asarray(radiance, np.float64)
+        if int(np.prod(R.shape)) != W * X * Y:
+            raise ValueError(f"cannot reshape radiance of shape {tuple(R.shape)} into shape ({W},{X},{Y})")
         pxv, pyv = (np.array([-1.0, 1.0]), np.array([-1.0, 1.0])) if pupil is None else \
             (h(pupil.x), h(pupil.y))
-        PX, PY = pxv.size - 1, pyv.size - 1
         # vertex coordinates per wavelength vertex: [W + 1][.. + 1]
-        fx_v, fy_v = np.broadcast_to(fxv, (W + 1, X + 1)), np.broadcast_to(fyv, (W + 1, Y + 1))
-        px_v, py_v = np.broadcast_to(pxv, (W + 1, PX + 1)), np.broadcast_to(pyv, (W + 1, PY + 1))
+        axes = [np.broadcast_to(v, (W + 1, v.size)) for v in (fxv, fyv, pxv, pyv)]
         if normalized_field or normalized_pupil:
             flo, fspan, plo, pspan = self._extents(wv)
             if normalized_field:
-                fx_v = fspan[0][:, None] * (fxv + 1) / 2 + flo[0][:, None]
-                fy_v = fspan[1][:, None] * (fyv + 1) / 2 + flo[1][:, None]
+                axes[0] = fspan[0][:, None] * (fxv + 1) / 2 + flo[0][:, None]
+                axes[1] = fspan[1][:, None] * (fyv + 1) / 2 + flo[1][:, None]
             if normalized_pupil:
-                px_v = pspan[0][:, None] * (pxv + 1) / 2 + plo[0][:, None]
-                py_v = pspan[1][:, None] * (pyv + 1) / 2 + plo[1][:, None]
-        # cell measures (cell_area): the field is an angle for an object at
-        # infinity and the pupil a position, else the other way round
-        at_inf = self.object_is_at_infinity
-
-        def measure(vx, vy, angular):
-            if angular:
-                return solid_angle_cells(vx, vy)
-            return np.abs(np.diff(vx, axis=-1)[..., :, None] * np.diff(vy, axis=-1)[..., None, :])
-
-        a_field = measure(fx_v, fy_v, at_inf)           # [W + 1][X][Y]
-        a_pupil = measure(px_v, py_v, not at_inf)       # [W + 1][PX][PY]
-        a_field = (a_field[:-1] + a_field[1:]) / 2      # cell centers along wavelength
-        a_pupil = (a_pupil[:-1] + a_pupil[1:]) / 2
-        shape = (W, X, Y, PX, PY)
-        import torch
-
-        from . import _trace
-
+                axes[2] = pspan[0][:, None] * (pxv + 1) / 2 + plo[0][:, None]
+                axes[3] = pspan[1][:, None] * (pyv + 1) / 2 + plo[1][:, None]
         # the rays of every cell are generated on the device (a seeded
-        # device generator places each ray in its cell)
+        # device generator places each ray in its cell); the field is an
+        # angle for an object at infinity and the pupil a position, else the
+        # other way round
         dev = _trace.device()
         gen = torch.Generator(device=dev)
         gen.manual_seed(int(seed))
-        T = lambda a: torch.as_tensor(np.ascontiguousarray(a, np.float64), device=dev)  # noqa: E731
-        u = torch.rand((5,) + shape, generator=gen, device=dev, dtype=torch.float64)
-        uw = u[0]
-        wvt = T(wv)
-        lam = wvt[:-1, None, None, None, None] + (wvt[1:] - wvt[:-1])[:, None, None, None, None] * uw
-
-        def between(v, axis_shape, uc):
-            """the coordinate at weight uw between wavelength vertices and
-            uc between the cell's two vertices along its own axis"""
-            v = T(v)
-            lo = v[:-1, :-1].reshape(axis_shape)       # [W][n] at the cell's lower vertex
-            hi = v[:-1, 1:].reshape(axis_shape)
-            lo2 = v[1:, :-1].reshape(axis_shape)        # next wavelength vertex
-            hi2 = v[1:, 1:].reshape(axis_shape)
-            a = lo + (lo2 - lo) * uw
-            b = hi + (hi2 - hi) * uw
-            return a + (b - a) * uc
-
-        fx = between(fx_v, (W, X, 1, 1, 1), u[1])
-        fy = between(fy_v, (W, 1, Y, 1, 1), u[2])
-        px = between(px_v, (W, 1, 1, PX, 1), u[3])
-        py = between(py_v, (W, 1, 1, 1, PY), u[4])
-        volume = (T(np.abs(np.diff(wv)))[:, None, None, None, None]
-                  * T(a_field)[:, :, :, None, None] * T(a_pupil)[:, None, None, :, :])
-        flux = T(R)[:, :, :, None, None] * volume
-        flat = lambda a: a.expand(shape).reshape(-1).contiguous()  # noqa: E731
-        rays = self.rayfunction(intensity=flat(flux), wavelength=flat(lam),
-                                field=Cartesian2dVectorArray(flat(fx), flat(fy)),
-                                pupil=Cartesian2dVectorArray(flat(px), flat(py)),
+        u = torch.rand((5, W, X, Y, pxv.size - 1, pyv.size - 1), generator=gen, device=dev, dtype=torch.float64)
+        lam, coords, flux = _scene.rays(wv, axes, R, u, self.object_is_at_infinity)
+        rays = self.rayfunction(intensity=flux, wavelength=lam,
+                                field=Cartesian2dVectorArray(coords[0], coords[1]),
+                                pupil=Cartesian2dVectorArray(coords[2], coords[3]),
                                 normalized_field=False, normalized_pupil=False).outputs
         if rays.position.x.ndim != 1:
             raise NotImplementedError("image of a system with several diffraction orders")
