@@ -13,8 +13,11 @@ record bytes are unchanged.
 
 from __future__ import annotations
 
+import collections
 import ctypes
 import dataclasses
+import struct
+import threading
 from typing import Sequence
 
 import numpy as np
@@ -23,21 +26,65 @@ from . import _lib
 from . import apertures as _ap
 from . import materials as _mat
 from . import rulings as _rl
+from . import transformations as _tf
 from .transformations import AbstractTransformation
 
 __all__ = ["CompiledSystem", "compile_surfaces", "affine_record"]
 
 
+_IDENTITY = _lib.Affine()
+_IDENTITY.m[:] = [1, 0, 0, 0, 1, 0, 0, 0, 1]
+
+# Flattened transformations by their content: the types and the parameter
+# bits of the primitive elements in order.  Composing one takes numpy about
+# 20 us, and a system is compiled again on every call (its parameters may
+# have changed), with three transformations a surface.
+_AFFINES: "collections.OrderedDict[tuple, _lib.Affine]" = collections.OrderedDict()
+_AFFINES_MAX = 1024
+_AFFINES_LOCK = threading.Lock()
+
+
+def _affine_key(t: AbstractTransformation):
+    """The content key of a transformation, or None if an element's type is
+    not one of the package's own (its affine map may depend on anything)."""
+    key = []
+    for e in t.elements():
+        kind = type(e)
+        if kind is _tf.Cartesian3dTranslation:
+            values = (e.x, e.y, e.z)
+        elif kind in (_tf.Cartesian3dRotationX, _tf.Cartesian3dRotationY, _tf.Cartesian3dRotationZ):
+            values = (e.angle,)
+        else:
+            return None
+        key.append(kind)
+        try:
+            key.append(struct.pack(f"{len(values)}d", *values))
+        except (struct.error, TypeError, ValueError):
+            return None
+    return tuple(key)
+
+
 def affine_record(t: None | AbstractTransformation) -> _lib.Affine:
-    a = _lib.Affine()
+    """The flattened record of a transformation (shared: copy, do not edit)."""
     if t is None:
-        a.kind = 0
-        a.m[:] = [1, 0, 0, 0, 1, 0, 0, 0, 1]
-        return a
+        return _IDENTITY
+    key = _affine_key(t)
+    if key is not None:
+        with _AFFINES_LOCK:
+            hit = _AFFINES.get(key)
+            if hit is not None:
+                _AFFINES.move_to_end(key)
+                return hit
+    a = _lib.Affine()
     af = t.affine()
     a.m[:] = [float(v) for v in af.matrix.ravel()]
     a.t[:] = [float(v) for v in af.vector]
     a.kind = 2 if af.has_rotation else 1
+    if key is not None:
+        with _AFFINES_LOCK:
+            _AFFINES[key] = a
+            while len(_AFFINES) > _AFFINES_MAX:
+                _AFFINES.popitem(last=False)
     return a
 
 

@@ -90,8 +90,10 @@ def _scalar(v) -> float:
 
 
 def _numel(v) -> int | None:
-    if isinstance(v, (torch.Tensor, np.ndarray)) and v.ndim > 0:
-        return int(np.prod(v.shape))
+    if isinstance(v, torch.Tensor):
+        return v.numel() if v.ndim > 0 else None
+    if isinstance(v, np.ndarray) and v.ndim > 0:
+        return int(v.size)
     return None
 
 
@@ -124,8 +126,10 @@ class _Out:
 
 
 def _make_rays(out: _Out, shape, scalars: dict) -> RayVectorArray:
+    flat = len(shape) == 1
+
     def shp(t):
-        return t.view(shape)
+        return t if flat else t.view(shape)
 
     def field(name):
         if name in out.t:

@@ -54,6 +54,7 @@ import torch
 
 from . import _lib, _trace
 from .rays import RayVectorArray
+from .sags import NoSag
 from .vectors import Cartesian3dVectorArray
 
 __all__ = ["solve_stop_rays", "rayfunction_stops", "field_pupil", "denormalize", "angles",
@@ -430,7 +431,7 @@ def _rayfunction_stops_path(system, wavelength, samples_pupil_stop, samples_fiel
     obj = back[-1]
     pl = _apply(obj.transformation, p, inverse=True)
     dl = _apply(obj.transformation, d, direction=True, inverse=True)
-    if obj.sag is not None:
+    if obj.sag is not None and type(obj.sag) is not NoSag:  # (a flat sag's normal is -z everywhere)
         from . import _ops
 
         q = _to_device(pl)

@@ -1,0 +1,68 @@
+"""The transformation records kept by content: an edited transformation, a
+negative zero and a subclass each get their own record."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from optika_amd import _compile
+from optika_amd.transformations import (
+    Cartesian3dRotationX,
+    Cartesian3dRotationY,
+    Cartesian3dRotationZ,
+    Cartesian3dTranslation,
+    TransformationList,
+)
+
+
+def _bytes(t):
+    return bytes(_compile.affine_record(t))
+
+
+def _fresh(t):
+    """The record of ``t`` composed without the kept ones."""
+    a = _compile._lib.Affine()
+    af = t.affine()
+    a.m[:] = [float(v) for v in af.matrix.ravel()]
+    a.t[:] = [float(v) for v in af.vector]
+    a.kind = 2 if af.has_rotation else 1
+    return bytes(a)
+
+
+@pytest.mark.parametrize("make", [
+    lambda: Cartesian3dTranslation(x=1.5),
+    lambda: Cartesian3dRotationX(30.0),
+    lambda: TransformationList([Cartesian3dRotationY(135.0), Cartesian3dTranslation(z=np.float32(0.1))]),
+    lambda: TransformationList([TransformationList([Cartesian3dRotationZ(7)]), Cartesian3dRotationX(-2.0)]),
+])
+def test_records_follow_the_content(make):
+    t = make()
+    assert _bytes(t) == _fresh(t) and _bytes(make()) == _fresh(t)
+    first = t.elements()[0]
+    if hasattr(first, "angle"):
+        first.angle = first.angle + 1.0
+    else:
+        first.x = -2.0
+    assert _bytes(t) == _fresh(t) != _fresh(make())
+
+
+def test_order_sign_of_zero_and_subclasses():
+    a, b = Cartesian3dRotationY(20.0), Cartesian3dTranslation(x=3.0)
+    assert _bytes(TransformationList([a, b])) != _bytes(TransformationList([b, a]))
+    for zero in (0.0, -0.0):
+        assert _bytes(Cartesian3dTranslation(x=zero)) == _fresh(Cartesian3dTranslation(x=zero))
+
+    class Shifted(Cartesian3dTranslation):
+        @property
+        def vector(self):
+            return np.array([9.0, 0.0, 0.0])
+
+    assert _bytes(Shifted(x=1.0)) == _fresh(Shifted(x=1.0)) != _bytes(Cartesian3dTranslation(x=1.0))
+    assert ctypes.sizeof(_compile._lib.Affine) == len(_bytes(None))
+
+
+def test_kept_records_are_bounded():
+    for i in range(_compile._AFFINES_MAX + 50):
+        _compile.affine_record(Cartesian3dTranslation(x=float(i)))
+    assert len(_compile._AFFINES) <= _compile._AFFINES_MAX
