@@ -384,6 +384,12 @@ int32_t optk_collect(const optk_collect_args *args, int64_t n, void *hip_stream)
 /* bytes of workspace the tiled binning of n rays needs (0: not applicable) */
 uint64_t optk_collect_workspace(const optk_collect_args *args, int64_t n);
 
+/* Flux-weighted mean cosine of n pixels, moment / image, and 1 where image is
+ * not above 0 (the second result of AbstractImagingSensor.collect).  float64
+ * device arrays; cosine may be the moment array itself. */
+int32_t optk_collect_cosine(const double *image, const double *moment, double *cosine, int64_t n,
+                            void *hip_stream);
+
 /* Sensor binning that allocates nothing.  No counterpart in the reference:
  * it is for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).

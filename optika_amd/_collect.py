@@ -46,7 +46,10 @@ def histogram(rays, wavelength_edges, x_range, y_range, num_x, num_y, where=None
     wl = full(rays.wavelength)
     inten = full(rays.intensity)
     u = rays.unvignetted
-    if isinstance(u, torch.Tensor) and u.ndim > 0:
+    if isinstance(u, torch.Tensor) and u.ndim > 0 and u.dtype == torch.bool:
+        # a bool is stored as the byte the kernels read
+        mask = u.reshape(-1).to(device=dev).contiguous().view(torch.uint8)
+    elif isinstance(u, torch.Tensor) and u.ndim > 0:
         mask = u.reshape(-1).to(device=dev, dtype=torch.uint8).contiguous()
     else:
         mask = torch.full((n,), 1 if bool(u) else 0, dtype=torch.uint8, device=dev)
@@ -94,9 +97,11 @@ def collect(sensor, rays, wavelength, where=True):
     hy = w.y * npx.y / 2
     image, moment = histogram(rays, wavelength, (-hx, hx), (-hy, hy), int(npx.x), int(npx.y),
                               where=None if (np.ndim(where) == 0 and bool(where)) else where)
-    cosine = torch.where(image > 0, moment / torch.where(image > 0, image, 1.0),
-                         torch.ones_like(image))
-    return image, cosine
+    # the moment's array becomes the cosine's
+    _lib.check(_lib.lib().optk_collect_cosine(image.data_ptr(), moment.data_ptr(),
+                                              moment.data_ptr(), image.numel(),
+                                              _trace.stream_handle()))
+    return image, moment
 
 
 def expose(image, scale: float, read_noise: float = 0.0, noise: bool = True, seed: int = 0):

@@ -334,6 +334,8 @@ def lib() -> ctypes.CDLL:
     L.optk_collect.argtypes = [ctypes.POINTER(CollectArgs), c_int64, c_void_p]
     L.optk_collect_workspace.restype = ctypes.c_uint64
     L.optk_collect_workspace.argtypes = [ctypes.POINTER(CollectArgs), c_int64]
+    L.optk_collect_cosine.restype = c_int32
+    L.optk_collect_cosine.argtypes = [c_void_p, c_void_p, c_void_p, c_int64, c_void_p]
     L.optk_collect_noalloc.restype = c_int32
     L.optk_collect_noalloc.argtypes = [ctypes.POINTER(CollectArgs), c_int64, c_void_p]
     L.optk_batch_create.restype = c_int32

@@ -1039,6 +1039,20 @@ __device__ __forceinline__ int linspace_bin(double x, double lo, double hi, int 
   return k;
 }
 
+// The same bin where the first guess needs no step, as it does but for points
+// within a rounding of an edge: two edges bracket the point, without the
+// walk's conversions and selects (three times the instructions, which had
+// bound the counting kernel).
+__device__ __forceinline__ int linspace_bin_near(double x, double lo, double hi, int num,
+                                                 double step, double inv) {
+  if (!(x >= lo) || !(x <= hi)) return -1;
+  const double k = floor((x - lo) * inv);
+  const double below = k * step + lo, above = (k + 1.0) * step + lo;
+  // (a last bin's `above` may differ from hi: a point short of it is in the bin)
+  if (k < (double)num && below <= x && x < above) return (int)k;
+  return linspace_bin(x, lo, hi, num, step, inv);
+}
+
 // The same bin by binary search over the edges formed as numpy forms them
 // (e_j = j * step + lo for j < num, e_num = hi; non-decreasing, since each
 // of the two roundings is monotone): the largest j < num with e_j <= x.
@@ -1073,35 +1087,44 @@ __device__ __forceinline__ int edges_bin(double x, const double *e, int num) {
 //   count:   block b bins the rays of its chunk once, stores each ray's key
 //            (tile << 10 | pixel in tile, -1 when not binned), counts the
 //            rays per tile in LDS and writes its row counts[b][*] (coalesced)
-//   offsets: one wavefront per tile scans the tile's column of block counts
-//            (in place: exclusive offsets) and leaves the tile's total
+//   offsets: scans each tile's column of block counts (in place: exclusive
+//            offsets) and leaves the tile's total
 //   base:    exclusive scan of the totals (one block)
 //   scatter: block b reads its chunk's keys and writes one record per ray at
-//            base[tile] + offsets[tile][b] + rank: with CT_CHUNK rays per
-//            block a tile receives runs of ~CT_CHUNK / tiles records, whole
+//            base[tile] + offsets[tile][b] + rank: with T.chunk rays per
+//            block a tile receives runs of ~chunk / tiles records, whole
 //            cache lines for a 2048^2 image
 //   tiles:   blocks sum a tile's rays with LDS float64 atomics and add its
 //            pixels to the image (one block per tile, or CT_SPLIT blocks and
 //            float64 atomics for a tile holding many rays)
-// Records: float32 rays pack (pixel, weight, cosine) into one 16-byte
-// store; float64 rays keep a 2-byte pixel array beside (weight, cosine).
-// The moment weight x cosine is formed in float64 in the tiles kernel, as
-// the one-pass kernel forms it.
+// Records: float32 rays pack (pixel, weight, cosine) into 12 bytes; float64
+// rays keep a 2-byte pixel array beside (weight, cosine).  The moment
+// weight x cosine is formed in float64 in the tiles kernel, as the one-pass
+// kernel forms it.
+//
+// Bound: memory.  A float32 ray costs 13 B in + 4 B out in count, 12 B in +
+// 12 B out in scatter and 12 B in tiles, 53 B in all.
 constexpr int CT_SIDE = 32;
 constexpr int CT_PIX = CT_SIDE * CT_SIDE;
 constexpr int CT_MAX_TILES = 16384;
-constexpr int64_t CT_CHUNK = 32768;  // rays per block in count / scatter
-constexpr int CT_THREADS = 1024;     // threads per count / scatter block
+// Rays per block in count / scatter: CT_BLOCKS blocks (two per CU) share the
+// rays evenly, within these limits.  Below CT_CHUNK_MIN the blocks' rows of
+// counts would outweigh their rays; above CT_CHUNK a block's runs per tile
+// are long enough.
+constexpr int64_t CT_CHUNK = 32768;
+constexpr int64_t CT_CHUNK_MIN = 4096;
+constexpr int64_t CT_BLOCKS = 512;
+constexpr int CT_THREADS = 1024;  // threads per count / scatter block
 
 struct RecordF32 {
-  uint32_t pix;
+  uint32_t key;  // pixel in tile in the low 10 bits
   float inten, dz;
-  uint32_t pad;
 };
+static_assert(sizeof(RecordF32) == 12, "three dwords a record");
 
 struct TiledParams {
   CollectParams C;
-  int32_t tiles_x, tiles_y, num_tiles, blocks;
+  int32_t tiles_x, tiles_y, num_tiles, blocks, chunk;
   int32_t *counts;      // [blocks][num_tiles], then exclusive offsets in place
   int32_t *base;        // [num_tiles + 1]
   int32_t *keys;        // [n] tile << 10 | pixel, -1 when not binned
@@ -1110,80 +1133,119 @@ struct TiledParams {
   RecordF32 *sorted32;  // float32 rays
 };
 
-constexpr int CT_UNROLL = 4;  // rays per thread per step of scatter / tiles
+constexpr int CT_UNROLL = 4;  // rays per thread per step of count / scatter / tiles
 
-// position, wavelength and mask of one ray, for the key
-struct BinIn {
-  double x, y, w;
-  bool live;
+// position, wavelength and mask of one ray as stored, for the key
+template <typename Real> struct BinIn {
+  Real x, y, w;
+  uint8_t live;
 };
 
-template <bool F32> __device__ __forceinline__ BinIn bin_load(const CollectParams &C, int64_t i) {
-  BinIn b;
-  b.live = !(C.unvignetted && !C.unvignetted[i]);
-  if (F32) {
-    b.x = C.pxf[i];
-    b.y = C.pyf[i];
-    b.w = C.wavelengthf[i];
-  } else {
-    b.x = C.px[i];
-    b.y = C.py[i];
-    b.w = C.wavelength[i];
-  }
-  return b;
-}
+template <bool F32> struct RayArrays;
+template <> struct RayArrays<true> {
+  typedef float Real;
+  static __device__ __forceinline__ const float *x(const CollectParams &C) { return C.pxf; }
+  static __device__ __forceinline__ const float *y(const CollectParams &C) { return C.pyf; }
+  static __device__ __forceinline__ const float *w(const CollectParams &C) { return C.wavelengthf; }
+  static __device__ __forceinline__ const float *inten(const CollectParams &C) { return C.intensityf; }
+  static __device__ __forceinline__ const float *dz(const CollectParams &C) { return C.dzf; }
+};
+template <> struct RayArrays<false> {
+  typedef double Real;
+  static __device__ __forceinline__ const double *x(const CollectParams &C) { return C.px; }
+  static __device__ __forceinline__ const double *y(const CollectParams &C) { return C.py; }
+  static __device__ __forceinline__ const double *w(const CollectParams &C) { return C.wavelength; }
+  static __device__ __forceinline__ const double *inten(const CollectParams &C) { return C.intensity; }
+  static __device__ __forceinline__ const double *dz(const CollectParams &C) { return C.dz; }
+};
 
 // tile << 10 | pixel in tile, or -1 when the ray is masked or outside
-__device__ __forceinline__ int32_t bin_key(const TiledParams &T, const BinIn &b) {
-  if (!b.live) return -1;
-  const int bw = edges_bin(b.w, T.C.wedges, T.C.nw);
-  const int bx = linspace_bin(b.x, T.C.x_lo, T.C.x_hi, T.C.nx, T.C.x_step, T.C.x_inv);
-  const int by = linspace_bin(b.y, T.C.y_lo, T.C.y_hi, T.C.ny, T.C.y_step, T.C.y_inv);
-  if (bw < 0 || bx < 0 || by < 0) return -1;
-  const int tile = (bw * T.tiles_x + bx / CT_SIDE) * T.tiles_y + by / CT_SIDE;
-  return (tile << 10) | ((bx % CT_SIDE) * CT_SIDE + by % CT_SIDE);
+__device__ __forceinline__ int32_t bin_key(const TiledParams &T, double w_lo, double w_hi, double x,
+                                           double y, double w, bool live) {
+  if (!live || !(w >= w_lo) || !(w <= w_hi)) return -1;
+  const int ix = linspace_bin_near(x, T.C.x_lo, T.C.x_hi, T.C.nx, T.C.x_step, T.C.x_inv);
+  const int iy = linspace_bin_near(y, T.C.y_lo, T.C.y_hi, T.C.ny, T.C.y_step, T.C.y_inv);
+  if (ix < 0 || iy < 0) return -1;
+  const uint32_t bw = T.C.nw == 1 ? 0 : edges_bin(w, T.C.wedges, T.C.nw);
+  const uint32_t bx = ix, by = iy;
+  const uint32_t tile = (bw * T.tiles_x + bx / CT_SIDE) * T.tiles_y + by / CT_SIDE;
+  return (int32_t)(tile << 10 | (bx % CT_SIDE) * CT_SIDE | by % CT_SIDE);
 }
 
 // count and scatter hold one 32-bit word per tile in dynamic LDS; both are
-// specialised by the rays' precision (one set of array pointers live)
+// specialised by the rays' precision (one set of array pointers live).
+// CT_UNROLL rays are loaded before any is binned, and the outer edges of the
+// wavelength bins once per block; the bound on the waves keeps two blocks on a
+// CU.  2^24 float32 rays: 62 us, 4.6 TB/s (one ray at a time with the edges
+// read again for each and every bin walked: 92 us; one block a CU: 85 us).
 template <bool F32>
-__global__ __launch_bounds__(CT_THREADS) void collect_count(const TiledParams T) {
+__global__ __launch_bounds__(CT_THREADS, 8) void collect_count(const TiledParams T) {
+  typedef RayArrays<F32> A;
+  typedef typename A::Real Real;
   extern __shared__ int32_t cnt[];
   for (int t = threadIdx.x; t < T.num_tiles; t += CT_THREADS) cnt[t] = 0;
+  const double w_lo = T.C.wedges[0], w_hi = T.C.wedges[T.C.nw];
   __syncthreads();
-  const int64_t lo = (int64_t)blockIdx.x * CT_CHUNK;
-  const int64_t hi = lo + CT_CHUNK < T.C.n ? lo + CT_CHUNK : T.C.n;
-  // one ray per thread per step (unrolling the binning's rare exact walks
-  // would exhaust the scalar registers that hold their exec masks)
-  for (int64_t i = lo + threadIdx.x; i < hi; i += CT_THREADS) {
-    const int32_t key = bin_key(T, bin_load<F32>(T.C, i));
-    if (key >= 0) atomicAdd(&cnt[key >> 10], 1);
-    T.keys[i] = key;
+  const int64_t lo = (int64_t)blockIdx.x * T.chunk;
+  const int m = (int)(lo + T.chunk < T.C.n ? T.chunk : T.C.n - lo);
+  const Real *px = A::x(T.C) + lo, *py = A::y(T.C) + lo, *pw = A::w(T.C) + lo;
+  const uint8_t *pl = T.C.unvignetted ? T.C.unvignetted + lo : nullptr;
+  int32_t *keys = T.keys + lo;
+  for (int i0 = threadIdx.x; i0 < m; i0 += CT_UNROLL * CT_THREADS) {
+    BinIn<Real> in[CT_UNROLL];
+#pragma unroll
+    for (int u = 0; u < CT_UNROLL; ++u) {
+      const int i = i0 + u * CT_THREADS;
+      const int k = i < m ? i : m - 1;
+      in[u].x = __builtin_nontemporal_load(px + k);
+      in[u].y = __builtin_nontemporal_load(py + k);
+      in[u].w = __builtin_nontemporal_load(pw + k);
+      in[u].live = pl ? __builtin_nontemporal_load(pl + k) : 1;  // (read once)
+    }
+#pragma unroll
+    for (int u = 0; u < CT_UNROLL; ++u) {
+      const int i = i0 + u * CT_THREADS;
+      if (i >= m) break;
+      const int32_t key = bin_key(T, w_lo, w_hi, in[u].x, in[u].y, in[u].w, in[u].live != 0);
+      if (key >= 0) atomicAdd(&cnt[key >> 10], 1);
+      keys[i] = key;
+    }
   }
   __syncthreads();
   for (int t = threadIdx.x; t < T.num_tiles; t += CT_THREADS)
     T.counts[(int64_t)blockIdx.x * T.num_tiles + t] = cnt[t];
 }
 
-__global__ __launch_bounds__(256) void collect_offsets(const TiledParams T) {
-  const int lane = threadIdx.x & 63;
-  const int t = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  if (t >= T.num_tiles) return;  // whole wavefronts
-  int32_t *col = T.counts + t;  // entry b at col[b * num_tiles]
+// Exclusive scan of each tile's column of block counts.  A block takes 64
+// tiles: lane = tile, so that every row is read and written as 256
+// consecutive bytes, and its 16 wavefronts share the rows (sums first, then
+// the offsets, the second reading out of L2).  A wavefront per tile had read
+// one word of each row's line: 28 us for 512 blocks and 4096 tiles, now 7.6.
+constexpr int CT_OFF_GROUPS = 16;
+__global__ __launch_bounds__(64 * CT_OFF_GROUPS) void collect_offsets(const TiledParams T) {
+  __shared__ int32_t part[CT_OFF_GROUPS][64];
+  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const int t = blockIdx.x * 64 + lane;
+  const bool in = t < T.num_tiles;
+  const int per = (T.blocks + CT_OFF_GROUPS - 1) / CT_OFF_GROUPS;
+  const int b0 = g * per < T.blocks ? g * per : T.blocks;
+  const int b1 = b0 + per < T.blocks ? b0 + per : T.blocks;
+  int32_t *col = T.counts + (in ? t : 0);
+  int32_t sum = 0;
+#pragma unroll 8
+  for (int b = b0; b < b1; ++b) sum += col[(int64_t)b * T.num_tiles];
+  part[g][lane] = sum;
+  __syncthreads();
   int32_t carry = 0;
-  for (int b0 = 0; b0 < T.blocks; b0 += 64) {
-    const int b = b0 + lane;
-    const int64_t k = (int64_t)b * T.num_tiles;
-    const int32_t c = b < T.blocks ? col[k] : 0;
-    int32_t incl = c;
-    for (int off = 1; off < 64; off <<= 1) {
-      const int32_t v = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += v;
-    }
-    if (b < T.blocks) col[k] = carry + incl - c;
-    carry += __shfl(incl, 63, 64);
+  for (int k = 0; k < g; ++k) carry += part[k][lane];
+  if (!in) return;
+  if (g == CT_OFF_GROUPS - 1) T.base[t] = carry + sum;  // the tile's total, scanned by collect_base
+#pragma unroll 8
+  for (int b = b0; b < b1; ++b) {
+    const int32_t c = col[(int64_t)b * T.num_tiles];
+    col[(int64_t)b * T.num_tiles] = carry;
+    carry += c;
   }
-  if (lane == 0) T.base[t] = carry;  // the tile's total, scanned by collect_base
 }
 
 __global__ __launch_bounds__(1024) void collect_base(const TiledParams T) {
@@ -1223,8 +1285,8 @@ __global__ __launch_bounds__(CT_THREADS) void collect_scatter(const TiledParams 
   for (int t = threadIdx.x; t < T.num_tiles; t += CT_THREADS)
     cursor[t] = T.base[t] + T.counts[(int64_t)blockIdx.x * T.num_tiles + t];
   __syncthreads();
-  const int64_t lo = (int64_t)blockIdx.x * CT_CHUNK;
-  const int64_t hi = lo + CT_CHUNK < T.C.n ? lo + CT_CHUNK : T.C.n;
+  const int64_t lo = (int64_t)blockIdx.x * T.chunk;
+  const int64_t hi = lo + T.chunk < T.C.n ? lo + T.chunk : T.C.n;
   for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += CT_UNROLL * CT_THREADS) {
     int32_t key[CT_UNROLL];
     double a[CT_UNROLL], c[CT_UNROLL];
@@ -1244,7 +1306,7 @@ __global__ __launch_bounds__(CT_THREADS) void collect_scatter(const TiledParams 
       if (key[u] < 0) continue;
       const int32_t slot = atomicAdd(&cursor[key[u] >> 10], 1);
       if (F32) {
-        T.sorted32[slot] = RecordF32{(uint32_t)(key[u] & 1023), (float)a[u], (float)c[u], 0u};
+        T.sorted32[slot] = RecordF32{(uint32_t)key[u], (float)a[u], (float)c[u]};
       } else {
         T.sorted_pix[slot] = (uint16_t)(key[u] & 1023);
         T.sorted_ab[slot] = double2{a[u], c[u]};
@@ -1254,74 +1316,90 @@ __global__ __launch_bounds__(CT_THREADS) void collect_scatter(const TiledParams 
 }
 
 // Images of at most CT_STAGED_TILES tiles: the scatter stages each
-// sub-chunk of CT_SUB rays in LDS in tile order (a local counting sort) and
+// sub-chunk of rays in LDS in tile order (a local counting sort) and
 // then writes it out, so that one tile's records leave the block as
 // consecutive stores, whole cache lines, instead of one scattered store per
-// ray that concurrent blocks complete piecewise.  Float32 rays stage their
-// 16-byte records; float64 rays stage (weight, cosine) and the 2-byte pixel.
-//   1. zero the local counts            2. load, rank within the tile (LDS atomic)
-//   3. scan the counts (local offsets)  4. place records and global slots in LDS
-//   5. write out in local order, advance the tiles' cursors
-constexpr int CT_SUB = CT_UNROLL * CT_THREADS;  // rays per sub-chunk
-constexpr int CT_STAGED_TILES = 4096;
+// ray that concurrent blocks complete piecewise.  A staged record keeps its
+// key, from whose tile the writing thread finds the record's place.
+//   1. rank each ray within its tile (LDS atomic on the local counts)
+//   2. scan the counts: local offsets, and where each tile's run goes
+//   3. place the records in LDS, load the next sub-chunk's rays
+//   4. write out in local order, clear the counts
+// Thread t owns tiles 4 t .. 4 t + 3 and keeps their next global slots in
+// registers; the local counts are 16 bits, two to a word.  With 6 bytes a
+// tile the sub-chunk fills the rest of the CU's LDS, one block to a CU: the
+// two ends of every (tile, sub-chunk) run are partly written cache lines,
+// and with runs too short or too many of them open at once they leave the
+// L2 before the next run completes them (2^24 float32 rays on a 361-tile
+// spot, a sub-chunk of 4096 rays and two blocks a CU: 118 us, half as many
+// writes again and the lines read back in; 8192 rays and one block: 86 us,
+// 4.7 TB/s; the earlier 4096 rays with 16-byte records and three words a
+// tile: 144 us).
+constexpr int CT_OWN = 4;  // tiles per thread
+constexpr int CT_STAGED_TILES = CT_OWN * CT_THREADS;
 
 template <bool F32> struct StageRecord;
 template <> struct StageRecord<true> {
-  RecordF32 r;
+  static constexpr int RAYS = 8;  // per thread and sub-chunk
+  RecordF32 r[RAYS * CT_THREADS];
 };
 template <> struct StageRecord<false> {
-  double2 ab;
+  static constexpr int RAYS = 6;
+  double2 ab[RAYS * CT_THREADS];
+  int32_t key[RAYS * CT_THREADS];
 };
 
 template <bool F32>
-__global__ __launch_bounds__(CT_THREADS) void collect_scatter_staged(const TiledParams T) {
-  extern __shared__ int32_t dyn[];
-  int32_t *cursor = dyn;                    // [num_tiles] next global slot of each tile
-  int32_t *loff = dyn + T.num_tiles;        // [num_tiles] local counts, then local offsets
-  int32_t *lcnt = dyn + 2 * T.num_tiles;    // [num_tiles] local counts of the pass
-  __shared__ StageRecord<F32> stage[CT_SUB];
-  __shared__ uint16_t stage_pix[F32 ? 1 : CT_SUB];
-  __shared__ int32_t dest[CT_SUB];
+__global__ __launch_bounds__(CT_THREADS, 4) void collect_scatter_staged(const TiledParams T) {
+  typedef RayArrays<F32> A;
+  typedef typename A::Real Real;
+  constexpr int RAYS = StageRecord<F32>::RAYS, SUB = RAYS * CT_THREADS;
+  static_assert(SUB < 65536, "local counts and offsets of 16 bits");
+  __shared__ int4 place[CT_STAGED_TILES / CT_OWN];   // global slot of a tile's local record 0
+  __shared__ uint2 local[CT_STAGED_TILES / CT_OWN];  // local counts, then local offsets
+  __shared__ StageRecord<F32> stage;
   __shared__ int32_t wsum[CT_THREADS / 64];
-  __shared__ int32_t total;
+  int32_t *const slot0 = (int32_t *)place;
+  uint32_t *const packed = (uint32_t *)local;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int per = (T.num_tiles + CT_THREADS - 1) / CT_THREADS;  // tiles scanned per thread
-  const int t0 = tid * per;
-  for (int t = tid; t < T.num_tiles; t += CT_THREADS)
-    cursor[t] = T.base[t] + T.counts[(int64_t)blockIdx.x * T.num_tiles + t];
-  const int64_t lo = (int64_t)blockIdx.x * CT_CHUNK;
-  const int64_t hi = lo + CT_CHUNK < T.C.n ? lo + CT_CHUNK : T.C.n;
-  for (int64_t s0 = lo; s0 < hi; s0 += CT_SUB) {
-    for (int t = tid; t < T.num_tiles; t += CT_THREADS) loff[t] = 0;
-    __syncthreads();
-    typedef typename std::conditional<F32, float, double>::type Real;
-    int32_t key[CT_UNROLL], rank[CT_UNROLL];
-    Real a[CT_UNROLL], c[CT_UNROLL];
+  int32_t next[CT_OWN];  // next global slot of the thread's tiles
 #pragma unroll
-    for (int u = 0; u < CT_UNROLL; ++u) {
-      const int64_t i = s0 + (int64_t)u * CT_THREADS + tid;
-      key[u] = -1;
-      a[u] = c[u] = Real(0);
-      if (i < hi) {
-        key[u] = T.keys[i];
-        if constexpr (F32) {
-          a[u] = T.C.intensityf[i];
-          c[u] = T.C.dzf[i];
-        } else {
-          a[u] = T.C.intensity[i];
-          c[u] = T.C.dz[i];
-        }
-      }
-    }
+  for (int j = 0; j < CT_OWN; ++j) {
+    const int t = CT_OWN * tid + j;
+    next[j] = t < T.num_tiles ? T.base[t] + T.counts[(int64_t)blockIdx.x * T.num_tiles + t] : 0;
+  }
+  local[tid] = uint2{0u, 0u};
+  const int64_t lo = (int64_t)blockIdx.x * T.chunk;
+  const int m = (int)(lo + T.chunk < T.C.n ? T.chunk : T.C.n - lo);
+  const int32_t *keys = T.keys + lo;
+  const Real *pa = A::inten(T.C) + lo, *pc = A::dz(T.C) + lo;
+  int32_t key[RAYS];
+  Real a[RAYS], c[RAYS];
+  auto load = [&](int s0) {
 #pragma unroll
-    for (int u = 0; u < CT_UNROLL; ++u) rank[u] = key[u] >= 0 ? atomicAdd(&loff[key[u] >> 10], 1) : 0;
-    __syncthreads();
-    // exclusive scan of loff: per-thread runs of `per` tiles, wave scan, scan of the wave sums
-    int32_t sum = 0;
-    for (int j = 0; j < per; ++j) {
-      const int t = t0 + j;
-      if (t < T.num_tiles) sum += loff[t];
+    for (int u = 0; u < RAYS; ++u) {
+      const int i = s0 + u * CT_THREADS + tid;
+      const int k = i < m ? i : m - 1;
+      key[u] = i < m ? __builtin_nontemporal_load(keys + k) : -1;
+      a[u] = __builtin_nontemporal_load(pa + k);
+      c[u] = __builtin_nontemporal_load(pc + k);
     }
+  };
+  load(0);
+  __syncthreads();
+  for (int s0 = 0; s0 < m; s0 += SUB) {
+    uint32_t rank[RAYS];
+#pragma unroll
+    for (int u = 0; u < RAYS; ++u) {
+      const int sh = (key[u] >> 10 & 1) * 16;
+      rank[u] = key[u] >= 0 ? atomicAdd(&packed[key[u] >> 11], 1u << sh) >> sh & 0xffffu : 0u;
+    }
+    __syncthreads();
+    // exclusive scan of the counts: the thread's four, a wave scan, the wave sums
+    const uint2 pk = local[tid];
+    const int32_t cnt[CT_OWN] = {(int32_t)(pk.x & 0xffffu), (int32_t)(pk.x >> 16),
+                                 (int32_t)(pk.y & 0xffffu), (int32_t)(pk.y >> 16)};
+    const int32_t sum = cnt[0] + cnt[1] + cnt[2] + cnt[3];
     int32_t incl = sum;
     for (int off = 1; off < 64; off <<= 1) {
       const int32_t v = __shfl_up(incl, off, 64);
@@ -1329,55 +1407,51 @@ __global__ __launch_bounds__(CT_THREADS) void collect_scatter_staged(const Tiled
     }
     if (lane == 63) wsum[wave] = incl;
     __syncthreads();
-    if (wave == 0) {
-      const int32_t w = lane < CT_THREADS / 64 ? wsum[lane] : 0;
-      int32_t wi = w;
-      for (int off = 1; off < 64; off <<= 1) {
-        const int32_t v = __shfl_up(wi, off, 64);
-        if (lane >= off) wi += v;
-      }
-      if (lane < CT_THREADS / 64) wsum[lane] = wi - w;
-      if (lane == 63) total = wi;
+    int32_t run = incl - sum, n_sub = 0;
+#pragma unroll
+    for (int w = 0; w < CT_THREADS / 64; ++w) {
+      const int32_t v = wsum[w];
+      if (w < wave) run += v;
+      n_sub += v;
     }
-    __syncthreads();
-    int32_t run = wsum[wave] + incl - sum;
-    for (int j = 0; j < per; ++j) {
-      const int t = t0 + j;
-      if (t < T.num_tiles) {
-        const int32_t cnt = loff[t];
-        lcnt[t] = cnt;
-        loff[t] = run;
-        run += cnt;
-      }
+    int32_t off[CT_OWN], at[CT_OWN];
+#pragma unroll
+    for (int j = 0; j < CT_OWN; ++j) {
+      off[j] = run;
+      at[j] = next[j] - run;
+      next[j] += cnt[j];
+      run += cnt[j];
     }
+    local[tid] = uint2{(uint32_t)off[0] | (uint32_t)off[1] << 16,
+                       (uint32_t)off[2] | (uint32_t)off[3] << 16};
+    place[tid] = int4{at[0], at[1], at[2], at[3]};
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < CT_UNROLL; ++u) {
+    for (int u = 0; u < RAYS; ++u) {
       if (key[u] < 0) continue;
-      const int tile = key[u] >> 10;
-      const int32_t p = loff[tile] + rank[u];
+      const uint32_t p = (packed[key[u] >> 11] >> (key[u] >> 10 & 1) * 16 & 0xffffu) + rank[u];
       if constexpr (F32) {
-        stage[p].r = RecordF32{(uint32_t)(key[u] & 1023), a[u], c[u], 0u};
+        stage.r[p] = RecordF32{(uint32_t)key[u], a[u], c[u]};
       } else {
-        stage[p].ab = double2{a[u], c[u]};
-        stage_pix[p] = (uint16_t)(key[u] & 1023);
+        stage.ab[p] = double2{a[u], c[u]};
+        stage.key[p] = key[u];
       }
-      dest[p] = cursor[tile] + rank[u];
     }
+    if (s0 + SUB < m) load(s0 + SUB);
     __syncthreads();
-    const int32_t n_sub = total;
+    local[tid] = uint2{0u, 0u};
     for (int32_t p = tid; p < n_sub; p += CT_THREADS) {
       if constexpr (F32) {
-        T.sorted32[dest[p]] = stage[p].r;
+        const RecordF32 r = stage.r[p];
+        T.sorted32[slot0[r.key >> 10] + p] = r;
       } else {
-        T.sorted_ab[dest[p]] = stage[p].ab;
-        T.sorted_pix[dest[p]] = stage_pix[p];
+        const int32_t k = stage.key[p];
+        const int32_t slot = slot0[k >> 10] + p;
+        T.sorted_ab[slot] = stage.ab[p];
+        T.sorted_pix[slot] = (uint16_t)(k & 1023);
       }
     }
-    for (int j = 0; j < per; ++j) {
-      const int t = t0 + j;
-      if (t < T.num_tiles) cursor[t] += lcnt[t];
-    }
+    __syncthreads();
   }
 }
 
@@ -1418,7 +1492,7 @@ __global__ __launch_bounds__(256) void collect_tiles(const TiledParams T) {
       if (j < hi) {
         if (F32) {
           const RecordF32 r = T.sorted32[j];
-          pix[u] = (int)r.pix;
+          pix[u] = (int)(r.key & 1023u);
           a[u] = r.inten;
           c[u] = r.dz;
         } else {
@@ -1454,6 +1528,17 @@ __global__ __launch_bounds__(256) void collect_tiles(const TiledParams T) {
       T.C.moment[k] += acc_b[p];
     }
   }
+}
+
+// Flux-weighted mean cosine of each pixel, 1 where no flux arrived.  Bound by
+// its 24 bytes a pixel: 16 us for 2048^2; as comparisons, selects and a
+// division of whole images, 65 us.
+__global__ __launch_bounds__(256) void collect_cosine(const double *image, const double *moment,
+                                                      double *cosine, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double w = image[i], m = moment[i];
+  cosine[i] = w > 0.0 ? m / w : 1.0;
 }
 
 // One ray per thread.  Rays of a wavefront that land in the same bin are
@@ -2083,40 +2168,77 @@ int32_t optk_expose(const optk_expose_args *args, int64_t n, void *hip_stream) {
 }
 
 
-// Workspace of the tiled binning (sections 256-byte aligned); fills T's
-// pointers when ws is given.  0 when the image has too many tiles or the
-// rays are too many for 32-bit slots.
-static uint64_t tiled_layout(int nw, int nx, int ny, int64_t n, bool f32, void *ws,
-                             TiledParams *T) {
-  const int64_t tx = (nx + CT_SIDE - 1) / CT_SIDE, ty = (ny + CT_SIDE - 1) / CT_SIDE;
-  const int64_t tiles = (int64_t)nw * tx * ty;
-  if (tiles > CT_MAX_TILES || n <= 0 || n > INT32_MAX) return 0;
-  const int64_t blocks = (n + CT_CHUNK - 1) / CT_CHUNK;
+// Workspace of the tiled binning (sections 256-byte aligned) with `chunk`
+// rays a block and `record` bytes a sorted ray.
+static uint64_t tiled_bytes(int64_t tiles, int64_t chunk, int64_t n, bool f32, uint64_t record) {
+  const int64_t blocks = (n + chunk - 1) / chunk;
   auto up = [](uint64_t b) { return (b + 255) & ~(uint64_t)255; };
-  const uint64_t s_counts = up((uint64_t)blocks * tiles * 4);
-  const uint64_t s_base = up((uint64_t)(tiles + 1) * 4);
-  const uint64_t s_keys = up((uint64_t)n * 4);
-  const uint64_t s_pix = f32 ? 0 : up((uint64_t)n * 2);
-  const uint64_t s_val = up((uint64_t)n * 16);
-  const uint64_t total = s_counts + s_base + s_keys + s_pix + s_val;
-  if (T) {
-    T->tiles_x = (int32_t)tx;
-    T->tiles_y = (int32_t)ty;
-    T->num_tiles = (int32_t)tiles;
-    T->blocks = (int32_t)blocks;
-    char *p = (char *)ws;
-    T->counts = (int32_t *)p;
-    p += s_counts;
-    T->base = (int32_t *)p;
-    p += s_base;
-    T->keys = (int32_t *)p;
-    p += s_keys;
-    T->sorted_pix = f32 ? nullptr : (uint16_t *)p;
-    p += s_pix;
-    T->sorted_ab = f32 ? nullptr : (double2 *)p;
-    T->sorted32 = f32 ? (RecordF32 *)p : nullptr;
-  }
-  return total;
+  return up((uint64_t)blocks * tiles * 4) + up((uint64_t)(tiles + 1) * 4) + up((uint64_t)n * 4) +
+         (f32 ? 0 : up((uint64_t)n * 2)) + up((uint64_t)n * record);
+}
+
+// tiles of an image; 0 when they are too many for the tiled binning, or the
+// rays too many for 32-bit slots
+static int64_t tile_count(int nw, int nx, int ny, int64_t n) {
+  const int64_t tiles = (int64_t)nw * ((nx + CT_SIDE - 1) / CT_SIDE) * ((ny + CT_SIDE - 1) / CT_SIDE);
+  return tiles > CT_MAX_TILES || n <= 0 || n > INT32_MAX ? 0 : tiles;
+}
+
+// rays per block of the count and scatter kernels where workspace is no limit
+static int64_t preferred_chunk(int64_t n) {
+  const int64_t c = (n + CT_BLOCKS - 1) / CT_BLOCKS;
+  const int64_t even = (c + CT_THREADS - 1) / CT_THREADS * CT_THREADS;
+  return even < CT_CHUNK_MIN ? CT_CHUNK_MIN : (even > CT_CHUNK ? CT_CHUNK : even);
+}
+
+// Bytes of the smallest workspace the tiled binning is offered (0: not
+// applicable): blocks of CT_CHUNK rays and 16 bytes a record.
+static uint64_t tiled_least(int nw, int nx, int ny, int64_t n, bool f32) {
+  const int64_t tiles = tile_count(nw, nx, ny, n);
+  return tiles ? tiled_bytes(tiles, CT_CHUNK, n, f32, 16) : 0;
+}
+
+// Bytes of workspace optk_collect_workspace() asks for: room for the
+// preferred chunk, but no more than the library's own scratch where the
+// smallest layout fits that.
+static uint64_t tiled_wanted(int nw, int nx, int ny, int64_t n, bool f32) {
+  const uint64_t least = tiled_least(nw, nx, ny, n, f32);
+  if (!least) return 0;
+  uint64_t want = tiled_bytes(tile_count(nw, nx, ny, n), preferred_chunk(n), n, f32, f32 ? 12 : 16);
+  if (least <= OPTK_COLLECT_SCRATCH_BYTES && want > OPTK_COLLECT_SCRATCH_BYTES)
+    want = OPTK_COLLECT_SCRATCH_BYTES;
+  return want > least ? want : least;
+}
+
+// Lays the tiled binning's arrays out in ws with the smallest chunk from the
+// preferred one up that fits; false if ws is too small for it.
+static bool tiled_layout(int nw, int nx, int ny, int64_t n, bool f32, void *ws, uint64_t ws_bytes,
+                         TiledParams *T) {
+  const uint64_t least = tiled_least(nw, nx, ny, n, f32);
+  if (!least || !ws || ws_bytes < least) return false;
+  const int64_t tiles = tile_count(nw, nx, ny, n);
+  const uint64_t record = f32 ? sizeof(RecordF32) : sizeof(double2);
+  int64_t chunk = preferred_chunk(n);
+  while (chunk < CT_CHUNK && tiled_bytes(tiles, chunk, n, f32, record) > ws_bytes)
+    chunk = 2 * chunk < CT_CHUNK ? 2 * chunk : CT_CHUNK;
+  T->tiles_x = (int32_t)((nx + CT_SIDE - 1) / CT_SIDE);
+  T->tiles_y = (int32_t)((ny + CT_SIDE - 1) / CT_SIDE);
+  T->num_tiles = (int32_t)tiles;
+  T->chunk = (int32_t)chunk;
+  T->blocks = (int32_t)((n + chunk - 1) / chunk);
+  auto up = [](uint64_t b) { return (b + 255) & ~(uint64_t)255; };
+  char *p = (char *)ws;
+  T->counts = (int32_t *)p;
+  p += up((uint64_t)T->blocks * tiles * 4);
+  T->base = (int32_t *)p;
+  p += up((uint64_t)(tiles + 1) * 4);
+  T->keys = (int32_t *)p;
+  p += up((uint64_t)n * 4);
+  T->sorted_pix = f32 ? nullptr : (uint16_t *)p;
+  p += f32 ? 0 : up((uint64_t)n * 2);
+  T->sorted_ab = f32 ? nullptr : (double2 *)p;
+  T->sorted32 = f32 ? (RecordF32 *)p : nullptr;
+  return true;
 }
 
 }  // extern "C"
@@ -2189,8 +2311,8 @@ static int32_t collect_launch(const optk_collect_args *a, int64_t n, void *ws, u
     return OPTK_OK;
   }
   TiledParams T;
-  const uint64_t need = tiled_layout(a->n_wavelength, a->nx, a->ny, n, f32, ws, &T);
-  if (need == 0 || !ws || ws_bytes < need) {
+  std::memset(&T, 0, sizeof(T));
+  if (!tiled_layout(a->n_wavelength, a->nx, a->ny, n, f32, ws, ws_bytes, &T)) {
     hipLaunchKernelGGL(collect_kernel<false>, grid_for(n), dim3(256), 0, s, C);
     OPTK_HIP_CHECK(hipGetLastError());
     return OPTK_OK;
@@ -2201,16 +2323,17 @@ static int32_t collect_launch(const optk_collect_args *a, int64_t n, void *ws, u
     hipLaunchKernelGGL(collect_count<true>, dim3((unsigned)T.blocks), dim3(CT_THREADS), lds, s, T);
   else
     hipLaunchKernelGGL(collect_count<false>, dim3((unsigned)T.blocks), dim3(CT_THREADS), lds, s, T);
-  hipLaunchKernelGGL(collect_offsets, dim3((unsigned)((T.num_tiles + 3) / 4)), dim3(256), 0, s, T);
+  hipLaunchKernelGGL(collect_offsets, dim3((unsigned)((T.num_tiles + 63) / 64)), dim3(64 * CT_OFF_GROUPS), 0,
+                     s, T);
   hipLaunchKernelGGL(collect_base, dim3(1), dim3(1024), 0, s, T);
   if (T.num_tiles <= CT_STAGED_TILES) {
     if (f32) {
       hipLaunchKernelGGL(collect_scatter_staged<true>, dim3((unsigned)T.blocks), dim3(CT_THREADS),
-                         3 * lds, s, T);
+                         0, s, T);
       hipLaunchKernelGGL(collect_tiles<true>, dim3((unsigned)(T.num_tiles * CT_SPLIT)), dim3(256), 0, s, T);
     } else {
       hipLaunchKernelGGL(collect_scatter_staged<false>, dim3((unsigned)T.blocks), dim3(CT_THREADS),
-                         3 * lds, s, T);
+                         0, s, T);
       hipLaunchKernelGGL(collect_tiles<false>, dim3((unsigned)(T.num_tiles * CT_SPLIT)), dim3(256), 0, s, T);
     }
   } else if (f32) {
@@ -2272,8 +2395,7 @@ int32_t optk_collect_noalloc(const optk_collect_args *a, int64_t n, void *hip_st
     // tiled workspace exceeds the scratch
     if (n > INT32_MAX)
       return fail(OPTK_EINVAL, "optk_collect_noalloc: at most 2^31 - 1 rays per call");
-    need = tiled_layout(a->n_wavelength, a->nx, a->ny, n, a->precision == OPTK_F32, nullptr,
-                        nullptr);
+    need = tiled_least(a->n_wavelength, a->nx, a->ny, n, a->precision == OPTK_F32);
     if (need > OPTK_COLLECT_SCRATCH_BYTES)
       return fail(OPTK_EINVAL,
                   "optk_collect_noalloc: " + std::to_string(n) + " rays need " +
@@ -2287,12 +2409,23 @@ int32_t optk_collect_noalloc(const optk_collect_args *a, int64_t n, void *hip_st
     const int32_t rc = scratch_address(&ws);
     if (rc) return rc;
   }
-  return collect_launch(a, n, ws, need, hip_stream);
+  return collect_launch(a, n, ws, need ? OPTK_COLLECT_SCRATCH_BYTES : 0, hip_stream);
+}
+
+int32_t optk_collect_cosine(const double *image, const double *moment, double *cosine, int64_t n,
+                            void *hip_stream) {
+  if (n < 0) return fail(OPTK_EINVAL, "negative count");
+  if (!image || !moment || !cosine) return fail(OPTK_EINVAL, "missing image");
+  if (n == 0) return OPTK_OK;
+  hipLaunchKernelGGL(collect_cosine, grid_for(n), dim3(256), 0, (hipStream_t)hip_stream, image,
+                     moment, cosine, n);
+  OPTK_HIP_CHECK(hipGetLastError());
+  return OPTK_OK;
 }
 
 uint64_t optk_collect_workspace(const optk_collect_args *a, int64_t n) {
   if (!a || n <= 0 || a->n_wavelength < 1 || a->nx < 1 || a->ny < 1) return 0;
-  return tiled_layout(a->n_wavelength, a->nx, a->ny, n, a->precision == OPTK_F32, nullptr, nullptr);
+  return tiled_wanted(a->n_wavelength, a->nx, a->ny, n, a->precision == OPTK_F32);
 }
 
 }  // extern "C"
