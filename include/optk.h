@@ -570,6 +570,38 @@ int32_t optk_gemm_bf16_silu_back_sums(int64_t m, const void *a, int64_t lda, con
                                       const float *pre, int64_t ldc, float *c, void *out16, float *sums,
                                       float *workspace, void *hip_stream);
 
+/* Forward pass, weighted mean-square loss and backward pass of the 5 -> 4 x
+ * 256 SiLU -> 3 network over `rows` rows (a multiple of 64), down to what the
+ * hidden layers' weight gradients are the products of: act[l] holds the
+ * outputs of layer l and dpre[l] the gradient at the pre-activations of layer
+ * l + 1, bf16 [rows][256], so that gW of layer l + 1 is dpre[l]^T act[l].
+ * The other gradients are written to grad (float32, laid out as the
+ * parameters p: layer by layer, weights [out][in] then bias; the hidden
+ * layers' weights are left alone).
+ *   y [rows][3] = network(x [rows][5]);
+ *   loss = sum_r sum_j weight[j] (y - target)^2 / rows (one float32)
+ * p16: the parameters in bf16 (hidden layers used); wt16[l]: the weights of
+ * hidden layer l + 1 transposed, bf16 [in][out].  workspace: rows / 64 * 3076
+ * floats.  bf16 arrays 16-byte aligned. */
+typedef struct optk_train_args {
+  const float *x;
+  const float *target;
+  const float *weight;
+  const float *p;
+  const uint16_t *p16;
+  const uint16_t *wt16[3];
+  uint16_t *act[3];
+  uint16_t *dpre[3];
+  float *y;
+  float *grad;
+  float *loss;
+  float *workspace;
+  int64_t workspace_count;
+  int64_t rows;
+} optk_train_args;
+
+int32_t optk_train_pass(const optk_train_args *args, void *hip_stream);
+
 /* elementwise and small-layer pieces of the forward and backward passes
  * (argument use per op below; rows x cols row-major arrays) */
 enum {

@@ -198,6 +198,17 @@ class Tune(ctypes.Structure):
                 ("pad", c_int32), ("ms", c_double)]
 
 
+class TrainArgs(ctypes.Structure):
+    """optk_train_args."""
+
+    _fields_ = [
+        ("x", c_void_p), ("target", c_void_p), ("weight", c_void_p), ("p", c_void_p),
+        ("p16", c_void_p), ("wt16", c_void_p * 3), ("act", c_void_p * 3), ("dpre", c_void_p * 3),
+        ("y", c_void_p), ("grad", c_void_p), ("loss", c_void_p), ("workspace", c_void_p),
+        ("workspace_count", c_int64), ("rows", c_int64),
+    ]
+
+
 class MlpArgs(ctypes.Structure):
     _fields_ = [("f32", c_void_p * 8), ("u16", c_void_p * 4), ("rows", c_int64), ("count", c_int64),
                 ("cols", c_int32), ("inner", c_int32), ("flag", c_int32), ("pad", c_int32),
@@ -334,6 +345,8 @@ def lib() -> ctypes.CDLL:
     L.optk_collect.argtypes = [ctypes.POINTER(CollectArgs), c_int64, c_void_p]
     L.optk_collect_workspace.restype = ctypes.c_uint64
     L.optk_collect_workspace.argtypes = [ctypes.POINTER(CollectArgs), c_int64]
+    L.optk_train_pass.restype = c_int32
+    L.optk_train_pass.argtypes = [ctypes.POINTER(TrainArgs), c_void_p]
     L.optk_collect_cosine.restype = c_int32
     L.optk_collect_cosine.argtypes = [c_void_p, c_void_p, c_void_p, c_int64, c_void_p]
     L.optk_collect_noalloc.restype = c_int32

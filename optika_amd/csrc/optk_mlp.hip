@@ -522,6 +522,366 @@ __global__ __launch_bounds__(256) void transpose16(const uint16_t *__restrict__ 
 }
 
 // ---------------------------------------------------------------------------
+// The network's training pass over one 64-row tile: forward, loss, and the
+// backward products down to the first layer, in one kernel.
+//
+// As separate kernels the pass moved each layer's float32 pre-activations
+// (67 MB at 65,536 rows) to memory and back, read every activation and
+// gradient again for the next product, and took 25 launches, 340 us of a
+// 470 us step at 65,536 rows; this kernel takes 173 us there, and the sums
+// over its tiles 6.  Here a tile's activations and gradients pass from layer to
+// layer through LDS, and the SiLU derivatives of the three lower layers (as
+// float32, 96 registers a lane) wait in registers for the way back; memory
+// sees what the weight gradients' products read: three layers' activations
+// and three layers' gradients, 3 KB a row.
+//  - eight wavefronts of 32 columns each, two to a SIMD with up to 256
+//    registers; lane (fr, g) holds columns col, col + 1 (col = 32 wave +
+//    2 fr) of rows 16 mt + 4 g + q, so that its weights' rows are its
+//    columns, k contiguous;
+//  - a layer's weights (128 KB, L2-resident) stream through a register ring
+//    three 32-wide k chunks ahead, the first three requested before the
+//    elementwise work of the layer before;
+//  - the products sum the same 32-wide k chunks in the same order as
+//    gemm_panel; sums over rows leave one partial per tile, added up by
+//    train_reduce in a fixed order.
+// Bound: latency.  Its 51 GFLOP and 200 MB would take 40 us; the wavefronts
+// of the one block a CU holds go through products and elementwise work in
+// step, and only two are there to cover each other's waits.
+// ---------------------------------------------------------------------------
+
+constexpr int TT_ROWS = 64, TT_THREADS = 512, TT_IN = 5, TT_OUT = 3;
+// a tile's partial sums: first layer's weights and bias, the hidden layers'
+// biases, the last layer's weights and bias, the loss
+constexpr int TT_B0 = PK * TT_IN, TT_B1 = TT_B0 + PK, TT_B2 = TT_B1 + PK, TT_B3 = TT_B2 + PK,
+              TT_W4 = TT_B3 + PK, TT_B4 = TT_W4 + PK * TT_OUT, TT_LOSS = TT_B4 + TT_OUT,
+              TT_SUMS = TT_LOSS + 1;
+// the same in the flat parameter vector (layer by layer, weights then bias)
+constexpr int TP_W1 = TT_B0 + PK, TP_B1 = TP_W1 + PK * PK, TP_W2 = TP_B1 + PK, TP_B2 = TP_W2 + PK * PK,
+              TP_W3 = TP_B2 + PK, TP_B3 = TP_W3 + PK * PK, TP_W4 = TP_B3 + PK,
+              TP_B4 = TP_W4 + PK * TT_OUT;
+
+__global__ __launch_bounds__(TT_THREADS, 2) void train_tile(const optk_train_args T) {
+  __shared__ __attribute__((aligned(16))) PanelRow A[2][TT_ROWS];
+  __shared__ __attribute__((aligned(16))) float w4[TT_OUT * PK];
+  __shared__ __attribute__((aligned(16))) float4 dys[TT_ROWS];
+  __shared__ float xs[TT_ROWS * TT_IN];
+  __shared__ float red[TT_THREADS / 64][TT_OUT + 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int fr = lane & 15, g = lane >> 4, fk = 8 * g;
+  const int col = 32 * wave + 2 * fr;
+  const int64_t row0 = (int64_t)blockIdx.x * TT_ROWS;
+  float *sums = T.workspace + (int64_t)blockIdx.x * TT_SUMS;
+
+  // keeps the scheduler from mixing the stages of a layer, or more than two
+  // rows' elements, which would need more registers than there are
+  auto stage = [](int e) {
+    if (e % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr int AHEAD = 3;  // k chunks of weights requested before their product
+  uint4 b[AHEAD + 1][2];
+  const uint16_t *br;
+  auto request = [&](int c) {
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+      b[c % (AHEAD + 1)][nt] = *reinterpret_cast<const uint4 *>(br + nt * PK + 32 * c);
+  };
+  auto weights = [&](const uint16_t *bt) {
+    br = bt + (int64_t)col * PK + fk;
+#pragma unroll
+    for (int c = 0; c < AHEAD; ++c) request(c);
+  };
+  floatx4 acc[4][2];
+  auto product = [&](const PanelRow *a) {
+#pragma unroll
+    for (int c = 0; c < PK / 32; ++c) {
+      stage(0);
+      if (c + AHEAD < PK / 32) request(c + AHEAD);
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) {
+        const bf16x8 av = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(&a[16 * mt + fr][32 * c + fk]));
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              av, __builtin_bit_cast(bf16x8, b[c % (AHEAD + 1)][nt]),
+              c == 0 ? floatx4{0.0f, 0.0f, 0.0f, 0.0f} : acc[mt][nt], 0, 0, 0);
+      }
+    }
+  };
+  // a layer's rows out of LDS, 16 bytes a thread, whole rows of 512 bytes
+  auto copy_out = [&](const PanelRow *a, uint16_t *out) {
+#pragma unroll
+    for (int j = 0; j < TT_ROWS * PK / 8 / TT_THREADS; ++j) {
+      const int seg = tid + TT_THREADS * j, r = seg >> 5, s = seg & 31;
+      *reinterpret_cast<uint4 *>(out + (row0 + r) * PK + 8 * s) = *reinterpret_cast<const uint4 *>(&a[r][8 * s]);
+    }
+  };
+  // sum over the tile's rows of a lane's column: its own 16 rows, then the
+  // four row groups, in a fixed order
+  auto over_rows = [&](float v) {
+    v += __shfl_xor(v, 16, 64);
+    v += __shfl_xor(v, 32, 64);
+    return v;
+  };
+  // activation into a, derivative into d
+  auto activate = [&](float v0, float v1, float (&d)[2], PanelRow *a, int row) {
+    const float s0 = sigmoid(v0), s1 = sigmoid(v1);
+    d[0] = s0 * (1.0f + v0 * (1.0f - s0));
+    d[1] = s1 * (1.0f + v1 * (1.0f - s1));
+    // computed here, not where they are used: v and s would wait instead
+    asm volatile("" : "+v"(d[0]), "+v"(d[1]));
+    *reinterpret_cast<uint32_t *>(&a[row][col]) = pack_bf16(v0 * s0, v1 * s1);
+  };
+
+  weights(T.p16 + TP_W1);
+  for (int i = tid; i < TT_ROWS * TT_IN; i += TT_THREADS) xs[i] = T.x[row0 * TT_IN + i];
+  for (int i = tid; i < TT_OUT * PK; i += TT_THREADS) w4[i] = T.p[TP_W4 + i];
+  float d0[16][2], d1[16][2], d2[16][2], d3[16][2];
+  {
+    float w0[2][TT_IN], bias[2];
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      bias[nt] = T.p[TT_B0 + col + nt];
+#pragma unroll
+      for (int k = 0; k < TT_IN; ++k) w0[nt][k] = T.p[(col + nt) * TT_IN + k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      stage(e);
+      const int row = 16 * (e >> 2) + 4 * g + (e & 3);
+      float v[2] = {bias[0], bias[1]};
+#pragma unroll
+      for (int k = 0; k < TT_IN; ++k) {
+        const float xv = xs[row * TT_IN + k];
+        v[0] += xv * w0[0][k];
+        v[1] += xv * w0[1][k];
+      }
+      activate(v[0], v[1], d0[e], A[0], row);
+    }
+  }
+  __syncthreads();
+  auto forward = [&](int bias_at, float (&d)[16][2], PanelRow *out) {
+    const float2 bias = *reinterpret_cast<const float2 *>(T.p + bias_at + col);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      stage(e);
+      activate(acc[e >> 2][0][e & 3] + bias.x, acc[e >> 2][1][e & 3] + bias.y, d[e], out,
+               16 * (e >> 2) + 4 * g + (e & 3));
+    }
+  };
+  stage(0);
+  product(A[0]);
+  stage(0);
+  weights(T.p16 + TP_W2);
+  copy_out(A[0], T.act[0]);
+  stage(0);
+  forward(TP_B1, d1, A[1]);
+  __syncthreads();
+  stage(0);
+  product(A[1]);
+  stage(0);
+  weights(T.p16 + TP_W3);
+  copy_out(A[1], T.act[1]);
+  stage(0);
+  forward(TP_B2, d2, A[0]);
+  __syncthreads();
+  stage(0);
+  product(A[0]);
+  stage(0);
+  copy_out(A[0], T.act[2]);
+  stage(0);
+  forward(TP_B3, d3, A[1]);
+  __syncthreads();
+  // last layer, loss and its gradient: eight threads a row, 32 features each
+  // (each starting at its own four, so that they meet in no LDS bank)
+  {
+    const int row = tid >> 3, part = tid & 7;
+    float s[TT_OUT] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      stage(i);
+      const int c = 32 * part + 4 * ((i + part) & 7);
+      const uint2 a = *reinterpret_cast<const uint2 *>(&A[1][row][c]);
+      const float h[4] = {__uint_as_float(a.x << 16), __uint_as_float(a.x & 0xffff0000u),
+                          __uint_as_float(a.y << 16), __uint_as_float(a.y & 0xffff0000u)};
+#pragma unroll
+      for (int j = 0; j < TT_OUT; ++j) {
+        const float4 w = *reinterpret_cast<const float4 *>(&w4[j * PK + c]);
+        s[j] += (h[0] * w.x + h[1] * w.y) + (h[2] * w.z + h[3] * w.w);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < TT_OUT; ++j)
+#pragma unroll
+      for (int o = 1; o < 8; o *= 2) s[j] += __shfl_xor(s[j], o, 64);
+    float dy = 0.0f, loss = 0.0f;
+    if (part < TT_OUT) {
+      const int64_t at = (row0 + row) * TT_OUT + part;
+      const float y = (part == 0 ? s[0] : part == 1 ? s[1] : s[2]) + T.p[TP_B4 + part];
+      const float wj = T.weight[part], d = y - T.target[at];
+      T.y[at] = y;
+      dy = 2.0f * wj * d / (float)T.rows;
+      loss = wj * d * d / (float)T.rows;
+      reinterpret_cast<float *>(&dys[row])[part] = dy;
+    }
+#pragma unroll
+    for (int o = 8; o < 64; o *= 2) dy += __shfl_xor(dy, o, 64);
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2) loss += __shfl_xor(loss, o, 64);
+    if (lane < TT_OUT) red[wave][lane] = dy;
+    if (lane == TT_OUT) red[wave][TT_OUT] = loss;
+  }
+  weights(T.wt16[2]);
+  __syncthreads();
+  if (tid <= TT_OUT) {
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < TT_THREADS / 64; ++w) v += red[w][tid];
+    sums[TT_B4 + tid] = v;  // the last layer's bias, then the loss
+  }
+  {
+    float wv[TT_OUT][2], gw[TT_OUT][2], gb[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < TT_OUT; ++j)
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) {
+        wv[j][nt] = w4[j * PK + col + nt];
+        gw[j][nt] = 0.0f;
+      }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      stage(e);
+      const int row = 16 * (e >> 2) + 4 * g + (e & 3);
+      const float4 t = dys[row];
+      const float dy[TT_OUT] = {t.x, t.y, t.z};
+      const uint32_t h = *reinterpret_cast<const uint32_t *>(&A[1][row][col]);
+      const float hv[2] = {__uint_as_float(h << 16), __uint_as_float(h & 0xffff0000u)};
+      float v[2] = {0.0f, 0.0f};
+#pragma unroll
+      for (int j = 0; j < TT_OUT; ++j)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+          v[nt] += dy[j] * wv[j][nt];
+          gw[j][nt] += hv[nt] * dy[j];
+        }
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) {
+        v[nt] *= d3[e][nt];
+        gb[nt] += v[nt];
+      }
+      *reinterpret_cast<uint32_t *>(&A[0][row][col]) = pack_bf16(v[0], v[1]);
+    }
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+#pragma unroll
+      for (int j = 0; j < TT_OUT; ++j) {
+        const float v = over_rows(gw[j][nt]);
+        if (lane < 16) sums[TT_W4 + j * PK + col + nt] = v;
+      }
+      const float v = over_rows(gb[nt]);
+      if (lane < 16) sums[TT_B3 + col + nt] = v;
+    }
+  }
+  __syncthreads();
+  auto backward = [&](const float (&d)[16][2], int bias_at, PanelRow *out) {
+    float gb[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      stage(e);
+      const float v0 = acc[e >> 2][0][e & 3] * d[e][0], v1 = acc[e >> 2][1][e & 3] * d[e][1];
+      gb[0] += v0;
+      gb[1] += v1;
+      *reinterpret_cast<uint32_t *>(&out[16 * (e >> 2) + 4 * g + (e & 3)][col]) = pack_bf16(v0, v1);
+    }
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      const float v = over_rows(gb[nt]);
+      if (lane < 16) sums[bias_at + col + nt] = v;
+    }
+  };
+  stage(0);
+  product(A[0]);
+  stage(0);
+  weights(T.wt16[1]);
+  copy_out(A[0], T.dpre[2]);
+  stage(0);
+  backward(d2, TT_B2, A[1]);
+  __syncthreads();
+  stage(0);
+  product(A[1]);
+  stage(0);
+  weights(T.wt16[0]);
+  copy_out(A[1], T.dpre[1]);
+  stage(0);
+  backward(d1, TT_B1, A[0]);
+  __syncthreads();
+  stage(0);
+  product(A[0]);
+  stage(0);
+  copy_out(A[0], T.dpre[0]);
+  stage(0);
+  {
+    // read the inputs again: the compiler would keep those of the first layer
+    // in 80 registers all the way
+    int again = 0;
+    asm volatile("" : "+v"(again));
+    const float *xin = xs + again;
+    float gw[2][TT_IN], gb[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+      for (int k = 0; k < TT_IN; ++k) gw[nt][k] = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      stage(e);
+      const int row = 16 * (e >> 2) + 4 * g + (e & 3);
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) {
+        const float v = acc[e >> 2][nt][e & 3] * d0[e][nt];
+        gb[nt] += v;
+#pragma unroll
+        for (int k = 0; k < TT_IN; ++k) gw[nt][k] += v * xin[row * TT_IN + k];
+      }
+    }
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+#pragma unroll
+      for (int k = 0; k < TT_IN; ++k) {
+        const float v = over_rows(gw[nt][k]);
+        if (lane < 16) sums[(col + nt) * TT_IN + k] = v;
+      }
+      const float v = over_rows(gb[nt]);
+      if (lane < 16) sums[TT_B0 + col + nt] = v;
+    }
+  }
+}
+
+// Adds the tiles' partial sums as reduce_partials does (fixed order) and puts
+// each where it belongs in the gradient; the last is the loss.
+__global__ __launch_bounds__(64 * RED_WAVES) void train_reduce(const float *__restrict__ partial, int tiles,
+                                                               float *__restrict__ grad,
+                                                               float *__restrict__ loss) {
+  __shared__ float red[RED_WAVES][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int j = blockIdx.x * 64 + lane;
+  float s = 0.0f;
+  if (j < TT_SUMS) {
+#pragma unroll 8
+    for (int z = w; z < tiles; z += RED_WAVES) s += partial[(int64_t)z * TT_SUMS + j];
+  }
+  red[w][lane] = s;
+  __syncthreads();
+  if (w != 0 || j >= TT_SUMS) return;
+  float t = 0.0f;
+#pragma unroll
+  for (int u = 0; u < RED_WAVES; ++u) t += red[u][lane];
+  if (j == TT_LOSS)
+    *loss = t;
+  else
+    grad[j < TT_B1 ? j : j < TT_B2 ? TP_B1 + j - TT_B1 : j < TT_B3 ? TP_B2 + j - TT_B2 : TP_B3 + j - TT_B3] = t;
+}
+
+// ---------------------------------------------------------------------------
 // elementwise and small-layer kernels
 // ---------------------------------------------------------------------------
 
@@ -1698,6 +2058,33 @@ int32_t optk_gemm_bf16_silu_back_sums(int64_t m, const void *a, int64_t lda, con
     e = hipGetLastError();
   }
   if (e != hipSuccess) return fail(OPTK_EDEVICE, std::string("gemm_silu_back_sums launch: ") + hipGetErrorString(e));
+  return OPTK_OK;
+}
+
+int32_t optk_train_pass(const optk_train_args *args, void *hip_stream) {
+  if (!args) return fail(OPTK_EINVAL, "null argument");
+  const optk_train_args &T = *args;
+  if (T.rows <= 0 || T.rows % TT_ROWS || T.rows / TT_ROWS > INT32_MAX)
+    return fail(OPTK_EINVAL, "train_pass: rows must be a positive multiple of 64");
+  const void *wide[] = {T.p16, T.wt16[0], T.wt16[1], T.wt16[2], T.act[0], T.act[1], T.act[2],
+                        T.dpre[0], T.dpre[1], T.dpre[2]};
+  for (const void *q : wide)
+    if (!q || (uintptr_t)q % 16)
+      return fail(OPTK_EINVAL, "train_pass: bf16 arrays must be given, 16-byte aligned");
+  if (!T.x || !T.target || !T.weight || !T.p || !T.y || !T.grad || !T.loss || !T.workspace)
+    return fail(OPTK_EINVAL, "train_pass: missing array");
+  if ((uintptr_t)T.p % 8) return fail(OPTK_EINVAL, "train_pass: the parameters need 8-byte alignment");
+  const int64_t tiles = T.rows / TT_ROWS;
+  if (T.workspace_count < tiles * TT_SUMS) return fail(OPTK_EINVAL, "train_pass: workspace too small");
+  hipStream_t s = (hipStream_t)hip_stream;
+  hipLaunchKernelGGL(train_tile, dim3((unsigned)tiles), dim3(TT_THREADS), 0, s, T);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(train_reduce, dim3((TT_SUMS + 63) / 64), dim3(64 * RED_WAVES), 0, s, T.workspace,
+                       (int)tiles, T.grad, T.loss);
+    e = hipGetLastError();
+  }
+  if (e != hipSuccess) return fail(OPTK_EDEVICE, std::string("train_pass launch: ") + hipGetErrorString(e));
   return OPTK_OK;
 }
 

@@ -154,29 +154,7 @@ class MLP:
             H = WIDTHS[1]
             self.pre = [f(rows, H) for _ in range(4)]
             self.act = [h(rows, H) for _ in range(4)]
-            self.y = f(rows, 3)
-            if train:
-                self.dy = f(rows, 3)
-                # two bf16 gradient buffers: the backward GEMM of a layer
-                # reads one while its epilogue writes the previous layer's
-                # gradient into the other
-                self.dpre16 = h(rows, H)
-                self.dpre16_b = h(rows, H)
-                self.dpre32 = f(rows, H)
-                # the hidden layers' bf16 weights transposed ([in][out]): the
-                # backward product's B operand with k contiguous
-                self.wt16 = [h(H, H) for _ in range(3)]
-                self.ones = torch.ones(rows, 1, dtype=torch.float32, device=self.dev)
-                # split the weight-gradient GEMM's k = rows so that its four
-                # 128 x 128 output tiles make ~2 blocks per CU
-                split = max(1, min(128, rows // 512))
-                while rows % (32 * split):
-                    split //= 2
-                self.split = split
-                # also the per-block partials of the small outer products
-                # (at most min(512, rows / 32) blocks of H x 8)
-                self.ws = f(max(split * H * H, min(512, (rows + 31) // 32) * H * 8))
-                self.loss_part = f((rows * 3 + 255) // 256)
+            self._forward_y = f(rows, 3)
             self._buf_key = key
 
     def forward(self, x: torch.Tensor, train: bool = False) -> torch.Tensor:
@@ -184,6 +162,7 @@ class MLP:
         rows = x.shape[0]
         assert rows % 64 == 0 and x.dtype == torch.float32 and x.is_contiguous()
         self._buffers(rows, train)
+        self.y = self._forward_y
         H = WIDTHS[1]
         _op(_lib.MLP_DENSE_IN, f32=[x, self.view(self.p, 0, 0), self.view(self.p, 0, 1),
                                     self.pre[0]],
@@ -202,48 +181,58 @@ class MLP:
         return self.y
 
     # -- backward --------------------------------------------------------
+    def _train_buffers(self, rows):
+        if getattr(self, "_train_rows", None) == rows:
+            return
+        f = lambda *s: torch.empty(s, dtype=torch.float32, device=self.dev)  # noqa: E731
+        h = lambda *s: torch.empty(s, dtype=torch.int16, device=self.dev)  # noqa: E731
+        H = WIDTHS[1]
+        # what the hidden layers' weight gradients are products of
+        self.train_act = [h(rows, H) for _ in range(3)]
+        self.dpre16 = [h(rows, H) for _ in range(3)]
+        # the hidden layers' bf16 weights transposed ([in][out]): the
+        # backward product's B operand with k contiguous
+        self.wt16 = [h(H, H) for _ in range(3)]
+        self.train_y = f(rows, 3)
+        # split the weight-gradient GEMM's k = rows so that its four
+        # 128 x 128 output tiles make ~2 blocks per CU
+        split = max(1, min(128, rows // 512))
+        while rows % (32 * split):
+            split //= 2
+        self.split = split
+        # also the partial sums of the 64-row tiles (3076 each)
+        self.ws = f(max(split * H * H, rows // 64 * 3076))
+        self._train_rows = rows
+
     def loss_grad(self, x, target, weight) -> torch.Tensor:
         """Forward, weighted-MSE loss and gradients into ``self.g``;
         returns the loss (a device scalar).  rows: a multiple of 128."""
         rows = x.shape[0]
         if rows % 128:
             raise ValueError("training batches must hold a multiple of 128 rows")
+        assert x.dtype == torch.float32 and x.is_contiguous()
         H = WIDTHS[1]
-        self.forward(x, train=True)
-        _op(_lib.MLP_MSE_GRAD, f32=[self.y, target, weight, self.dy, self.loss_part], rows=rows,
-            cols=3)
-        g = self.g
-        # output layer
-        _op(_lib.MLP_OUTER_GRAD, f32=[None, self.dy, self.view(g, 4, 0), self.ws],
-            u16=[self.act[3]], rows=rows, cols=H, inner=3, count=self.ws.numel(), flag=0)
-        _op(_lib.MLP_OUTER_GRAD, f32=[self.dy, self.ones, self.view(g, 4, 1), self.ws],
-            rows=rows, cols=3, inner=1, count=self.ws.numel(), flag=1)
-        # the last hidden layer's dpre (bf16) and its column sums, that
-        # layer's bias gradient; the other bias gradients come with the
-        # backward products below
-        _op(_lib.MLP_DENSE_OUT_BACK, f32=[self.dy, self.view(self.p, 4, 0), self.pre[3], None,
-                                          self.view(g, 3, 1), self.ws], u16=[self.dpre16],
-            rows=rows, cols=H, inner=3, count=self.ws.numel())
+        self._train_buffers(rows)
         for layer in (1, 2, 3):
             _op(_lib.MLP_TRANSPOSE16, u16=[self.view(self.p16, layer, 0), self.wt16[layer - 1]],
                 rows=H, cols=H)
-        d16, d16_next = self.dpre16, self.dpre16_b
+        loss = torch.empty((), dtype=torch.float32, device=self.dev)
+        a = _lib.TrainArgs()
+        a.x, a.target, a.weight = x.data_ptr(), target.data_ptr(), weight.data_ptr()
+        a.p, a.p16 = self.p.data_ptr(), self.p16.data_ptr()
+        for i in range(3):
+            a.wt16[i] = self.wt16[i].data_ptr()
+            a.act[i] = self.train_act[i].data_ptr()
+            a.dpre[i] = self.dpre16[i].data_ptr()
+        a.y, a.grad, a.loss = self.train_y.data_ptr(), self.g.data_ptr(), loss.data_ptr()
+        a.workspace, a.workspace_count, a.rows = self.ws.data_ptr(), self.ws.numel(), rows
+        _lib.check(_lib.lib().optk_train_pass(ctypes.byref(a), _stream()))
+        self.y = self.train_y
         for layer in (3, 2, 1):
             # weight gradient: gW[o][i] = sum_r dpre[r][o] act[r][i]
-            _gemm(1, 0, H, H, rows, d16, H, self.act[layer - 1], H, self.view(g, layer, 0),
-                  H, self.split, self.ws)
-            # back to the previous layer: dpre = (dpre W) * silu'(pre), the
-            # derivative in the GEMM's epilogue with the column sums (that
-            # layer's bias gradient); the float32 dpre is kept only for the
-            # first layer's weight gradient
-            _gemm_silu_back_sums(rows, d16, H, self.wt16[layer - 1], H, self.pre[layer - 1], H,
-                                 self.dpre32 if layer == 1 else None, d16_next,
-                                 self.view(g, layer - 1, 1), self.ws)
-            d16, d16_next = d16_next, d16
-        # first layer (float32)
-        _op(_lib.MLP_OUTER_GRAD, f32=[self.dpre32, x, self.view(g, 0, 0), self.ws], rows=rows,
-            cols=H, inner=5, count=self.ws.numel(), flag=1)
-        return self.loss_part.sum()
+            _gemm(1, 0, H, H, rows, self.dpre16[layer - 1], H, self.train_act[layer - 1], H,
+                  self.view(self.g, layer, 0), H, self.split, self.ws)
+        return loss
 
     def adam_step(self, lr, beta1=0.9, beta2=0.999, eps=1e-8):
         self.t += 1
