@@ -23,7 +23,7 @@ one core.
 Other workloads (``--workload``): ``spectrograph`` (the EUV spectrograph,
 4 counted surfaces, two diffraction orders, Mo/Si multilayers on both
 mirrors; 50M rays) and ``tolerance`` (4096 perturbed spectrographs with
-log-uniform ray counts in one persistent batched launch, autotuned and
+log-uniform ray counts in one batched launch, autotuned and
 replayed from a hipGraph), ``surrogate`` (the learned surrogate alone) and
 ``stops`` (normalized field/pupil coordinates: the stop solve on the
 device, then the trace of the denormalized grid, both inside each step) and
@@ -493,7 +493,7 @@ def run_tolerance(args):
     config = {
         "workload": f"tolerance batch: {N} perturbed EUV spectrographs (decenter 50 um, tilt "
                     "0.01 deg, radii 0.1 %, line spacing 0.5 %, seed 3), ray counts log-uniform "
-                    f"1k-64k ({n} rays) x 2 orders, one persistent launch, hipGraph replay",
+                    f"1k-64k ({n} rays) x 2 orders, one launch, hipGraph replay",
         "instances": N,
         "rays": n,
         "paths": P,

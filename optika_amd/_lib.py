@@ -404,7 +404,8 @@ def lib() -> ctypes.CDLL:
                       ("optk_mlp_args", MlpArgs), ("optk_surrogate_desc", SurrogateDesc),
                       ("optk_surrogate_io", SurrogateIO), ("optk_stop_args", StopArgs),
                       ("optk_pupil_args", PupilArgs), ("optk_denormalize_args", DenormalizeArgs),
-                      ("optk_expose_args", ExposeArgs), ("optk_scene_args", SceneArgs)]:
+                      ("optk_expose_args", ExposeArgs), ("optk_scene_args", SceneArgs),
+                      ("optk_train_args", TrainArgs)]:
         size = L.optk_sizeof(name.encode())
         if size != ctypes.sizeof(cls):
             raise OptkError(f"record {name}: C size {size} != binding size {ctypes.sizeof(cls)}")

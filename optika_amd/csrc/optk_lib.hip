@@ -152,8 +152,7 @@ __device__ __forceinline__ Ray<double> load_ray(const GridIn &g, int64_t i) {
                   g.object_at_infinity);
 }
 
-// bytes of LDS a batched or stop-solve launch stages: the spec, then the
-// surface records
+// bytes of LDS a stop-solve launch stages: the spec, then the surface records
 static size_t staged_bytes(int num_surfaces) {
   return sizeof(TraceSpec) + sizeof(optk_surface) * (size_t)num_surfaces;
 }
@@ -1758,6 +1757,7 @@ int64_t optk_sizeof(const char *name) {
   if (s == "optk_pupil_args") return sizeof(optk_pupil_args);
   if (s == "optk_denormalize_args") return sizeof(optk_denormalize_args);
   if (s == "optk_scene_args") return sizeof(optk_scene_args);
+  if (s == "optk_train_args") return sizeof(optk_train_args);
   if (s == "optk_expose_args") return sizeof(optk_expose_args);
   return -1;
 }
