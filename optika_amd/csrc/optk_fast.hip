@@ -452,11 +452,13 @@ const SpecRays32 SPEC_RAYS32[NUM_SIGNATURES] = {
                         OPTK_SIGNATURE_SPECTROGRAPH_TILTED>,
 };
 
-// kernels of one entry point: by feature set (geometric, toroid + rulings,
-// all; all with the per-surface accumulation), for either I/O layout
+// kernels of one entry point by feature set (geometric, toroid + rulings,
+// all): without and with the per-surface accumulation, and in the entry
+// point's fixed layout
 template <typename In> struct KernelSet {
   typedef void (*Kernel)(FastArgs, In, FRaysOut);
-  Kernel any[4];
+  Kernel any[3];
+  Kernel accumulating[3];
   Kernel special[3];  // the entry point's fixed-layout form (IO_SENSOR for the
                       // grid, IO_FULL for rays), by feature set
 };
@@ -480,7 +482,7 @@ int32_t launch(const KernelSet<In> &ks, bool special, const optk_system *sys, co
   if (accum) acc = *accum;
   const int f = sys->features;
   const int which = f == 0 ? 0 : (f == (FEAT_TOROID | FEAT_RULINGS) ? 1 : 2);
-  typename KernelSet<In>::Kernel kern = accum ? ks.any[3] : ks.any[which];
+  typename KernelSet<In>::Kernel kern = accum ? ks.accumulating[which] : ks.any[which];
   if (!accum && special) kern = ks.special[which];
   // whole rounds of resident blocks; each block loops over its share
   const int64_t blocks = resident_grid((const void *)kern, TRACE_BLOCK, n);
@@ -686,7 +688,9 @@ int32_t fast_trace_rays(const optk_system *sys, const FRaysIn &in, const FRaysOu
                         hipStream_t stream) {
   static const KernelSet<FRaysIn> ks = {
       {trace_rays_f32<0, false>, trace_rays_f32<FEAT_TOROID | FEAT_RULINGS, false>,
-       trace_rays_f32<FEAT_ALL, false>, trace_rays_f32<FEAT_ALL, true>},
+       trace_rays_f32<FEAT_ALL, false>},
+      {trace_rays_f32<0, true>, trace_rays_f32<FEAT_TOROID | FEAT_RULINGS, true>,
+       trace_rays_f32<FEAT_ALL, true>},
       {trace_rays_f32<0, false, IO_FULL>, trace_rays_f32<FEAT_TOROID | FEAT_RULINGS, false, IO_FULL>,
        trace_rays_f32<FEAT_ALL, false, IO_FULL>}};
   const SpecRays32 spec = (sys->signature >= 0 && !generic) ? SPEC_RAYS32[sys->signature] : nullptr;
@@ -698,7 +702,9 @@ int32_t fast_trace_grid(const optk_system *sys, const FGridIn &in, const FRaysOu
                         hipStream_t stream) {
   static const KernelSet<FGridIn> ks = {
       {trace_grid_f32<0, false>, trace_grid_f32<FEAT_TOROID | FEAT_RULINGS, false>,
-       trace_grid_f32<FEAT_ALL, false>, trace_grid_f32<FEAT_ALL, true>},
+       trace_grid_f32<FEAT_ALL, false>},
+      {trace_grid_f32<0, true>, trace_grid_f32<FEAT_TOROID | FEAT_RULINGS, true>,
+       trace_grid_f32<FEAT_ALL, true>},
       {trace_grid_f32<0, false, IO_SENSOR>, trace_grid_f32<FEAT_TOROID | FEAT_RULINGS, false, IO_SENSOR>,
        trace_grid_f32<FEAT_ALL, false, IO_SENSOR>}};
   const SpecGrid32 spec = (sys->signature >= 0 && !generic) ? SPEC_GRID32[sys->signature] : nullptr;
